@@ -5,6 +5,7 @@
 // issued has completed, as the reference's calls do.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <chrono>
 #include <cmath>
 #include <cstdio>
@@ -431,8 +432,57 @@ void cuda_shutdown_(void) {
 }
 
 // ------------------------------------------------------------- extended
+// Does the device loop advance the tree with the marching kernels?
+static bool marches() {
+  return tree_step2_eligible(g_tree) && g_tree.blocking == 1 &&
+         march_applies(dev_view(g_tree, g_tree.layers[1], true, true));
+}
+
+// n root steps in the marching kernels.  The run ends with a two-step launch
+// (n even) or a single step (n odd), so level 2 then holds the state two
+// steps (one step) before level 1.
+static int run_marched(int n, int use_graph) {
+  LayerRec *R = layer(1);
+  const int K = march_plan(R->nx, R->ny).steps;
+  auto enqueue = [&](int k) -> int {
+    const hipError_t e = launch_march_linear(dev_view(g_tree, *R, true, true), k, g_stream);
+    if (e != hipSuccess) return fail(200 + (int)e, "marching launch failed: %s", hipGetErrorString(e));
+    R->cur = 1 - R->cur;
+    g_tree.ctl_in = 1 - g_tree.ctl_in;
+    return 0;
+  };
+  int body = std::max(0, (n - (n % 2 ? 1 : 2)) / K);
+  n -= body * K;
+  // Launches per captured graph (an even number: it replays from the level
+  // parity it was captured at).  Capturing pays from a few replays on.
+  constexpr int kPer = 8;
+  if (use_graph && body >= 4 * kPer) {
+    hipGraph_t graph = nullptr;
+    hipGraphExec_t exec = nullptr;
+    HIPCHK(hipStreamBeginCapture(g_stream, hipStreamCaptureModeThreadLocal));
+    int r = 0;
+    for (int k = 0; k < kPer && !r; ++k) r = enqueue(K);
+    hipError_t ce = hipStreamEndCapture(g_stream, &graph);
+    if (r) return r;
+    HIPCHK(ce);
+    HIPCHK(hipGraphInstantiate(&exec, graph, nullptr, nullptr, 0));
+    for (; body >= kPer; body -= kPer) HIPCHK(hipGraphLaunch(exec, g_stream));
+    HIPCHK(hipStreamSynchronize(g_stream));
+    (void)hipGraphExecDestroy(exec);
+    (void)hipGraphDestroy(graph);
+  }
+  for (; body > 0; --body)
+    if (int r = enqueue(K)) return r;
+  for (; n >= 2; n -= 2)
+    if (int r = enqueue(2)) return r;
+  if (n > 0)
+    if (int r = tree_enqueue_root_step(g_tree, g_stream)) return r;
+  return sync();
+}
+
 // n root steps of the device loop, no output files
 static int run_plain(int n, int use_graph) {
+  if (marches()) return run_marched(n, use_graph);
   if (tree_step2_eligible(g_tree) && n >= 2) {
     // a linear single layer: two root steps per launch; a graph of two
     // launches (four steps) brings the level parity back for replay
@@ -896,9 +946,14 @@ int gcomcot_autotune_(int *reps, int *variant, int *blocking, float *ms_per_step
       if (ms < best) { best = ms; bv = v; bb = 0; }
     }
     if (!R->nl) {
+      const bool march = march_applies(dev_view(g_tree, *R, true, true));
+      const int K = march_plan(R->nx, R->ny).steps;
       for (int sh = 0; sh < kStep2Shapes; ++sh) {
         float ms;
-        if (int r = time_it([&] { return launch_step2(d, R->sph != 0, sh, g_stream); }, 2, &ms))
+        // mode 1 (shape 0) is the marching kernels where they apply
+        if (int r = sh == 0 && march
+                        ? time_it([&] { return launch_march_linear(d, K, g_stream); }, K, &ms)
+                        : time_it([&] { return launch_step2(d, R->sph != 0, sh, g_stream); }, 2, &ms))
           return r;
         if (ms < best) { best = ms; bb = sh + 1; }
       }

@@ -38,5 +38,7 @@ enum Coef {
   kR6,       // COS_N
   kNumCoef
 };
+// floats per row of the row-major copy that the marching kernels read
+constexpr int kRowCoef = 8;
 
 }  // namespace gc

@@ -19,6 +19,7 @@ struct DevLayer {
   float kfric;     // (0.5*DT*GRAV)*FM*FM, the Fortran's CONST*FM*FM
   const float *h;
   const float *coef;   // per-row table (comcot_consts.h), spherical only
+  const float *rowc;   // R1, R11, R6, R3, R5, F2, F4, 0 of each row (kRowCoef floats a row)
   const float *r24;    // optional R2|R4 planes (drop-in fallback), else null
   const float *z1, *m1, *n1;
   float *z2, *m2, *n2;
@@ -70,6 +71,19 @@ hipError_t launch_step2(const DevLayer &L, bool sph, int shape, hipStream_t st);
 constexpr int kStep2Shapes = 7;
 // tile of two-step shape `shape`
 void step2_shape(int shape, int *tx, int *ty);
+
+// Root steps of a spherical linear outermost layer without children in the
+// marching kernels (march.hip): 2 or 4 per launch, level 1 in, level 2 out,
+// bookkeeping as launch_step2.  march_plan gives the steps per launch that
+// suit a layer and how its waves split it; march_applies says whether a
+// layer's view can take them (row-major coefficients, no R2/R4 planes, no
+// MAX_AMP maximum or sponge, planes within 4 GB).
+struct MarchPlan {
+  int steps, seg, seg_side;
+};
+MarchPlan march_plan(int nx, int ny);
+bool march_applies(const DevLayer &L);
+hipError_t launch_march_linear(const DevLayer &L, int steps, hipStream_t st);
 
 // Reference-semantics maximum (no wet test) plus the wet max/arrival.
 hipError_t launch_max(const DevLayer &L, float *zmax_raw, hipStream_t st);

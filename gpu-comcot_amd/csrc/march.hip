@@ -1,0 +1,422 @@
+// Register-marching kernels: several root steps of a linear outermost layer
+// in one pass over its planes.
+//
+// A wavefront owns a strip of 64 columns and marches along J.  Lane l holds
+// column c0 - K + l; each iteration loads one row of Z, M, N, H and moves K
+// time steps one row further, step s working s rows behind step 1, so every
+// intermediate row lives in registers and neighbouring columns are read
+// from the neighbouring lane (DPP wave shifts, free as VALU operands).
+// There is no LDS and no barrier.  A step makes one column on each side
+// invalid, so a strip writes 64 - 2K columns, and a segment of SEG rows
+// takes SEG + 2K iterations.
+//
+// Against the LDS tiles (k_step2) a cell costs about a third of the
+// instructions (no staging, no index arithmetic per cell, no halo ring of
+// a tile recomputed) and K steps share one read and one write of the
+// planes.
+//
+// Values are those of the single-step kernels bit for bit: the same
+// operations on the same operands in the same order (MASS_S
+// mass.f90:61-100, OPEN boundaries.f90:22-202, MOMT_S moment.f90:65-149,
+// the wet maximum and first arrival step by step).
+#include <hip/hip_runtime.h>
+
+#include <algorithm>
+
+#include "comcot_consts.h"
+#include "kernels.h"
+
+namespace gc {
+
+namespace {
+
+constexpr int kWave = 64;
+constexpr int kMarchBlock = 256;
+
+// Value of the lane one column to the west (I - 1) / east (I + 1); the
+// outermost lane of the wave gets 0 (its results are never stored).
+__device__ __forceinline__ float west(float v) {
+  return __int_as_float(
+      __builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x138, 0xf, 0xf, true));
+}
+__device__ __forceinline__ float east(float v) {
+  return __int_as_float(
+      __builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x130, 0xf, 0xf, true));
+}
+
+// Planes are read and written through one buffer descriptor over the
+// layer's block (every plane of a layer lies in one allocation, behind its
+// depth plane): a lane's column is the vector offset, plane and row the
+// scalar one, so rows cost no per-lane address arithmetic.  A lane that has
+// nothing to store gives offset kNoStore, which the descriptor's range check
+// drops: the row loop has no branch around a store.  (With branches the
+// compiler has to assume the shorter path when it counts outstanding memory
+// operations, and a wait for the next row's loads then also waits for
+// stores.)
+typedef __amdgpu_buffer_rsrc_t Block;
+constexpr int kNoStore = -1;
+__device__ __forceinline__ Block block_of(const DevLayer &L, unsigned bytes) {
+  return __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(L.h), 0, bytes, 0x00027000);
+}
+__device__ __forceinline__ unsigned plane_off(const DevLayer &L, const void *p) {
+  return (unsigned)(reinterpret_cast<unsigned long long>(p) -
+                    reinterpret_cast<unsigned long long>(L.h));
+}
+__device__ __forceinline__ float get(Block b, int voff, unsigned soff) {
+  return __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(b, voff, (int)soff, 0));
+}
+template <bool ST>
+__device__ __forceinline__ void put(Block b, int voff, unsigned soff, float v) {
+  __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(v), b, voff, (int)soff, ST ? 2 : 0);
+}
+
+// A lane mask held in scalar registers as this lane's condition.
+__device__ __forceinline__ bool lanes(unsigned long long m) {
+  return __builtin_amdgcn_inverse_ballot_w64(m);
+}
+
+// Work of one wave: lane 0's column, rows j0..j1 to write.
+struct Strip {
+  int c0, j0, j1;
+};
+
+// Row coefficients of MASS_S / MOMT_S at one row: one scalar load of eight
+// floats (constant address space: nothing writes the table while kernels
+// run).
+struct RowCoef {
+  float r1, r11, r6, r3, r5, f2, f4;
+};
+__device__ __forceinline__ RowCoef row_coef(const DevLayer &L, int j) {
+  typedef float Row8 __attribute__((ext_vector_type(kRowCoef)));
+  typedef const __attribute__((address_space(4))) Row8 *ConstPtr;
+  const Row8 c = ((ConstPtr)(unsigned long long)L.rowc)[(j < 1 ? 1 : (j > L.ny ? L.ny : j)) - 1];
+  return {c[0], c[1], c[2], c[3], c[4], c[5], c[6]};
+}
+
+// OPEN (boundaries.f90:22-202) at one ring cell: a, b are the two flux
+// components it combines (an average along the edge or a corner's own
+// flux, and the flux across), cc = sqrt(g H), neg says which way the wave
+// leaves.
+__device__ __forceinline__ float radiate(float h, float cc, float a, float b, bool neg) {
+  float zz = sqrtf(a * a + b * b) / cc;
+  if (neg) zz = -zz;
+  if (fabsf(zz) > kUB) zz = 0.0f;
+  return h > kGx ? zz : 0.0f;
+}
+
+// K linear root steps of strip S.  COL: the strip holds column I = 1 or NX
+// or its halo leaves the grid there; ROW: the same for rows.  Loads are
+// then clamped to the grid and OPEN and the index limits of the Fortran
+// loops apply; otherwise all of that compiles away.  Each row is
+// loaded D rows ahead of its use.  MX: the wet maximum and first
+// arrival are kept.
+template <int K, bool COL, bool ROW, bool MX, bool ST>
+__device__ __forceinline__ void march_linear(const DevLayer &L, const Strip S, int step,
+                                             unsigned block_bytes) {
+  // Rows in flight.  The row loop is unrolled by D, so a row's registers stay
+  // put until its turn: rotating them would wait for loads just issued.
+  constexpr int D = COL || ROW ? 2 : 4;
+  const int nx = L.nx, ny = L.ny, lane = threadIdx.x & (kWave - 1);
+  const int i = S.c0 - K + lane;
+  const int ic = COL ? min(max(i, 1), nx) : i;
+  const int vld = (ic - 1) * 4;
+  const bool own = lane >= K && lane < kWave - K && (!COL || i <= nx);
+  const bool west_end = COL && i == 1, east_end = COL && i == nx;
+  const int vst = own ? vld : kNoStore;
+  const int ra = S.j0 - K, rb = S.j1 + K;
+  const Block B = block_of(L, block_bytes);
+  const unsigned pitch = (unsigned)nx * 4u;
+  const unsigned oz1 = plane_off(L, L.z1), om1 = plane_off(L, L.m1), on1 = plane_off(L, L.n1),
+                 oz2 = plane_off(L, L.z2), om2 = plane_off(L, L.m2), on2 = plane_off(L, L.n2),
+                 omax = plane_off(L, L.zmax), oarr = plane_off(L, L.arrival);
+  auto base = [&](int j) {
+    const int jc = ROW ? min(max(j, 1), ny) : j;
+    return (unsigned)(jc - 1) * pitch;
+  };
+
+  // levels s = 0..K: Z, M at that level's newest row, M, N and N*R6 one row
+  // below (level 0's newest row is the row just loaded)
+  float Z[K + 1], M[K + 1], Mb[K], Nb[K], NRb[K];
+  // per row r, r-1, ...: depth, momentum factors, wet masks, maximum, arrival
+  float H[K + 1], R2[K], R4[K + 1], CC[K], zm[K];
+  // (zl: the maximum as loaded; below: how many of the steps so far left it
+  // under the arrival threshold, so the first arrival is step + below)
+  float zl[K];
+  int below[K];
+  unsigned long long wet[K + 1];  // lane masks of H > GX
+  RowCoef C[K + 1];
+#pragma unroll
+  for (int s = 0; s <= K; ++s) Z[s] = M[s] = H[s] = R4[s] = 0.0f, wet[s] = 0;
+#pragma unroll
+  for (int s = 0; s < K; ++s) {
+    Mb[s] = Nb[s] = NRb[s] = R2[s] = CC[s] = zm[s] = 0.0f;
+    zl[s] = 0.0f;
+    below[s] = 0;
+  }
+#pragma unroll
+  for (int s = 0; s <= K; ++s) C[s] = row_coef(L, ra);
+
+  float ph[D], pz[D], pm[D], pn[D], pq[D];
+  auto load = [&](int j, int k) {
+    const unsigned b = base(ROW ? j : min(j, rb));
+    ph[k] = get(B, vld, b);
+    pz[k] = get(B, vld, oz1 + b);
+    pm[k] = get(B, vld, om1 + b);
+    pn[k] = get(B, vld, on1 + b);
+    if (MX) pq[k] = get(B, vld, omax + b);
+  };
+#pragma unroll
+  for (int k = 0; k < D; ++k) load(ra + k, k);
+  RowCoef cnext = row_coef(L, ra);
+
+  auto row = [&](int r, int k) __attribute__((always_inline)) {  // k: the row's load slot
+    // ---- row r enters: shift the per-row values down
+#pragma unroll
+    for (int s = K; s > 0; --s) {
+      H[s] = H[s - 1];
+      C[s] = C[s - 1];
+      R4[s] = R4[s - 1];
+      wet[s] = wet[s - 1];
+    }
+#pragma unroll
+    for (int s = K - 1; s > 0; --s) {
+      R2[s] = R2[s - 1];
+      if (COL) CC[s] = CC[s - 1];
+      if (MX) {
+        zm[s] = zm[s - 1];
+        zl[s] = zl[s - 1];
+        below[s] = below[s - 1];
+      }
+    }
+    C[0] = cnext;
+    const float h = ph[k];
+    float zc = pz[k], mc = pm[k], nc = pn[k];
+    if (MX) {
+      zm[0] = zl[0] = pq[k];
+      below[0] = 0;
+    }
+    cnext = row_coef(L, r + 1);
+    load(r + D, k);
+    const float he = east(h);
+    H[0] = h;
+    wet[0] = __builtin_amdgcn_ballot_w64(h > kGx);
+    R2[0] = C[0].f2 * (0.5f * (h + he));   // used where both cells are wet: HP > 0
+    R4[1] = C[1].f4 * (0.5f * (H[1] + h));
+    if (COL) CC[0] = sqrtf(kGrav * h);
+
+#pragma unroll
+    for (int s = 0; s < K; ++s) {  // step s + 1 at row q
+      const int q = r - s;
+      const float hq = H[s];
+      // continuity
+      const float nr = nc * C[s].r6;
+      const float mw = west(mc);
+      float zz = zc - C[s].r1 * (mc - mw) - C[s].r11 * (nr - NRb[s]);
+      if (fabsf(zz) < kEps) zz = 0.0f;
+      const float t = zz + hq;
+      float zn = t <= kEps ? -hq : zz;
+      zn = lanes(wet[s]) ? zn : 0.0f;
+      bool w = lanes(wet[s] & __builtin_amdgcn_ballot_w64(t > kGx));
+      if (ROW && (q == 1 || q == ny)) {
+        // bottom and top rows; the corners take their own fluxes
+        const float b = q == 1 ? nc : Nb[s];
+        const float u = west_end ? mc : mw;
+        const bool corner = west_end | east_end;
+        const float a = corner ? u : 0.5f * (mc + mw);
+        bool neg = q == 1 ? b > 0.0f : b < 0.0f;
+        neg |= corner & (west_end ? u > 0.0f : u < 0.0f);
+        zn = radiate(hq, sqrtf(kGrav * hq), a, b, neg);
+        w = hq + zn > kGx;
+      } else if (COL) {
+        // left and right columns
+        const float u = west_end ? mc : mw;
+        const float a = (west_end & !(H[s + 1] > kGx)) ? nc : 0.5f * (nc + Nb[s]);
+        const bool neg = west_end ? u > 0.0f : u < 0.0f;
+        const bool ring = west_end | east_end;
+        const float zr = radiate(hq, CC[s], a, u, neg);
+        zn = ring ? zr : zn;
+        w = ring ? hq + zr > kGx : w;
+      }
+      // momentum: M at row q, N at row q - 1
+      const float ns = ROW && q == 1 ? nc : Nb[s];
+      const float tn = nc + east(nc) + ns + east(ns);
+      float mn = mc - R2[s] * (east(zn) - zn) + C[s].r3 * tn;
+      // M(I) needs I and I + 1 wet; |M| < EPS goes to 0
+      mn = lanes(wet[s] & (wet[s] >> 1) & ~__builtin_amdgcn_ballot_w64(fabsf(mn) < kEps)) ? mn : 0.0f;
+      if (COL) mn = east_end ? 0.0f : mn;
+      const float sum = Mb[s] + mc;
+      float sw = west(sum);
+      if (COL) sw = west_end ? sum : sw;
+      const float tm = sw + Mb[s] + mc;
+      float nn = Nb[s] - R4[s + 1] * (zn - Z[s + 1]) - C[s + 1].r5 * tm;
+      nn = lanes(wet[s + 1] & wet[s] & ~__builtin_amdgcn_ballot_w64(fabsf(nn) < kEps)) ? nn : 0.0f;
+      if (ROW && q - 1 == ny) nn = 0.0f;
+      if (MX) {  // wet maximum and first arrival of step s + 1 at row q
+        zm[s] = (w & (zn > zm[s])) ? zn : zm[s];
+        below[s] += zm[s] >= L.arr_thr ? 0 : 1;
+      }
+      // the level below is done with its rows
+      Mb[s] = mc;
+      Nb[s] = nc;
+      NRb[s] = nr;
+      // hand over: the next step works one row behind, on the values this
+      // level held before this iteration
+      const float zo = Z[s + 1], mo = M[s + 1];
+      Z[s + 1] = zn;
+      M[s + 1] = mn;
+      if (s + 1 < K) {
+        zc = zo;
+        mc = mo;
+        nc = nn;
+      } else {
+        const unsigned g = (unsigned)(q - 1) * pitch;
+        const int vq = q >= S.j0 && q <= S.j1 ? vst : kNoStore;
+        const int vn = q - 1 >= S.j0 && q - 1 <= S.j1 ? vst : kNoStore;
+        put<ST>(B, vq, oz2 + g, zn);
+        put<ST>(B, vq, om2 + g, mn);
+        put<ST>(B, vn, on2 + g - pitch, nn);
+        if (MX) {
+          put<false>(B, zm[s] != zl[s] ? vq : kNoStore, omax + g, zm[s]);
+          const bool hit = !(zl[s] >= L.arr_thr) & (below[s] < K);
+          put<false>(B, hit ? vq : kNoStore, oarr + g, __int_as_float(step + below[s]));
+        }
+      }
+    }
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  // Rows beyond rb (the unrolled loop's remainder) load row rb again and
+  // store nothing.  The first loads are waited for here (vmcnt 0): otherwise
+  // the wait at the loop's head has to serve the entry, where they are the
+  // newest operations, and would stop for everything in flight on each turn.
+  __builtin_amdgcn_s_waitcnt(0x0f70);
+  for (int r = ra; r <= rb; r += D)
+#pragma unroll
+    for (int u = 0; u < D; ++u) row(r + u, u);
+}
+
+// How the waves of a launch split a layer: strips of W columns in segments
+// of seg rows.  Strip 0 and the strips from east on reach the grid's side
+// columns; their waves cost more per row, so they take shorter segments
+// (seg_side) and come first in the grid.
+struct MarchGrid {
+  int nstrip, east, seg, nseg, seg_side, nseg_side, side_blocks, per_xcd;
+};
+
+// Side blocks first, then blocks in XCD order (block b runs on XCD b % 8;
+// each XCD takes one contiguous run of waves, so strips that share halo
+// columns meet in one L2).
+template <int K, bool MX, bool ST>
+__global__ void __launch_bounds__(kMarchBlock) k_march_linear(DevLayer L, MarchGrid G, unsigned block_bytes) {
+  constexpr int W = kWave - 2 * K, WB = kMarchBlock / kWave;
+  const int wb = threadIdx.x >> 6;
+  int step = 0;
+  if (MX) {
+    step = L.ctl[L.ctl_in] + 1;
+    if (L.advance && blockIdx.x == 0 && threadIdx.x == 0) L.ctl[1 - L.ctl_in] = step + K - 1;
+  }
+  Strip S;
+  if ((int)blockIdx.x < G.side_blocks) {
+    const int w = __builtin_amdgcn_readfirstlane(blockIdx.x * WB + wb);
+    const int nside = 1 + G.nstrip - G.east;
+    if (w >= nside * G.nseg_side) return;
+    const int k = w % nside;
+    S.c0 = (k == 0 ? 0 : G.east + k - 1) * W + 1;
+    S.j0 = (w / nside) * G.seg_side + 1;
+    S.j1 = min(S.j0 + G.seg_side - 1, L.ny);
+    march_linear<K, true, true, MX, ST>(L, S, step, block_bytes);
+    return;
+  }
+  const int b = blockIdx.x - G.side_blocks, mid = G.east - 1;
+  const int w = __builtin_amdgcn_readfirstlane(((b & 7) * G.per_xcd + (b >> 3)) * WB + wb);
+  if (w >= mid * G.nseg) return;
+  S.c0 = (1 + w % mid) * W + 1;
+  S.j0 = (w / mid) * G.seg + 1;
+  S.j1 = min(S.j0 + G.seg - 1, L.ny);
+  if (S.j0 - K < 2 || S.j1 + K > L.ny - 1) march_linear<K, false, true, MX, ST>(L, S, step, block_bytes);
+  else march_linear<K, false, false, MX, ST>(L, S, step, block_bytes);
+}
+
+// Bytes from a layer's depth plane to the end of its last plane; the
+// descriptor of the marching kernels spans them.  ~0 if a plane lies before.
+unsigned long long block_span(const DevLayer &L) {
+  const char *lo = reinterpret_cast<const char *>(L.h), *hi = lo;
+  for (const void *p : {(const void *)L.z1, (const void *)L.m1, (const void *)L.n1,
+                        (const void *)L.z2, (const void *)L.m2, (const void *)L.n2,
+                        (const void *)L.zmax, (const void *)L.arrival})
+    if (p) {
+      if (reinterpret_cast<const char *>(p) < lo) return ~0ull;
+      hi = std::max(hi, reinterpret_cast<const char *>(p));
+    }
+  return (unsigned long long)(hi - lo) + 4ull * L.nx * L.ny;
+}
+
+template <int K, bool MX, bool ST>
+hipError_t launch_k(const DevLayer &L, int seg, int seg_side, hipStream_t st) {
+  constexpr int W = kWave - 2 * K, WB = kMarchBlock / kWave;
+  MarchGrid G;
+  G.nstrip = (L.nx + W - 1) / W;
+  // first strip whose last lane lies beyond column NX - 1
+  G.east = L.nx - 1 >= W + kWave - K ? (L.nx - 1 - kWave + K) / W + 1 : 1;
+  G.east = std::min(G.east, G.nstrip);
+  G.seg = seg;
+  G.nseg = (L.ny + seg - 1) / seg;
+  G.seg_side = seg_side;
+  G.nseg_side = (L.ny + seg_side - 1) / seg_side;
+  const long long side = (long long)(1 + G.nstrip - G.east) * G.nseg_side;
+  const long long mid = (long long)(G.east - 1) * G.nseg;
+  G.side_blocks = (int)((side + WB - 1) / WB);
+  G.per_xcd = (int)((mid + 8 * WB - 1) / (8 * WB));
+  const long long blocks = (long long)G.side_blocks + 8LL * G.per_xcd;
+  if (blocks > 0x7fffffff) return hipErrorInvalidValue;
+  hipLaunchKernelGGL((k_march_linear<K, MX, ST>), dim3((unsigned)blocks), dim3(kMarchBlock), 0, st,
+                     L, G, (unsigned)block_span(L));
+  return hipGetLastError();
+}
+
+template <int K>
+hipError_t launch_k(const DevLayer &L, const MarchPlan &p, hipStream_t st) {
+  if (L.zmax)
+    return L.stream_out ? launch_k<K, true, true>(L, p.seg, p.seg_side, st)
+                        : launch_k<K, true, false>(L, p.seg, p.seg_side, st);
+  return L.stream_out ? launch_k<K, false, true>(L, p.seg, p.seg_side, st)
+                      : launch_k<K, false, false>(L, p.seg, p.seg_side, st);
+}
+
+}  // namespace
+
+// Rows of strips per SIMD decide the split.  With few of them a wave has
+// its SIMD to itself, an instruction then takes about 8 cycles instead of 4,
+// and a launch lasts as long as one wave's rows: short segments, and two
+// steps a launch where four would only add 2K rows to each.  Measured, us
+// per root step (two-step tiles before):
+//   517x391 (4 rows per SIMD)     K = 2, 8 rows 5.05, K = 4, 8 rows 5.58 (6.9)
+//   1024x768 (14)                 K = 4, 8 rows 5.57, 12 rows 6.9, 16 rows 7.1,
+//                                 K = 2, 8 rows 5.74 (11.0; best tile 8.5)
+//   2051x1537 (55)                K = 4, 12 rows 11.1, 16 rows 11.2, 8 rows 11.5 (28.8)
+//   4096x3072 (222)               K = 4, 24 rows 29.7, 16 rows 31, K = 2 49.7,
+//                                 K = 6, 32 rows 29.6 (99.6; best tile 72)
+// Side strips run OPEN on every row (about 1.6 times the time per row).
+MarchPlan march_plan(int nx, int ny) {
+  const long long rows = (long long)((nx + 55) / 56) * ny / 1024;
+  MarchPlan p;
+  p.steps = rows < 10 ? 2 : 4;
+  p.seg = rows < 32 ? 8 : (rows < 120 ? 12 : 24);
+  p.seg_side = rows < 120 ? 4 : 12;
+  return p;
+}
+
+bool march_applies(const DevLayer &L) {
+  return L.is_root && L.rowc && !L.r24 && !L.zraw && !L.sponge_cx && block_span(L) < 0xffffffffull;
+}
+
+hipError_t launch_march_linear(const DevLayer &L, int steps, hipStream_t st) {
+  if (!march_applies(L)) return hipErrorInvalidValue;
+  const MarchPlan p = march_plan(L.nx, L.ny);
+  switch (steps) {
+    case 2: return launch_k<2>(L, p, st);
+    case 4: return launch_k<4>(L, p, st);
+    default: return hipErrorInvalidValue;
+  }
+}
+
+}  // namespace gc

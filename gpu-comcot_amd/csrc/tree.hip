@@ -88,6 +88,7 @@ size_t Tree::device_bytes() const {
 static void free_layer(LayerRec &L) {
   if (L.block) (void)hipFree(L.block);
   if (L.r24) (void)hipFree(L.r24);
+  if (L.rowc) (void)hipFree(L.rowc);
   if (L.deform) (void)hipFree(L.deform);
   if (L.sponge) (void)hipFree(L.sponge);
   if (L.sc_pos) (void)hipFree(L.sc_pos);
@@ -250,10 +251,23 @@ int tree_create_layer(Tree &T, hipStream_t st, int id, int parent, int level, in
   return 0;
 }
 
+// The row-major copy of a spherical layer's table.
+static int upload_rowc(LayerRec &L, const float *coef) {
+  if (!L.sph) return 0;
+  static const int order[kRowCoef - 1] = {kR1, kR11, kR6, kR3, kR5, kF2, kF4};
+  std::vector<float> rows((size_t)kRowCoef * L.ny, 0.0f);
+  for (int j = 0; j < L.ny; ++j)
+    for (int k = 0; k < kRowCoef - 1; ++k)
+      rows[(size_t)j * kRowCoef + k] = coef[(size_t)order[k] * L.ny + j];
+  if (!L.rowc) HIPCHK(hipMalloc(&L.rowc, rows.size() * sizeof(float)));
+  HIPCHK(hipMemcpy(L.rowc, rows.data(), rows.size() * sizeof(float), hipMemcpyHostToDevice));
+  return 0;
+}
+
 int tree_upload_coef(LayerRec &L, const std::vector<float> &coef) {
   if (coef.size() != (size_t)kNumCoef * L.ny) return fail(9, "coefficient table size");
   HIPCHK(hipMemcpy(L.coef, coef.data(), coef.size() * sizeof(float), hipMemcpyHostToDevice));
-  return 0;
+  return upload_rowc(L, coef.data());
 }
 
 int tree_alloc_r24(LayerRec &L, const float *R2, const float *R4) {
@@ -289,6 +303,7 @@ DevLayer dev_view(const Tree &T, const LayerRec &L, bool with_max, bool advance)
   d.kfric = L.kfric;
   d.h = L.h;
   d.coef = L.coef;
+  d.rowc = L.rowc;
   d.r24 = L.r24;
   d.z1 = L.z[L.cur];
   d.m1 = L.m[L.cur];
@@ -707,6 +722,8 @@ int tree_checkpoint_load(Tree &T, hipStream_t st, const char *path, long long *d
     LayerRec &L = T.layers[c.id];
     HIPCHK(hipMemcpy(L.block, buf.data(), buf.size(), hipMemcpyHostToDevice));
     L.cur = c.cur;
+    const size_t at = (size_t)(reinterpret_cast<char *>(L.coef) - static_cast<char *>(L.block));
+    if (int e = upload_rowc(L, reinterpret_cast<const float *>(buf.data() + at))) return e;
   }
   const int n32 = (int)steps;
   const int ctl[2] = {n32, n32};

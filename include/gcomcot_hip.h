@@ -349,9 +349,12 @@ int gcomcot_output_flush_(long long *nfiles);
  * clears the per-layer choices.  Returns 0 or an error code. */
 int gcomcot_autotune_(int *reps, int *variant, int *blocking, float *ms_per_step);
 
-/* Two root steps per launch (temporal blocking) in gcomcot_run_steps_ for
- * a linear outermost layer without nested layers: *mode 0 = off, 1..7 =
- * on with tiles of 64x8, 32x16, 64x16 (256 threads), 64x16 (512 and 1024
+/* Several root steps per launch (temporal blocking) in gcomcot_run_steps_
+ * for a linear outermost layer without nested layers: *mode 0 = off; 1 =
+ * two or four steps per launch in the marching kernels where they apply (a
+ * spherical layer registered with its row table, no MAX_AMP maximum kept,
+ * planes within 4 GB), else as below; 1..7 = two steps per launch with
+ * tiles of 64x8, 32x16, 64x16 (256 threads), 64x16 (512 and 1024
  * threads), 32x16 (512 threads), 64x32 (1024 threads) (default 1; the
  * autotuner picks among them).  Results are bitwise
  * those of single steps; afterwards level 2 holds the state two steps

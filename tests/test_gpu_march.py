@@ -1,0 +1,58 @@
+"""The marching kernels (csrc/march.hip) against the oracle, bit for bit, at
+the sizes where their split can go wrong: layers narrower than a strip, one
+column either side of the strip widths (60 and 56 columns) and of a wave,
+layers of a few rows, a row count off every segment length, and step counts
+that end on every remainder of the launches' two and four steps."""
+import pytest
+
+from gcomcot import DeviceRun
+from gcomcot import scenarios as S
+from helpers import compare_device_oracle
+from oracle.bind import Oracle
+
+pytestmark = pytest.mark.gpu
+
+SIZES = [(8, 7), (24, 5), (55, 24), (57, 33), (60, 13), (61, 40), (64, 29), (65, 26), (112, 31),
+         (121, 17), (123, 50), (181, 9), (1150, 611)]
+
+
+@pytest.mark.parametrize("nx,ny", SIZES, ids=[f"{a}x{b}" for a, b in SIZES])
+def test_marched_layer_matches_oracle(nx, ny):
+    sc = S.custom(laycord=0, laygov=0, nx=nx, ny=ny, cx=0.4)
+    orc = Oracle(sc, 32, pow_mode=1)
+    dev = DeviceRun(sc)
+    try:
+        for n, graph in [(2, True), (3, True), (4, False), (5, True), (1, True), (6, True)] + \
+                ([(73, True)] if nx < 200 else [(135, True), (16, False)]):
+            print(f"[gpu] march {nx}x{ny} run {n} graph={graph}", flush=True)
+            dev.run(n, graph=graph)
+            orc.step(n)
+            compare_device_oracle(sc, dev, orc, f"march {nx}x{ny} after {n}")
+    finally:
+        dev.close()
+
+
+@pytest.mark.parametrize("nx,ny", [(2051, 1537), (4099, 1711)], ids=["2051x1537", "4099x1711"])
+def test_marched_large_layer_matches_tiles(nx, ny):
+    """Layers large enough for the longer segments, against the tile kernels
+    (one step per launch), which the oracle pins."""
+    import numpy as np
+    from gcomcot._lib import ip, lib
+    sc = S.linear_layer(nx=nx, ny=ny)
+    got = []
+    try:
+        for mode in (0, 1):
+            print(f"[gpu] march {nx}x{ny} mode {mode}", flush=True)
+            assert lib().gcomcot_set_temporal_blocking_(ip(mode)) == 0
+            dev = DeviceRun(sc)
+            dev.run(31)
+            dev.run(10, graph=False)
+            got.append((dev.state(1), dev.maxima(1)))
+            dev.close()
+    finally:
+        lib().gcomcot_set_temporal_blocking_(ip(1))
+    (a, am), (b, bm) = got
+    for k in ("z1", "m1", "n1"):
+        assert np.array_equal(a[k].view(np.int32), b[k].view(np.int32)), k
+    for k in ("zmax_wet", "arrival"):
+        assert np.array_equal(am[k].view(np.int32), bm[k].view(np.int32)), k
