@@ -7,8 +7,13 @@
 // a special-case fix-up (V_DIV_FIXUP).  The momentum kernels spend about a
 // fifth of their instructions on fourteen divisions per cell.
 //
-// div_inrange(a, b) is the same sequence without the scalings and the
-// fix-up.  V_DIV_SCALE leaves both operands unchanged, and V_DIV_FIXUP
+// div_inrange(a, b) is that sequence without the scalings, the fix-up and
+// the first residual correction.  The refined reciprocal is 1/b correctly
+// rounded for every b (all 2^23 significands, on the device), and then one
+// correction q + (a - b q)/b rounds to the IEEE quotient: before that
+// rounding it is within 2.3 * 2^-24 ulp of a/b, which leaves per divisor
+// only the numerators whose quotient comes that close to a midpoint; they
+// are all enumerated in tests/quotient_check.cpp, and none rounds wrongly.  V_DIV_SCALE leaves both operands unchanged, and V_DIV_FIXUP
 // passes the quotient through, unless b is 0, denormal or so large that
 // 1/b is, a is 0 or below 2^-103 in magnitude, a/b is below 2^-126 or the
 // exponents differ by 96 or more; for the other (a, b) the result is the
@@ -61,7 +66,7 @@ GC_FD_HD bool div_inrange_applies(float a, float b, float q) {
 
 #if defined(__HIPCC__) || defined(__HIP__)
 // div_inrange split in two: the refined reciprocal of b (three operations
-// that depend on b alone), and the quotient from it.  div_by(a, b,
+// that depend on b alone), and the quotient from it (three more).  div_by(a, b,
 // recip_refined(b)) is div_inrange(a, b) bit for bit, so quotients with one
 // divisor can share the first part.
 __device__ __forceinline__ float recip_refined(float b) {
@@ -70,11 +75,8 @@ __device__ __forceinline__ float recip_refined(float b) {
   return fmaf(e, y, y);
 }
 __device__ __forceinline__ float div_by(float a, float b, float y) {
-  float q = a * y;
-  const float r0 = fmaf(-b, q, a);
-  q = fmaf(r0, y, q);
-  const float r1 = fmaf(-b, q, a);
-  return fmaf(r1, y, q);
+  const float q = a * y;
+  return fmaf(fmaf(-b, q, a), y, q);
 }
 __device__ __forceinline__ float div_inrange(float a, float b) {
   return div_by(a, b, recip_refined(b));
@@ -97,6 +99,13 @@ __device__ __forceinline__ float sqrt_inrange(float x) {
   const float rp = fmaf(-sp, s, x);
   const float t = rm <= 0.0f ? sm : s;
   return rp > 0.0f ? sp : t;
+}
+
+// WAVE_BREAKING's threshold on |Z2 - Z1| is DT * 0.08 * sqrt(g D); this times
+// a hardware sqrt(D) is a safe lower bound of it (2^-12 below, against
+// rounding errors of 2^-21), and 0 where D is.
+__device__ __forceinline__ float breaking_floor(float dt) {
+  return 0.08f * 3.1316129f * 0.99975586f * dt;  // 0.08 sqrt(g) (1 - 2^-12) DT
 }
 #endif
 

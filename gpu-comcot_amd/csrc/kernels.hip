@@ -361,9 +361,15 @@ __device__ __forceinline__ float dq2_at(const DevLayer &L, const A &s, int i, in
 // range gives a quotient far below it either way; on a dry cell (DZ = 0,
 // DZDT_F = 0) only the quotient's sign matters, and both forms give +0 for
 // 0 and a positive value otherwise, whose size REF = DZDT/0 = +inf ignores.
+// zt = breaking_floor(DT): a surface that moved by no more than zt*sqrt(D)
+// (hardware square root, off by an ulp) moved by less than DZDT_F*DT, which
+// takes the square root, the quotient and the comparison of almost every
+// wave away (27 -> 8 instructions per cell); on a dry cell both are 0 and
+// any movement passes on to the exact test, as it must.
 template <class A>
 __device__ __forceinline__ float breaking_coef(const DevLayer &L, const A &s, int i, int j,
-                                               float rdt) {
+                                               float rdt, float zt) {
+  if (!(fabsf(s.Z2(i, j) - s.Z1(i, j)) > zt * __builtin_amdgcn_sqrtf(s.DZ(i, j)))) return 1.0f;
   float c = sqrt_inrange(kGrav * s.DZ(i, j));
   float dzdt_f = 0.08f * c;
   float dzdt_i = 0.65f * c;
@@ -460,8 +466,7 @@ __device__ float nl_x(const DevLayer &L, const A &s, int i, int j, float brk) {
   if (L.fric) XP = div_inrange(XP, 1.0f + FF);
   if (fabsf(XP) < kEps) XP = 0.0f;
   const float lim = kVLimit * DD;
-  if (XP > lim) XP = lim;
-  if (XP < -lim) XP = -lim;
+  if (fabsf(XP) > lim) XP = copysignf(lim, XP);
   return XP;
 }
 
@@ -550,8 +555,7 @@ __device__ float nl_y(const DevLayer &L, const A &s, int i, int j, float brk) {
   if (L.fric) XQ = div_inrange(XQ, 1.0f + FF);
   if (fabsf(XQ) < kEps) XQ = 0.0f;
   const float lim = kVLimit * DD;
-  if (XQ > lim) XQ = lim;
-  if (XQ < -lim) XQ = -lim;
+  if (fabsf(XQ) > lim) XQ = copysignf(lim, XQ);
   return XQ;
 }
 
@@ -723,7 +727,7 @@ __device__ __forceinline__ void tile_body(const DevLayer &L, int t, int ti0, int
     step = L.ctl[L.ctl_in] + 1;
     if (L.advance && t == 0 && tid == 0) L.ctl[1 - L.ctl_in] = step;
   }
-  const float rdt = recip_refined(L.dt);
+  const float rdt = recip_refined(L.dt), zt = breaking_floor(L.dt);
 #pragma unroll 1
   for (int idx = tid; idx < TX * TY; idx += kThreads) {
     const int i = ti0 + idx % TX, j = tj0 + idx / TX;
@@ -750,7 +754,7 @@ __device__ __forceinline__ void tile_body(const DevLayer &L, int t, int ti0, int
             IN || (r ? (i <= nx - 1 && j <= ny - 1) : (i >= 2 && i <= nx - 1 && j >= 2));
         const bool my =
             IN || (r ? (i <= nx - 1 && j <= ny - 1) : (i >= 2 && j >= 2 && j <= ny - 1));
-        const float brk = L.linchk == 1 ? breaking_coef(L, s, i, j, rdt) : 1.0f;
+        const float brk = L.linchk == 1 ? breaking_coef(L, s, i, j, rdt, zt) : 1.0f;
         m2v = mx ? nl_x<SPH, IN>(L, s, i, j, brk) : 0.0f;
         n2v = my ? nl_y<SPH, IN>(L, s, i, j, brk) : 0.0f;
       } else {
@@ -1242,7 +1246,7 @@ __global__ void __launch_bounds__(kThreads)
     if (L.advance && t == 0 && lane == 0) L.ctl[1 - L.ctl_in] = step;
   }
   const bool own = lane >= 2 && lane <= kStreamW - 3 && col_in;
-  const float rdt = recip_refined(L.dt);
+  const float rdt = recip_refined(L.dt), zt = breaking_floor(L.dt);
   for (int j = j0; j <= j1; ++j) {
     store_row(j + 2, ph, pm, pn);
     zq2 = pz;
@@ -1265,7 +1269,7 @@ __global__ void __launch_bounds__(kThreads)
       if (NL) {
         const bool mx = rt ? (i <= nx - 1 && j <= ny - 1) : (i >= 2 && i <= nx - 1 && j >= 2);
         const bool my = rt ? (i <= nx - 1 && j <= ny - 1) : (i >= 2 && j >= 2 && j <= ny - 1);
-        const float brk = L.linchk == 1 ? breaking_coef(L, r, i, j, rdt) : 1.0f;
+        const float brk = L.linchk == 1 ? breaking_coef(L, r, i, j, rdt, zt) : 1.0f;
         m2v = mx ? nl_x<SPH, false>(L, r, i, j, brk) : 0.0f;
         n2v = my ? nl_y<SPH, false>(L, r, i, j, brk) : 0.0f;
       } else {
