@@ -38,7 +38,10 @@ enum Coef {
   kR6,       // COS_N
   kNumCoef
 };
-// floats per row of the row-major copy that the marching kernels read
-constexpr int kRowCoef = 8;
+// The row-major copy that the marching kernels read: kRowCoef floats a row,
+// in groups of four (one scalar load each): continuity and R3; the X flux's
+// F2, 4 R3, R21, R0; the Y flux's F4, 4 R5, R22, R0; F2, F4, R5 of the linear
+// fluxes.
+constexpr int kRowCoef = 16;
 
 }  // namespace gc

@@ -4,6 +4,8 @@
 #include <hip/hip_runtime.h>
 #include <stddef.h>
 
+#include <algorithm>
+
 namespace gc {
 
 // What one step kernel needs of a layer.  Planes are column-major NX*NY
@@ -19,7 +21,7 @@ struct DevLayer {
   float kfric;     // (0.5*DT*GRAV)*FM*FM, the Fortran's CONST*FM*FM
   const float *h;
   const float *coef;   // per-row table (comcot_consts.h), spherical only
-  const float *rowc;   // R1, R11, R6, R3, R5, F2, F4, 0 of each row (kRowCoef floats a row)
+  const float *rowc;   // row-major copy of the coefficients (comcot_consts.h, kRowCoef floats a row)
   const float *r24;    // optional R2|R4 planes (drop-in fallback), else null
   const float *z1, *m1, *n1;
   float *z2, *m2, *n2;
@@ -72,6 +74,20 @@ constexpr int kStep2Shapes = 7;
 // tile of two-step shape `shape`
 void step2_shape(int shape, int *tx, int *ty);
 
+// Bytes from a layer's depth plane to the end of its last plane; the
+// descriptor of the marching kernels spans them.  ~0 if a plane lies before.
+inline unsigned long long block_span(const DevLayer &L) {
+  const char *lo = reinterpret_cast<const char *>(L.h), *hi = lo;
+  for (const void *p : {(const void *)L.z1, (const void *)L.m1, (const void *)L.n1,
+                        (const void *)L.z2, (const void *)L.m2, (const void *)L.n2,
+                        (const void *)L.zmax, (const void *)L.arrival})
+    if (p) {
+      if (reinterpret_cast<const char *>(p) < lo) return ~0ull;
+      hi = std::max(hi, reinterpret_cast<const char *>(p));
+    }
+  return (unsigned long long)(hi - lo) + 4ull * L.nx * L.ny;
+}
+
 // Root steps of a spherical linear outermost layer without children in the
 // marching kernels (march.hip): 2 or 4 per launch, level 1 in, level 2 out,
 // bookkeeping as launch_step2.  march_plan gives the steps per launch that
@@ -82,8 +98,20 @@ struct MarchPlan {
   int steps, seg, seg_side;
 };
 MarchPlan march_plan(int nx, int ny);
-bool march_applies(const DevLayer &L);
+inline bool march_applies(const DevLayer &L) {
+  return L.is_root && L.rowc && !L.r24 && !L.zraw && !L.sponge_cx && block_span(L) < 0xffffffffull;
+}
 hipError_t launch_march_linear(const DevLayer &L, int steps, hipStream_t st);
+
+// One fused step of a nonlinear layer with friction and convection in the
+// marching kernels (march_nl.hip), in segments of seg rows; march_nl_seg
+// gives the segments that suit a layer, 0 where the LDS tiles are faster.
+inline bool march_nl_applies(const DevLayer &L, bool sph) {
+  return (!sph || L.rowc) && L.modscm == 1 && L.linchk == 1 && L.fric && !L.r24 && !L.zraw &&
+         !L.sponge_cx && block_span(L) < 0xffffffffull;
+}
+int march_nl_seg(int nx, int ny);
+hipError_t launch_march_nl(const DevLayer &L, bool sph, int seg, hipStream_t st);
 
 // Reference-semantics maximum (no wet test) plus the wet max/arrival.
 hipError_t launch_max(const DevLayer &L, float *zmax_raw, hipStream_t st);

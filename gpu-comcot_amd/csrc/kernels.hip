@@ -1146,175 +1146,6 @@ __global__ void __launch_bounds__(NT)
   else tile_body2<SPH, TX, TY, false, NT, false, !SPH>(L, t, ti0, tj0, sm, &stab);
 }
 
-// ---------------------------------------------------------- strip kernel
-// The fused step as a strip marching along J: a workgroup owns 252
-// interior columns (256 lanes, two halo lanes each side) and a segment of
-// rows.  Each iteration stores one prefetched input row into LDS row rings,
-// computes continuity for the row two ahead, prefetches the next input row
-// and computes the fluxes of the current row.  Halo overhead is ~1.6 % of
-// columns and (SEG+4)/SEG of rows, against (TX+4)(TY+4)/(TX*TY) for a tile.
-constexpr int kStreamW = 256;
-constexpr int kStreamI = kStreamW - 4;
-
-struct Ring {
-  float *m1, *n1, *h, *z2, *dz;  // m1/n1/h: 6 rows, z2/dz: 5 rows of kStreamW
-  int gi0;                       // global column of lane 0
-  float z1own;                   // Z1 of the calling thread's own cell
-  const gcdet::Tables *tab;      // pow/exp tables, LDS copy
-  __device__ __forceinline__ int o6(int i, int j) const {
-    return ((j + 12) % 6) * kStreamW + (i - gi0);
-  }
-  __device__ __forceinline__ int o5(int i, int j) const {
-    return ((j + 10) % 5) * kStreamW + (i - gi0);
-  }
-  __device__ __forceinline__ float M(int i, int j) const { return m1[o6(i, j)]; }
-  __device__ __forceinline__ float N(int i, int j) const { return n1[o6(i, j)]; }
-  __device__ __forceinline__ float H(int i, int j) const { return h[o6(i, j)]; }
-  __device__ __forceinline__ float Z2(int i, int j) const { return z2[o5(i, j)]; }
-  __device__ __forceinline__ float DZ(int i, int j) const { return dz[o5(i, j)]; }
-  // Z1 is only ever read at the thread's own cell (continuity, breaking)
-  __device__ __forceinline__ float Z1(int, int) const { return z1own; }
-  __device__ __forceinline__ float CF(const DevLayer &L, int k, int j) const {
-    return L.coef[k * L.ny + (j - 1)];
-  }
-};
-
-template <bool NL, bool SPH>
-__global__ void __launch_bounds__(kThreads)
-    __attribute__((amdgpu_waves_per_eu(
-        StepWaves<NL, SPH, (int)((6 * 3 + 5 * 2) * kStreamW * sizeof(float) + sizeof(gcdet::Tables))>::value)))
-    k_stream(DevLayer L, int nstrip, int nseg, int seg, int per_xcd) {
-  __shared__ float sm[(6 * 3 + 5 * 2) * kStreamW];
-  const int t = tile_of_block(per_xcd);
-  if (t >= nstrip * nseg) return;
-  const int strip = t / nseg, sg = t % nseg;
-  const int nx = L.nx, ny = L.ny;
-  const int c0 = strip * kStreamI + 1;
-  const int j0 = sg * seg + 1;
-  const int j1 = min(j0 + seg - 1, ny);
-  const int lane = threadIdx.x;
-  const int gi = c0 - 2 + lane;
-  const bool col_in = gi >= 1 && gi <= nx;
-  __shared__ gcdet::Tables stab;
-  Ring r{sm, sm + 6 * kStreamW, sm + 12 * kStreamW, sm + 18 * kStreamW, sm + 23 * kStreamW,
-         c0 - 2, 0.0f, &stab};
-  if (NL || !SPH) stage_tables(stab, lane);
-
-  auto load_row = [&](int j, float &h, float &m, float &n, float &z) {
-    const bool in = col_in && j >= 1 && j <= ny;
-    const size_t g = in ? (size_t)(j - 1) * nx + (gi - 1) : 0;
-    h = in ? L.h[g] : 0.0f;
-    m = in ? L.m1[g] : 0.0f;
-    n = in ? L.n1[g] : 0.0f;
-    z = in ? L.z1[g] : 0.0f;
-  };
-  auto store_row = [&](int j, float h, float m, float n) {
-    const int o = r.o6(gi, j);
-    r.h[o] = h;
-    r.m1[o] = m;
-    r.n1[o] = n;
-  };
-  // lane 0 has no left neighbour in LDS; its Z2 is never read
-  auto mass_row = [&](int j, float z1) {
-    float z2 = 0.0f, dz2 = 0.0f;
-    if (col_in && lane >= 1 && j >= 1 && j <= ny) {
-      r.z1own = z1;
-      mass_cell<NL, SPH, false>(L, r, gi, j, z2, dz2);
-    }
-    const int o = r.o5(gi, j);
-    r.z2[o] = z2;
-    r.dz[o] = dz2;
-  };
-
-  float zp[4];
-  {
-    float h, m, n;
-    for (int k = 0; k < 4; ++k) {
-      load_row(j0 - 2 + k, h, m, n, zp[k]);
-      store_row(j0 - 2 + k, h, m, n);
-    }
-  }
-  __syncthreads();
-  for (int k = 1; k < 4; ++k) mass_row(j0 - 2 + k, zp[k]);
-  float zq0 = zp[2], zq1 = zp[3], zq2 = 0.0f;
-  float ph, pm, pn, pz;
-  load_row(j0 + 2, ph, pm, pn, pz);
-
-  int step = 0;
-  if (L.zmax) {
-    step = L.ctl[L.ctl_in] + 1;
-    if (L.advance && t == 0 && lane == 0) L.ctl[1 - L.ctl_in] = step;
-  }
-  const bool own = lane >= 2 && lane <= kStreamW - 3 && col_in;
-  const float rdt = recip_refined(L.dt), zt = breaking_floor(L.dt);
-  for (int j = j0; j <= j1; ++j) {
-    store_row(j + 2, ph, pm, pn);
-    zq2 = pz;
-    __syncthreads();
-    mass_row(j + 2, zq2);
-    __syncthreads();
-    load_row(j + 3, ph, pm, pn, pz);
-    if (own) {
-      const int i = gi;
-      const size_t g = (size_t)(j - 1) * nx + (i - 1);
-      const bool rt = L.is_root;
-      float zo;
-      if (rt || (i >= 2 && j >= 2)) zo = r.Z2(i, j);
-      else if (i == 1 && j == 1) zo = r.Z2(2, 2);  // UPDATE ghosts, all_grids.f90:323-324
-      else if (i == 1) zo = r.Z2(2, j);
-      else zo = r.Z2(i, 2);
-      st_plane<false>(L.z2 + g, zo);
-      r.z1own = zq0;
-      float m2v, n2v;
-      if (NL) {
-        const bool mx = rt ? (i <= nx - 1 && j <= ny - 1) : (i >= 2 && i <= nx - 1 && j >= 2);
-        const bool my = rt ? (i <= nx - 1 && j <= ny - 1) : (i >= 2 && j >= 2 && j <= ny - 1);
-        const float brk = L.linchk == 1 ? breaking_coef(L, r, i, j, rdt, zt) : 1.0f;
-        m2v = mx ? nl_x<SPH, false>(L, r, i, j, brk) : 0.0f;
-        n2v = my ? nl_y<SPH, false>(L, r, i, j, brk) : 0.0f;
-      } else {
-        const int lo = rt ? 1 : 2;
-        const bool mx = i >= lo && i <= nx - 1 && j >= lo;
-        const bool my = j >= lo && j <= ny - 1 && i >= lo;
-        m2v = mx ? lin_x<SPH, false>(L, r, i, j) : 0.0f;
-        n2v = my ? lin_y<SPH, false>(L, r, i, j) : 0.0f;
-      }
-      if (L.sponge_cx) {
-        const float cx = L.sponge_cx[i - 1], cy = L.sponge_cy[j - 1];
-        if (cx > 0.0f || cy > 0.0f) {
-          m2v = m2v + cx * L.dt * r.M(i, j);
-          n2v = n2v + cy * L.dt * r.N(i, j);
-        }
-      }
-      st_plane<false>(L.m2 + g, m2v);
-      st_plane<false>(L.n2 + g, n2v);
-      if (L.zmax && (rt || (i >= 2 && j >= 2))) {
-        const float z2 = r.Z2(i, j);
-        if (r.H(i, j) + z2 > kGx) {
-          const float zm = L.zmax[g];
-          if (z2 >= L.arr_thr && !(zm >= L.arr_thr)) L.arrival[g] = step;
-          if (z2 > zm) L.zmax[g] = z2;
-        }
-      }
-      if (L.zraw) {
-        const float z2 = r.Z2(i, j);
-        if (!(L.zraw[g] >= z2)) L.zraw[g] = z2;
-      }
-    }
-    zq0 = zq1;
-    zq1 = zq2;
-  }
-}
-
-template <bool NL, bool SPH>
-hipError_t launch_stream(const DevLayer &L, int seg, hipStream_t st) {
-  const int ns = (L.nx + kStreamI - 1) / kStreamI, ng = (L.ny + seg - 1) / seg;
-  const int nt = ns * ng, per = (nt + 7) / 8;
-  hipLaunchKernelGGL((k_stream<NL, SPH>), dim3(8 * per), dim3(kThreads), 0, st, L, ns, ng, seg,
-                     per);
-  return hipGetLastError();
-}
-
 // Reference maximum recorder (GPUOutput.cu:46-53 semantics: no wet test)
 // plus the wet maximum / arrival of the extension, for maxamp_launch_.
 __global__ void k_max(DevLayer L, float *zmax_raw) {
@@ -2093,27 +1924,30 @@ hipError_t launch2_t(const DevLayer &L, hipStream_t st) {
   return hipGetLastError();
 }
 
-// Fused-step launch shapes: LDS tiles TX x TY (variants 0-5; 0 is the
-// default), then the strip kernel with SEG rows per segment (6-10).
-const int kVariants[][3] = {{1, 64, 8},   {1, 64, 16},  {1, 32, 32},  {1, 128, 8},
-                            {1, 64, 32},  {1, 32, 16},  {0, 256, 32}, {0, 256, 16},
-                            {0, 256, 24}, {0, 256, 48}, {0, 256, 64}};
+// Fused-step launch shapes: LDS tiles TX x TY (variants 0-5), then marching
+// strips with SEG rows per segment (6-10) for the nonlinear layers that can
+// take them (others: 64x8 tiles).  Variant 0, the default, is the marching
+// form too where march_nl_seg gives a segment.
+const int kVariants[][3] = {{1, 64, 8},  {1, 64, 16}, {1, 32, 32}, {1, 128, 8}, {1, 64, 32}, {1, 32, 16},
+                            {0, 60, 32}, {0, 60, 14}, {0, 60, 20}, {0, 60, 8},  {0, 60, 44}};
 
 }  // namespace
 
 int num_tile_variants() { return (int)(sizeof(kVariants) / sizeof(kVariants[0])); }
 void tile_variant_shape(int v, int *tx, int *ty) {
-  *tx = kVariants[v][0] ? kVariants[v][1] : -kVariants[v][1];  // negative: strip kernel
+  *tx = kVariants[v][0] ? kVariants[v][1] : -kVariants[v][1];  // negative: marching strips
   *ty = kVariants[v][2];
 }
 
 hipError_t launch_step(const DevLayer &L, int mode, bool nl, bool sph, int variant,
                        hipStream_t st) {
   if (variant < 0 || variant >= num_tile_variants()) return hipErrorInvalidValue;
-  if (mode == kFused && kVariants[variant][0] == 0) {
-    const int seg = kVariants[variant][2];
-    if (nl) return sph ? launch_stream<true, true>(L, seg, st) : launch_stream<true, false>(L, seg, st);
-    return sph ? launch_stream<false, true>(L, seg, st) : launch_stream<false, false>(L, seg, st);
+  if (mode == kFused && kVariants[variant][0] == 0 && !(nl && march_nl_applies(L, sph))) variant = 0;
+  if (mode == kFused && nl && march_nl_applies(L, sph)) {
+    const int seg = kVariants[variant][0] == 0 ? kVariants[variant][2]
+                    : variant == 0             ? march_nl_seg(L.nx, L.ny)
+                                               : 0;
+    if (seg > 0) return launch_march_nl(L, sph, seg, st);
   }
   if (mode == kMomentMass) {  // outermost linear layers with nested layers: 64x8
     if (nl) return hipErrorInvalidValue;

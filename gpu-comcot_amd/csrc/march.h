@@ -1,0 +1,85 @@
+// What the marching kernels (march.hip, march_nl.hip) share: a wavefront
+// holds a strip of 64 columns, one per lane, and marches along J with its
+// rows in registers.
+#pragma once
+
+#include <hip/hip_runtime.h>
+
+#include <algorithm>
+
+#include "comcot_consts.h"
+#include "kernels.h"
+
+namespace gc {
+
+constexpr int kWave = 64;
+constexpr int kMarchBlock = 256;
+
+// Value of the lane one column to the west (I - 1) / east (I + 1); the
+// outermost lane of the wave gets 0 (its results are never stored).
+__device__ __forceinline__ float west(float v) {
+  return __int_as_float(
+      __builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x138, 0xf, 0xf, true));
+}
+__device__ __forceinline__ float east(float v) {
+  return __int_as_float(
+      __builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x130, 0xf, 0xf, true));
+}
+
+// Planes are read and written through one buffer descriptor over the
+// layer's block (every plane of a layer lies in one allocation, behind its
+// depth plane): a lane's column is the vector offset, plane and row the
+// scalar one, so rows cost no per-lane address arithmetic.  A lane that has
+// nothing to store gives offset kNoStore, which the descriptor's range check
+// drops: the row loop has no branch around a store.  (With branches the
+// compiler has to assume the shorter path when it counts outstanding memory
+// operations, and a wait for the next row's loads then also waits for
+// stores.)
+typedef __amdgpu_buffer_rsrc_t Block;
+constexpr int kNoStore = -1;
+__device__ __forceinline__ Block block_of(const DevLayer &L, unsigned bytes) {
+  return __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(L.h), 0, bytes, 0x00027000);
+}
+__device__ __forceinline__ unsigned plane_off(const DevLayer &L, const void *p) {
+  return (unsigned)(reinterpret_cast<unsigned long long>(p) -
+                    reinterpret_cast<unsigned long long>(L.h));
+}
+__device__ __forceinline__ float get(Block b, int voff, unsigned soff) {
+  return __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(b, voff, (int)soff, 0));
+}
+template <bool ST>
+__device__ __forceinline__ void put(Block b, int voff, unsigned soff, float v) {
+  __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(v), b, voff, (int)soff, ST ? 2 : 0);
+}
+
+// A lane mask held in scalar registers as this lane's condition.
+__device__ __forceinline__ bool lanes(unsigned long long m) {
+  return __builtin_amdgcn_inverse_ballot_w64(m);
+}
+
+// Work of one wave: the first column and the rows j0..j1 it writes.
+struct Strip {
+  int c0, j0, j1;
+};
+
+// Group g of the row coefficients of row j (kRowCoef), by one scalar load
+// (constant address space: nothing writes the table while kernels run).
+typedef float Row4 __attribute__((ext_vector_type(4)));
+__device__ __forceinline__ Row4 row_coef(const DevLayer &L, int j, int g) {
+  typedef const __attribute__((address_space(4))) Row4 *ConstPtr;
+  const int q = (j < 1 ? 1 : (j > L.ny ? L.ny : j)) - 1;
+  return ((ConstPtr)(unsigned long long)L.rowc)[(size_t)q * (kRowCoef / 4) + g];
+}
+
+// OPEN (boundaries.f90:22-202) at one ring cell: a, b are the two flux
+// components it combines (an average along the edge or a corner's own
+// flux, and the flux across), cc = sqrt(g H), neg says which way the wave
+// leaves.
+__device__ __forceinline__ float radiate(float h, float cc, float a, float b, bool neg) {
+  float zz = sqrtf(a * a + b * b) / cc;
+  if (neg) zz = -zz;
+  if (fabsf(zz) > kUB) zz = 0.0f;
+  return h > kGx ? zz : 0.0f;
+}
+
+}  // namespace gc

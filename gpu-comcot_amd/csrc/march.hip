@@ -25,84 +25,11 @@
 
 #include "comcot_consts.h"
 #include "kernels.h"
+#include "march.h"
 
 namespace gc {
 
 namespace {
-
-constexpr int kWave = 64;
-constexpr int kMarchBlock = 256;
-
-// Value of the lane one column to the west (I - 1) / east (I + 1); the
-// outermost lane of the wave gets 0 (its results are never stored).
-__device__ __forceinline__ float west(float v) {
-  return __int_as_float(
-      __builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x138, 0xf, 0xf, true));
-}
-__device__ __forceinline__ float east(float v) {
-  return __int_as_float(
-      __builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x130, 0xf, 0xf, true));
-}
-
-// Planes are read and written through one buffer descriptor over the
-// layer's block (every plane of a layer lies in one allocation, behind its
-// depth plane): a lane's column is the vector offset, plane and row the
-// scalar one, so rows cost no per-lane address arithmetic.  A lane that has
-// nothing to store gives offset kNoStore, which the descriptor's range check
-// drops: the row loop has no branch around a store.  (With branches the
-// compiler has to assume the shorter path when it counts outstanding memory
-// operations, and a wait for the next row's loads then also waits for
-// stores.)
-typedef __amdgpu_buffer_rsrc_t Block;
-constexpr int kNoStore = -1;
-__device__ __forceinline__ Block block_of(const DevLayer &L, unsigned bytes) {
-  return __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(L.h), 0, bytes, 0x00027000);
-}
-__device__ __forceinline__ unsigned plane_off(const DevLayer &L, const void *p) {
-  return (unsigned)(reinterpret_cast<unsigned long long>(p) -
-                    reinterpret_cast<unsigned long long>(L.h));
-}
-__device__ __forceinline__ float get(Block b, int voff, unsigned soff) {
-  return __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(b, voff, (int)soff, 0));
-}
-template <bool ST>
-__device__ __forceinline__ void put(Block b, int voff, unsigned soff, float v) {
-  __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(v), b, voff, (int)soff, ST ? 2 : 0);
-}
-
-// A lane mask held in scalar registers as this lane's condition.
-__device__ __forceinline__ bool lanes(unsigned long long m) {
-  return __builtin_amdgcn_inverse_ballot_w64(m);
-}
-
-// Work of one wave: lane 0's column, rows j0..j1 to write.
-struct Strip {
-  int c0, j0, j1;
-};
-
-// Row coefficients of MASS_S / MOMT_S at one row: one scalar load of eight
-// floats (constant address space: nothing writes the table while kernels
-// run).
-struct RowCoef {
-  float r1, r11, r6, r3, r5, f2, f4;
-};
-__device__ __forceinline__ RowCoef row_coef(const DevLayer &L, int j) {
-  typedef float Row8 __attribute__((ext_vector_type(kRowCoef)));
-  typedef const __attribute__((address_space(4))) Row8 *ConstPtr;
-  const Row8 c = ((ConstPtr)(unsigned long long)L.rowc)[(j < 1 ? 1 : (j > L.ny ? L.ny : j)) - 1];
-  return {c[0], c[1], c[2], c[3], c[4], c[5], c[6]};
-}
-
-// OPEN (boundaries.f90:22-202) at one ring cell: a, b are the two flux
-// components it combines (an average along the edge or a corner's own
-// flux, and the flux across), cc = sqrt(g H), neg says which way the wave
-// leaves.
-__device__ __forceinline__ float radiate(float h, float cc, float a, float b, bool neg) {
-  float zz = sqrtf(a * a + b * b) / cc;
-  if (neg) zz = -zz;
-  if (fabsf(zz) > kUB) zz = 0.0f;
-  return h > kGx ? zz : 0.0f;
-}
 
 // K linear root steps of strip S.  COL: the strip holds column I = 1 or NX
 // or its halo leaves the grid there; ROW: the same for rows.  Loads are
@@ -144,7 +71,8 @@ __device__ __forceinline__ void march_linear(const DevLayer &L, const Strip S, i
   float zl[K];
   int below[K];
   unsigned long long wet[K + 1];  // lane masks of H > GX
-  RowCoef C[K + 1];
+  // row coefficients: R1 R11 R6 R3, and F2 F4 R5
+  Row4 C[K + 1], E[K + 1];
 #pragma unroll
   for (int s = 0; s <= K; ++s) Z[s] = M[s] = H[s] = R4[s] = 0.0f, wet[s] = 0;
 #pragma unroll
@@ -154,7 +82,7 @@ __device__ __forceinline__ void march_linear(const DevLayer &L, const Strip S, i
     below[s] = 0;
   }
 #pragma unroll
-  for (int s = 0; s <= K; ++s) C[s] = row_coef(L, ra);
+  for (int s = 0; s <= K; ++s) C[s] = row_coef(L, ra, 0), E[s] = row_coef(L, ra, 3);
 
   float ph[D], pz[D], pm[D], pn[D], pq[D];
   auto load = [&](int j, int k) {
@@ -167,7 +95,7 @@ __device__ __forceinline__ void march_linear(const DevLayer &L, const Strip S, i
   };
 #pragma unroll
   for (int k = 0; k < D; ++k) load(ra + k, k);
-  RowCoef cnext = row_coef(L, ra);
+  Row4 cnext = row_coef(L, ra, 0), enext = row_coef(L, ra, 3);
 
   auto row = [&](int r, int k) __attribute__((always_inline)) {  // k: the row's load slot
     // ---- row r enters: shift the per-row values down
@@ -175,6 +103,7 @@ __device__ __forceinline__ void march_linear(const DevLayer &L, const Strip S, i
     for (int s = K; s > 0; --s) {
       H[s] = H[s - 1];
       C[s] = C[s - 1];
+      E[s] = E[s - 1];
       R4[s] = R4[s - 1];
       wet[s] = wet[s - 1];
     }
@@ -189,19 +118,21 @@ __device__ __forceinline__ void march_linear(const DevLayer &L, const Strip S, i
       }
     }
     C[0] = cnext;
+    E[0] = enext;
     const float h = ph[k];
     float zc = pz[k], mc = pm[k], nc = pn[k];
     if (MX) {
       zm[0] = zl[0] = pq[k];
       below[0] = 0;
     }
-    cnext = row_coef(L, r + 1);
+    cnext = row_coef(L, r + 1, 0);
+    enext = row_coef(L, r + 1, 3);
     load(r + D, k);
     const float he = east(h);
     H[0] = h;
     wet[0] = __builtin_amdgcn_ballot_w64(h > kGx);
-    R2[0] = C[0].f2 * (0.5f * (h + he));   // used where both cells are wet: HP > 0
-    R4[1] = C[1].f4 * (0.5f * (H[1] + h));
+    R2[0] = E[0][0] * (0.5f * (h + he));   // used where both cells are wet: HP > 0
+    R4[1] = E[1][1] * (0.5f * (H[1] + h));
     if (COL) CC[0] = sqrtf(kGrav * h);
 
 #pragma unroll
@@ -209,9 +140,9 @@ __device__ __forceinline__ void march_linear(const DevLayer &L, const Strip S, i
       const int q = r - s;
       const float hq = H[s];
       // continuity
-      const float nr = nc * C[s].r6;
+      const float nr = nc * C[s][2];
       const float mw = west(mc);
-      float zz = zc - C[s].r1 * (mc - mw) - C[s].r11 * (nr - NRb[s]);
+      float zz = zc - C[s][0] * (mc - mw) - C[s][1] * (nr - NRb[s]);
       if (fabsf(zz) < kEps) zz = 0.0f;
       const float t = zz + hq;
       float zn = t <= kEps ? -hq : zz;
@@ -240,7 +171,7 @@ __device__ __forceinline__ void march_linear(const DevLayer &L, const Strip S, i
       // momentum: M at row q, N at row q - 1
       const float ns = ROW && q == 1 ? nc : Nb[s];
       const float tn = nc + east(nc) + ns + east(ns);
-      float mn = mc - R2[s] * (east(zn) - zn) + C[s].r3 * tn;
+      float mn = mc - R2[s] * (east(zn) - zn) + C[s][3] * tn;
       // M(I) needs I and I + 1 wet; |M| < EPS goes to 0
       mn = lanes(wet[s] & (wet[s] >> 1) & ~__builtin_amdgcn_ballot_w64(fabsf(mn) < kEps)) ? mn : 0.0f;
       if (COL) mn = east_end ? 0.0f : mn;
@@ -248,7 +179,7 @@ __device__ __forceinline__ void march_linear(const DevLayer &L, const Strip S, i
       float sw = west(sum);
       if (COL) sw = west_end ? sum : sw;
       const float tm = sw + Mb[s] + mc;
-      float nn = Nb[s] - R4[s + 1] * (zn - Z[s + 1]) - C[s + 1].r5 * tm;
+      float nn = Nb[s] - R4[s + 1] * (zn - Z[s + 1]) - E[s + 1][2] * tm;
       nn = lanes(wet[s + 1] & wet[s] & ~__builtin_amdgcn_ballot_w64(fabsf(nn) < kEps)) ? nn : 0.0f;
       if (ROW && q - 1 == ny) nn = 0.0f;
       if (MX) {  // wet maximum and first arrival of step s + 1 at row q
@@ -336,20 +267,6 @@ __global__ void __launch_bounds__(kMarchBlock) k_march_linear(DevLayer L, MarchG
   else march_linear<K, false, false, MX, ST>(L, S, step, block_bytes);
 }
 
-// Bytes from a layer's depth plane to the end of its last plane; the
-// descriptor of the marching kernels spans them.  ~0 if a plane lies before.
-unsigned long long block_span(const DevLayer &L) {
-  const char *lo = reinterpret_cast<const char *>(L.h), *hi = lo;
-  for (const void *p : {(const void *)L.z1, (const void *)L.m1, (const void *)L.n1,
-                        (const void *)L.z2, (const void *)L.m2, (const void *)L.n2,
-                        (const void *)L.zmax, (const void *)L.arrival})
-    if (p) {
-      if (reinterpret_cast<const char *>(p) < lo) return ~0ull;
-      hi = std::max(hi, reinterpret_cast<const char *>(p));
-    }
-  return (unsigned long long)(hi - lo) + 4ull * L.nx * L.ny;
-}
-
 template <int K, bool MX, bool ST>
 hipError_t launch_k(const DevLayer &L, int seg, int seg_side, hipStream_t st) {
   constexpr int W = kWave - 2 * K, WB = kMarchBlock / kWave;
@@ -403,10 +320,6 @@ MarchPlan march_plan(int nx, int ny) {
   p.seg = rows < 32 ? 8 : (rows < 120 ? 12 : 24);
   p.seg_side = rows < 120 ? 4 : 12;
   return p;
-}
-
-bool march_applies(const DevLayer &L) {
-  return L.is_root && L.rowc && !L.r24 && !L.zraw && !L.sponge_cx && block_span(L) < 0xffffffffull;
 }
 
 hipError_t launch_march_linear(const DevLayer &L, int steps, hipStream_t st) {

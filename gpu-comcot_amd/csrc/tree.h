@@ -34,7 +34,7 @@ struct LayerRec {
   float *zmax_raw = nullptr, *zmax_wet = nullptr, *coef = nullptr, *r24 = nullptr;
   float *dzp = nullptr, *xflux = nullptr, *yflux = nullptr;
   int *arrival = nullptr;
-  float *rowc = nullptr;    // row-major copy of seven coefficients (DevLayer::rowc)
+  float *rowc = nullptr;    // row-major copy of the coefficients (DevLayer::rowc)
   float *deform = nullptr;  // last seafloor deformation applied (on first use)
   float *sponge = nullptr;  // SPONGE_COEF: COEFX[NX] then COEFY[NY] (layer 1, when on)
   // SC_OPTION = 1 (Cartesian child of a spherical layer 1): POS, CXY, the

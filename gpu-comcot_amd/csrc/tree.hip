@@ -254,11 +254,15 @@ int tree_create_layer(Tree &T, hipStream_t st, int id, int parent, int level, in
 // The row-major copy of a spherical layer's table.
 static int upload_rowc(LayerRec &L, const float *coef) {
   if (!L.sph) return 0;
-  static const int order[kRowCoef - 1] = {kR1, kR11, kR6, kR3, kR5, kF2, kF4};
   std::vector<float> rows((size_t)kRowCoef * L.ny, 0.0f);
-  for (int j = 0; j < L.ny; ++j)
-    for (int k = 0; k < kRowCoef - 1; ++k)
-      rows[(size_t)j * kRowCoef + k] = coef[(size_t)order[k] * L.ny + j];
+  for (int j = 0; j < L.ny; ++j) {
+    auto c = [&](int k) { return coef[(size_t)k * L.ny + j]; };
+    const float row[kRowCoef] = {c(kR1), c(kR11), c(kR6),        c(kR3),   // times 4 is exact
+                                 c(kF2), 4.0f * c(kR3), c(kR21), c(kR0),
+                                 c(kF4), 4.0f * c(kR5), c(kR22), c(kR0),
+                                 c(kF2), c(kF4),        c(kR5),  0.0f};
+    std::copy(row, row + kRowCoef, rows.begin() + (size_t)j * kRowCoef);
+  }
   if (!L.rowc) HIPCHK(hipMalloc(&L.rowc, rows.size() * sizeof(float)));
   HIPCHK(hipMemcpy(L.rowc, rows.data(), rows.size() * sizeof(float), hipMemcpyHostToDevice));
   return 0;

@@ -56,3 +56,51 @@ def test_marched_large_layer_matches_tiles(nx, ny):
         assert np.array_equal(a[k].view(np.int32), b[k].view(np.int32)), k
     for k in ("zmax_wet", "arrival"):
         assert np.array_equal(am[k].view(np.int32), bm[k].view(np.int32)), k
+
+
+NL_SIZES = [(24, 9), (59, 30), (61, 33), (121, 47), (133, 61), (194, 59), (253, 74), (312, 45)]
+
+
+@pytest.mark.parametrize("laycord", [0, 1], ids=["sph", "cart"])
+@pytest.mark.parametrize("nx,ny", NL_SIZES, ids=[f"{a}x{b}" for a, b in NL_SIZES])
+def test_marched_nonlinear_layer_matches_oracle(nx, ny, laycord):
+    """Nonlinear layers in marching strips of every segment length, on beaches
+    that flood and break: side strips, end rows and middle segments."""
+    from gcomcot._lib import ip, lib
+    from helpers import BEACH, surf_zone
+    for sc in (S.custom(laycord=laycord, laygov=1, nx=nx, ny=ny, **BEACH),
+               surf_zone(laycord, nx=nx, ny=ny)):
+        orc = Oracle(sc, 32, pow_mode=1)
+        orc.step(40)
+        try:
+            for v in (6, 7, 9):
+                print(f"[gpu] march {sc.name} variant {v}", flush=True)
+                assert lib().gcomcot_set_tile_variant_(ip(v)) == 0
+                dev = DeviceRun(sc)
+                dev.run(40)
+                compare_device_oracle(sc, dev, orc, f"{sc.name} variant {v}")
+                dev.close()
+        finally:
+            lib().gcomcot_set_tile_variant_(ip(0))
+
+
+@pytest.mark.parametrize("clc", [0, 1], ids=["sph-child", "cart-child"])
+def test_marched_child_matches_oracle(clc):
+    """A nested layer wide and tall enough for middle segments: ghost row and
+    column, and the ranges of inner layers."""
+    from gcomcot._lib import ip, lib
+    from helpers import BEACH
+    sc = S.custom(nx=110, ny=84, laygov=0, child=dict(laycord=clc, laygov=1, footprint=(51, 41),
+                                                      rel_size=4, rel_time=3, corner=(8, 14)), **BEACH)
+    orc = Oracle(sc, 32, pow_mode=1)
+    orc.step(25)
+    try:
+        for v in (6, 7, 8, 9, 10):
+            print(f"[gpu] march child {clc} variant {v}", flush=True)
+            assert lib().gcomcot_set_tile_variant_(ip(v)) == 0
+            dev = DeviceRun(sc)
+            dev.run(25)
+            compare_device_oracle(sc, dev, orc, f"child {clc} variant {v}")
+            dev.close()
+    finally:
+        lib().gcomcot_set_tile_variant_(ip(0))
