@@ -1884,6 +1884,34 @@ __global__ void __launch_bounds__(NT)
   else tile_body2<SPH, TX, TY, false, NT, false, !SPH>(L, t, ti0, tj0, sm, &stab);
 }
 
+// The fused nonlinear step of layers too small to fill the chip: 32 x 8
+// tiles, one cell per thread.  Such a launch lasts as long as one thread's
+// chain of dependent operations (some 500 per cell at about 8 cycles each),
+// so the second cell of a 64 x 8 tile's thread costs more than the halo it
+// saves, and the smallest layers do not need the eight waves per SIMD that
+// the register limit of the large ones buys.
+template <bool SPH, int WAVES, bool ST>
+__global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(WAVES)))
+    k_step_small(DevLayer L, int tiles_x, int ntiles, int per_xcd) {
+  constexpr int TX = 32, TY = 8;
+  __shared__ float sm[6 * (TX + 4) * (TY + 4) + kNumCoef * (TY + 4)];
+  __shared__ gcdet::Tables stab;
+  const int t = tile_of_block(per_xcd);
+  if (t >= ntiles) return;
+  tile_step<kFused, true, SPH, TX, TY, ST, true>(L, t, tiles_x, sm, &stab);
+}
+
+template <bool SPH, int WAVES>
+hipError_t launch_small(const DevLayer &L, hipStream_t st) {
+  const int tx = (L.nx + 31) / 32, ty = (L.ny + 7) / 8;
+  const int nt = tx * ty, per = (nt + 7) / 8;
+  if (L.stream_out)
+    hipLaunchKernelGGL((k_step_small<SPH, WAVES, true>), dim3(8 * per), dim3(kThreads), 0, st, L, tx, nt, per);
+  else
+    hipLaunchKernelGGL((k_step_small<SPH, WAVES, false>), dim3(8 * per), dim3(kThreads), 0, st, L, tx, nt, per);
+  return hipGetLastError();
+}
+
 template <int MODE, bool NL, bool SPH, int TX, int TY>
 hipError_t launch_t(const DevLayer &L, hipStream_t st) {
   const int tx = (L.nx + TX - 1) / TX, ty = (L.ny + TY - 1) / TY;
@@ -1933,6 +1961,9 @@ const int kVariants[][3] = {{1, 64, 8},  {1, 64, 16}, {1, 32, 32}, {1, 128, 8}, 
 
 }  // namespace
 
+// Nonlinear layers up to this many cells take the 32 x 8 tiles by default.
+constexpr long long kSmallCells = 1200000;
+
 int num_tile_variants() { return (int)(sizeof(kVariants) / sizeof(kVariants[0])); }
 void tile_variant_shape(int v, int *tx, int *ty) {
   *tx = kVariants[v][0] ? kVariants[v][1] : -kVariants[v][1];  // negative: marching strips
@@ -1948,6 +1979,14 @@ hipError_t launch_step(const DevLayer &L, int mode, bool nl, bool sph, int varia
                     : variant == 0             ? march_nl_seg(L.nx, L.ny)
                                                : 0;
     if (seg > 0) return launch_march_nl(L, sph, seg, st);
+  }
+  // Measured, us per step (64x8 tiles; 32x8 with 4 and 8 waves per SIMD):
+  // 96x72 13.9; 9.4, 9.9.  517x391 14.4; 10.9, 11.3.  512x384 + 401x401 nest
+  // 84.9; 67.2, 67.9.  1024x768 21.0; 18.95, 18.3.  1201x901 24.5; 23.2, 22.8.
+  if (mode == kFused && nl && variant == 0 && (long long)L.nx * L.ny <= kSmallCells) {
+    const bool few = (long long)L.nx * L.ny <= kSmallCells / 3;
+    if (sph) return few ? launch_small<true, 4>(L, st) : launch_small<true, 8>(L, st);
+    return few ? launch_small<false, 4>(L, st) : launch_small<false, 8>(L, st);
   }
   if (mode == kMomentMass) {  // outermost linear layers with nested layers: 64x8
     if (nl) return hipErrorInvalidValue;
