@@ -25,6 +25,7 @@
 #include "detmath.h"
 #include "fastdiv.h"
 #include "kernels.h"
+#include "march.h"
 
 namespace gc {
 
@@ -1165,132 +1166,131 @@ __global__ void k_max(DevLayer L, float *zmax_raw) {
 }
 
 // ---------------------------------------------------------------- nesting
-__device__ __forceinline__ float pidx(const DevNest &N, const float *a, int i, int j) {
-  return a[(size_t)(j - 1) * N.pnx + (i - 1)];
-}
-
-// Parent-side forecast of the interface flux at line index k (NEWQ at
-// sub-step 2, all_grids.f90:706-720 and 778-790): one step of the
-// parent's linear momentum, spherical (R2/R3 or R4/R5) or Cartesian
-// (GRX*HM or GRY*HN).  side 0/1: lines I = IS-1 / IE (M); 2/3: J = JS-1 /
-// JE (N).
-__device__ float iface_forecast(const DevNest &N, int side, int k) {
-  const bool vert = side < 2;
-  float x;
-  if (vert) {
-    const int i = side == 0 ? N.is - 1 : N.ie, j = k, ip1 = i + 1, jm1 = j - 1;
-    const float hpc = pidx(N, N.ph, i, j) > kGx
-                          ? 0.5f * (pidx(N, N.ph, i, j) + pidx(N, N.ph, ip1 >= N.pnx ? N.pnx : ip1, j))
-                          : 0.0f;
-    if (N.p_sph) {
-      float tot_n = pidx(N, N.pn1, i, j) + pidx(N, N.pn1, ip1, j) + pidx(N, N.pn1, i, jm1) +
-                    pidx(N, N.pn1, ip1, jm1);
-      const float f2 = N.pcoef[kF2 * N.pny + (j - 1)];
-      float r2 = N.p_r24 ? pidx(N, N.pr24, i, j) : (N.p_nl ? f2 : f2 * fmaxf(hpc, 0.0f));
-      x = pidx(N, N.pm1, i, j) - r2 * (pidx(N, N.pz2, ip1, j) - pidx(N, N.pz2, i, j)) +
-          N.pcoef[kR3 * N.pny + (j - 1)] * tot_n;
-    } else {
-      float hm = hpc + 0.5f * (pidx(N, N.pz2, i, j) + pidx(N, N.pz2, ip1, j));
-      x = pidx(N, N.pm1, i, j) - N.pgrx * hm * (pidx(N, N.pz2, ip1, j) - pidx(N, N.pz2, i, j));
-    }
-  } else {
-    const int i = k, j = side == 2 ? N.js - 1 : N.je, jp1 = j + 1, im1 = i - 1;
-    const float hqc = pidx(N, N.ph, i, j) > kGx
-                          ? 0.5f * (pidx(N, N.ph, i, j) + pidx(N, N.ph, i, jp1 >= N.pny ? N.pny : jp1))
-                          : 0.0f;
-    if (N.p_sph) {
-      float tot_m = pidx(N, N.pm1, im1, j) + pidx(N, N.pm1, im1, jp1) + pidx(N, N.pm1, i, j) +
-                    pidx(N, N.pm1, i, jp1);
-      const float f4 = N.pcoef[kF4 * N.pny + (j - 1)];
-      float r4 = N.p_r24 ? N.pr24[(size_t)N.pnx * N.pny + (size_t)(j - 1) * N.pnx + (i - 1)]
-                         : (N.p_nl ? f4 : f4 * fmaxf(hqc, 0.0f));
-      x = pidx(N, N.pn1, i, j) - r4 * (pidx(N, N.pz2, i, jp1) - pidx(N, N.pz2, i, j)) -
-          N.pcoef[kR5 * N.pny + (j - 1)] * tot_m;
-    } else {
-      float hn = hqc + 0.5f * (pidx(N, N.pz2, i, j) + pidx(N, N.pz2, i, jp1));
-      x = pidx(N, N.pn1, i, j) - N.pgry * hn * (pidx(N, N.pz2, i, jp1) - pidx(N, N.pz2, i, j));
-    }
-  }
-  if (fabsf(x) < kEps) x = 0.0f;
-  return x;
-}
-
-// Both parent cells of the interface face at line index k wet in Z2?
-__device__ __forceinline__ bool iface_wet(const DevNest &N, int side, int k) {
-  const bool vert = side < 2;
-  const int fi = vert ? (side == 0 ? N.is - 1 : N.ie) : k;
-  const int fj = vert ? k : (side == 2 ? N.js - 1 : N.je);
-  const int ai = vert ? fi + 1 : fi, aj = vert ? fj : fj + 1;
-  return (pidx(N, N.ph, fi, fj) + pidx(N, N.pz2, fi, fj) > kGx) &&
-         (pidx(N, N.ph, ai, aj) + pidx(N, N.pz2, ai, aj) > kGx);
-}
-
-// Parent flux on the interface line at index k for sub-step t: JNQ takes
-// the parent's level-1 flux as is (all_grids.f90:484-487); NEWQ blends the
-// cached forecast with it where both parent cells are wet and is 0
-// elsewhere (all_grids.f90:703-727, 774-796).
-__device__ float iface_flux(const DevNest &N, int side, int k, int t) {
-  const bool vert = side < 2;
-  const int fi = vert ? (side == 0 ? N.is - 1 : N.ie) : k;
-  const int fj = vert ? k : (side == 2 ? N.js - 1 : N.je);
-  const float f1 = vert ? pidx(N, N.pm1, fi, fj) : pidx(N, N.pn1, fi, fj);
-  if (t == 1) return f1;
-  if (!iface_wet(N, side, k)) return 0.0f;
-  const float c1 = ((float)t - 1.0f) / (float)N.rel_time;
-  const float c2 = 1.0f - c1;
-  const float cached = t == 2 ? iface_forecast(N, side, k)
-                              : (vert ? N.yflux[(side & 1) * N.pny + (k - 1)]
-                                      : N.xflux[(side & 1) * N.pnx + (k - 1)]);
-  return c1 * cached + c2 * f1;
-}
-
-// JNQ / NEWQ for one child: threads over the four interface lines.  A
-// thread owns parent index k of one side: it writes the forecast cache at
-// k (t == 2, k in the line's full range JS-2..JE+2 / IS-2..IE+2) and, for
-// k in the footprint, the R child boundary fluxes of EDGEINTERP_VERT/HORI
-// (all_grids.f90:502-604), from the interface flux at k-1, k, k+1.
+// JNQ / NEWQ for one child (all_grids.f90:452-801): lanes over the four
+// interface lines, flattened to positions p = 0..jnq_threads-1: side 0/1 the
+// lines I = IS-1 / IE (M) with k = J from JS-2 to JE+2, side 2/3 the lines
+// J = JS-1 / JE (N) with k = I from IS-2 to IE+2.
+//
+// A wave covers 62 positions plus one on either side: each lane computes the
+// interface flux at its own k once and takes k - 1 and k + 1 from its
+// neighbours.  All loads of a lane (parent cells, row coefficients, the R
+// child cells it writes) are issued before any of them is used: the launch is
+// a few waves deep, so it lasts as long as its chain of dependent loads (the
+// form that evaluated three fluxes per thread behind their wet tests took 6.1
+// us per launch on a 512x384 + 401x401 nest, 7 - 8 us over a batch's nests).
 __device__ __forceinline__ int jnq_threads(const DevNest &N) {
   return 2 * (N.je - N.js + 5) + 2 * (N.ie - N.is + 5);
 }
+constexpr int kJnqSpan = 62;
+constexpr int kJnqLoads = 5;  // child cells loaded ahead; larger REL_SIZEs read the rest later
 
-__device__ void jnq_thread(const DevNest &N, int g, int t) {
+__device__ void jnq_wave(const DevNest &N, int w, int t) {
+  const int lane = threadIdx.x & 63;
   const int lv = N.je - N.js + 5, lh = N.ie - N.is + 5;  // k ranges incl. +-2
-  int side;
-  if (g < 2 * lv) { side = g / lv; g -= side * lv; }
-  else { g -= 2 * lv; if (g >= 2 * lh) return; side = 2 + g / lh; g -= (side - 2) * lh; }
+  const int p = w * kJnqSpan + lane - 1;
+  const bool in = p >= 0 && p < jnq_threads(N);
+  int g = in ? p : 0, side;
+  if (g < 2 * lv) {
+    side = g >= lv ? 1 : 0;
+    g -= side * lv;
+  } else {
+    g -= 2 * lv;
+    side = g >= lh ? 3 : 2;
+    g -= (side - 2) * lh;
+  }
   const bool vert = side < 2;
   const int k = (vert ? N.js : N.is) - 2 + g;
-  if (t == 2 && iface_wet(N, side, k)) {
-    const float x = iface_forecast(N, side, k);
-    if (vert) N.yflux[(side & 1) * N.pny + (k - 1)] = x;
-    else N.xflux[(side & 1) * N.pnx + (k - 1)] = x;
-  }
   const int lo = vert ? N.js : N.is, hi = vert ? N.je : N.ie;
-  if (k < lo || k > hi) return;
-  const float fm = iface_flux(N, side, k - 1, t);
-  const float f0 = iface_flux(N, side, k, t);
-  const float fp = iface_flux(N, side, k + 1, t);
-  const float fs = 0.5f * (fm + f0);
-  const float fe = 0.5f * (fp + f0);
-  const int nn = 2 * N.rel_size;
-  const float c1 = (fe - fs) / (float)nn;  // == REAL((fe-fs)/DBLE(nn)), all_grids.f90:538
-  const float c2 = -c1 + fs;
-  const int base = (k - lo) * N.rel_size + 1;
-  for (int kk = 1; kk <= N.rel_size; ++kk) {
-    const int c = base + kk;
-    int ci, cj;
-    if (vert) { ci = side == 0 ? 1 : N.cnx; cj = c; }
-    else { ci = c; cj = side == 2 ? 1 : N.cny; }
-    const size_t cg = (size_t)(cj - 1) * N.cnx + (ci - 1);
-    float v = 2.0f * (float)kk * c1 + c2;
-    if (N.ch[cg] + N.cz1[cg] <= kGx) v = 0.0f;
-    if (vert) N.cm1[cg] = v;
-    else N.cn1[cg] = v;
+  const int fi = vert ? (side == 0 ? N.is - 1 : N.ie) : k;
+  const int fj = vert ? k : (side == 2 ? N.js - 1 : N.je);
+  const int pnx = N.pnx, R = N.rel_size;
+  const size_t f = (size_t)(fj - 1) * pnx + (fi - 1);
+  const size_t a = vert ? f + 1 : f + pnx;  // the other cell of the face
+  // the line of child boundary cells that k feeds
+  const bool own = in && lane >= 1 && lane <= kJnqSpan && k >= lo && k <= hi;
+  const int base = (k - lo) * R + 1;  // cells base + 1 .. base + R (1-based along the line)
+  const size_t c0 = vert ? (size_t)base * N.cnx + (side == 0 ? 0 : N.cnx - 1)
+                         : (size_t)(side == 2 ? 0 : N.cny - 1) * N.cnx + base;
+  const size_t cs = vert ? N.cnx : 1;
+
+  const float *own1 = vert ? N.pm1 : N.pn1, *cross1 = vert ? N.pn1 : N.pm1;
+  const float f1 = own1[f];
+  float hf = 0, ha = 0, zf = 0, za = 0, x0 = 0, x1 = 0, x2 = 0, x3 = 0, rp = 0, rc = 0, cached = 0;
+  if (t > 1) {
+    hf = N.ph[f];
+    ha = N.ph[a];
+    zf = N.pz2[f];
+    za = N.pz2[a];
+    if (t > 2) {
+      cached = vert ? N.yflux[(side & 1) * N.pny + (k - 1)] : N.xflux[(side & 1) * pnx + (k - 1)];
+    } else if (N.p_sph) {
+      // TOT_N at (I, J), (I+1, J), (I, J-1), (I+1, J-1); TOT_M at (I-1, J),
+      // (I-1, J+1), (I, J), (I, J+1)
+      x0 = cross1[vert ? f : f - 1];
+      x1 = cross1[vert ? f + 1 : f - 1 + pnx];
+      x2 = cross1[vert ? f - pnx : f];
+      x3 = cross1[vert ? f + 1 - pnx : f + pnx];
+      rp = N.p_r24 ? N.pr24[vert ? f : (size_t)pnx * N.pny + f]
+                   : N.pcoef[(vert ? kF2 : kF4) * N.pny + (fj - 1)];
+      rc = N.pcoef[(vert ? kR3 : kR5) * N.pny + (fj - 1)];
+    }
   }
+  float hc[kJnqLoads], zc[kJnqLoads];
+#pragma unroll
+  for (int q = 0; q < kJnqLoads; ++q) {
+    const bool use = own && q < R;
+    hc[q] = use ? N.ch[c0 + q * cs] : 0.0f;
+    zc[q] = use ? N.cz1[c0 + q * cs] : 0.0f;
+  }
+
+  // Parent flux on the interface line at k: JNQ takes the parent's level-1
+  // flux as is (:484-487); NEWQ blends it with the forecast where both parent
+  // cells are wet and is 0 elsewhere (:703-727, 774-796).  The forecast, one
+  // step of the parent's linear momentum (:706-720, 778-790), is made at
+  // sub-step 2 and kept for the later ones.
+  float flux = f1;
+  if (t > 1) {
+    const bool wet = (hf + zf > kGx) && (ha + za > kGx);
+    if (t == 2) {
+      const float hm = hf > kGx ? 0.5f * (hf + ha) : 0.0f;
+      float x;
+      if (N.p_sph) {
+        const float tot = x0 + x1 + x2 + x3;
+        const float r = N.p_r24 || N.p_nl ? rp : rp * fmaxf(hm, 0.0f);
+        x = vert ? f1 - r * (za - zf) + rc * tot : f1 - r * (za - zf) - rc * tot;
+      } else {
+        const float h = hm + 0.5f * (zf + za);
+        x = f1 - (vert ? N.pgrx : N.pgry) * h * (za - zf);
+      }
+      if (fabsf(x) < kEps) x = 0.0f;
+      cached = x;
+      if (in && wet && lane >= 1 && lane <= kJnqSpan) {
+        if (vert) N.yflux[(side & 1) * N.pny + (k - 1)] = x;
+        else N.xflux[(side & 1) * pnx + (k - 1)] = x;
+      }
+    }
+    const float w1 = ((float)t - 1.0f) / (float)N.rel_time;
+    const float w2 = 1.0f - w1;
+    flux = wet ? w1 * cached + w2 * f1 : 0.0f;
+  }
+  // EDGEINTERP_VERT/HORI (:502-604)
+  const float fm = west(flux), fp = east(flux);
+  if (!own) return;
+  const float fs = 0.5f * (fm + flux);
+  const float fe = 0.5f * (fp + flux);
+  const float c1 = (fe - fs) / (float)(2 * R);  // == REAL((fe-fs)/DBLE(nn)), :538
+  const float c2 = -c1 + fs;
+  float *cf = vert ? N.cm1 : N.cn1;
+#pragma unroll
+  for (int q = 0; q < kJnqLoads; ++q)
+    if (q < R) cf[c0 + q * cs] = hc[q] + zc[q] <= kGx ? 0.0f : 2.0f * (float)(q + 1) * c1 + c2;
+  for (int q = kJnqLoads; q < R; ++q)
+    cf[c0 + q * cs] =
+        N.ch[c0 + q * cs] + N.cz1[c0 + q * cs] <= kGx ? 0.0f : 2.0f * (float)(q + 1) * c1 + c2;
 }
 
-__global__ void k_jnq(DevNest N, int t) {
-  jnq_thread(N, blockIdx.x * blockDim.x + threadIdx.x, t);
+__global__ void __launch_bounds__(128) k_jnq(DevNest N, int t) {
+  jnq_wave(N, blockIdx.x * 2 + (threadIdx.x >> 6), t);
 }
 
 // JNZ (all_grids.f90:342-421): parent Z2 over the footprint = mean of the
@@ -1362,23 +1362,20 @@ __global__ void k_jnz(DevNest N) { jnz_thread(N, blockIdx.x * blockDim.x + threa
 
 // ------------------------------------------------------------ batch forms
 // Several nests in one launch: nest n owns blocks [start[n], start[n+1]).
+// Each lane compares one start, so finding the nest costs one load.
 __device__ __forceinline__ int nest_of_block(const int *start, int nnest) {
-  int lo = 0, hi = nnest - 1;
-  const int b = blockIdx.x;
-  while (lo < hi) {  // last n with start[n] <= b
-    const int mid = (lo + hi + 1) >> 1;
-    if (start[mid] <= b) lo = mid;
-    else hi = mid - 1;
-  }
-  return lo;
+  const int b = blockIdx.x, lane = threadIdx.x & 63;
+  int n = 0;
+  for (int n0 = 0; n0 < nnest; n0 += 64)  // number of starts <= b
+    n += __popcll(__builtin_amdgcn_ballot_w64(n0 + lane < nnest && start[min(n0 + lane, nnest)] <= b));
+  return n - 1;
 }
 
-__global__ void k_jnq_multi(const DevNest *__restrict__ nests, const int *__restrict__ start,
-                            int nnest, int t) {
+__global__ void __launch_bounds__(128) k_jnq_multi(const DevNest *__restrict__ nests,
+                                                   const int *__restrict__ start, int nnest, int t) {
   const int n = __builtin_amdgcn_readfirstlane(nest_of_block(start, nnest));
   const DevNest N = nests[n];
-  const int g = (blockIdx.x - start[n]) * blockDim.x + threadIdx.x;
-  if (g < jnq_threads(N)) jnq_thread(N, g, t);
+  jnq_wave(N, (blockIdx.x - start[n]) * 2 + (threadIdx.x >> 6), t);
 }
 
 __global__ void k_jnz_multi(const DevNest *__restrict__ nests, const int *__restrict__ start,
@@ -2058,8 +2055,7 @@ hipError_t launch_max(const DevLayer &L, float *zmax_raw, hipStream_t st) {
 }
 
 hipError_t launch_jnq(const DevNest &N, int t, hipStream_t st) {
-  const int total = 2 * (N.je - N.js + 5) + 2 * (N.ie - N.is + 5);
-  hipLaunchKernelGGL(k_jnq, dim3((total + 127) / 128), dim3(128), 0, st, N, t);
+  hipLaunchKernelGGL(k_jnq, dim3(jnq_block_count(N)), dim3(128), 0, st, N, t);
   return hipGetLastError();
 }
 
@@ -2163,7 +2159,8 @@ hipError_t launch_batch(const BatchLaunch &B, int mode, bool nl, bool sph, int s
 }
 
 int jnq_block_count(const DevNest &N) {
-  return (2 * (N.je - N.js + 5) + 2 * (N.ie - N.is + 5) + 127) / 128;
+  const int total = 2 * (N.je - N.js + 5) + 2 * (N.ie - N.is + 5);
+  return (total + 2 * kJnqSpan - 1) / (2 * kJnqSpan);
 }
 int jnz_block_count(const DevNest &N) {
   return ((N.ie - N.is + 1) * (N.je - N.js + 1) + 127) / 128;
