@@ -80,6 +80,7 @@ struct Group {
   std::vector<int> start;  // nnest + 1
   size_t o_descs = 0, o_items = 0, o_qstart = 0, o_nests = 0, o_start = 0;
   int head = 0;            // index of this launch's 8 heads
+  bool dry = false;        // layers without their maximum planes (the tuner's)
   long long cells = 0;     // cell updates of a step group
   std::vector<std::pair<const Tree *, const LayerRec *>> recs;  // layer of each desc
   // stream lane: 0 and 2 = the two chains of nested scenarios, 1 = the
@@ -180,16 +181,25 @@ std::vector<Scenario *> active() {
   return a;
 }
 
-// Tuning classes: layer kind and whether the launch alone fills the chip
+// Tuning classes: layer kind and how far the launch alone fills the chip
 // (below ~4M cells a launch leaves CUs idle and favours smaller tiles).
 long long kind_key(int nl, int sph, long long cells) {
-  return ((long long)nl * 2 + sph) * 2 + (cells >= (4LL << 20) ? 1 : 0);
+  const int size = cells >= (4LL << 20) ? 3 : (cells >= (5LL << 18) ? 2 : (cells >= (1LL << 19) ? 1 : 0));
+  return ((long long)nl * 2 + sph) * 4 + size;
 }
 
-int shape_for(int nl, int sph, long long cells) {
+// Shape of a fused launch over `layers`: the caller's, the tuned one of its
+// class, else the one that suits layers of that size (see batch_rule_shape);
+// shapes that one of the layers cannot take fall back to 64 x 8 tiles.
+int shape_for(int nl, int sph, long long cells, const std::vector<DevLayer> &layers) {
   if (g_eng.forced_shape >= 0) return g_eng.forced_shape;
   auto it = g_eng.tuned.find(kind_key(nl, sph, cells));
-  return it == g_eng.tuned.end() ? batch_num_shapes() / 2 : it->second;
+  const int sh = it != g_eng.tuned.end() ? it->second
+                                         : batch_rule_shape(layers.data(), (int)layers.size(), nl != 0,
+                                                            batch_num_shapes());
+  for (const DevLayer &d : layers)
+    if (!batch_shape_takes(sh, d, nl != 0, sph != 0)) return kBatchGridShape;
+  return sh;
 }
 
 // Step group for layers of one kind and mode; tiles of tx x ty.
@@ -231,9 +241,11 @@ void flush_steps(std::vector<Pending> &pend, std::vector<Group> &out) {
     int tx = 64, ty = 8;
     if (p.mode == kTwoStep) {
       g.shape = g_eng.step2_shape;
+      for (auto &d : p.layers)
+        if (!step2_shape_takes(g.shape, d, p.sph != 0)) g.shape = kStep2TileShape;
       step2_shape(g.shape, &tx, &ty);
     } else {
-      g.shape = p.mode == kFused ? shape_for(p.nl, p.sph, cells) : batch_num_shapes() / 2;
+      g.shape = p.mode == kFused ? shape_for(p.nl, p.sph, cells, p.layers) : kBatchGridShape;
       batch_shape(g.shape, &tx, &ty);
     }
     for (auto &d : p.layers) add_layer_items(g, d, tx, ty);
@@ -459,6 +471,7 @@ BatchLaunch step_launch(const Plan &P, const Group &g) {
   B.qstart = reinterpret_cast<const int *>(P.arena + g.o_qstart);
   B.heads = P.heads + g.head;
   B.nitems = (int)g.items.size();
+  B.dry = g.dry ? 1 : 0;
   return B;
 }
 
@@ -541,7 +554,7 @@ int tune(const std::vector<Scenario *> &act) {
       ctl.push_back(s->tree.ctl_in);
       ahead.push_back(s->tree.mass_ahead);
     }
-    emit_step(act, probe);
+    emit_lanes(act, probe, -1);  // the launches as the plan splits them
     for (size_t i = 0; i < act.size(); ++i) {
       for (int k = 0; k < kMaxLayers; ++k) act[i]->tree.layers[k].cur = cur[i][k];
       act[i]->tree.ctl_in = ctl[i];
@@ -561,6 +574,11 @@ int tune(const std::vector<Scenario *> &act) {
     int best = 0;
     float best_ms = 1e30f;
     for (int sh = 0; sh < batch_num_shapes(); ++sh) {
+      bool takes = true;
+      for (auto &tr : g.recs)
+        takes = takes && batch_shape_takes(sh, dev_view(*tr.first, *tr.second, false, false), g.nl != 0,
+                                           g.sph != 0);
+      if (!takes) continue;
       int tx, ty;
       batch_shape(sh, &tx, &ty);
       Plan T;
@@ -571,6 +589,7 @@ int tune(const std::vector<Scenario *> &act) {
       d.nl = g.nl;
       d.sph = g.sph;
       d.shape = sh;
+      d.dry = true;
       // views at the layers' current time levels (the probe's later
       // sub-steps saw rotated ones): read level 1, write level 2 only
       for (auto &tr : g.recs) add_layer_items(d, dev_view(*tr.first, *tr.second, false, false), tx, ty);
@@ -620,6 +639,11 @@ int tune(const std::vector<Scenario *> &act) {
       int best = -1;
       float best_ms = 2 * one;  // two one-step launches
       for (int sh = 0; sh < kStep2Shapes && one > 0; ++sh) {
+        bool takes = true;
+        for (auto &tr : roots)
+          takes = takes && step2_shape_takes(sh, dev_view(*tr.first, *tr.second, false, false),
+                                             tr.second->sph != 0);
+        if (!takes) continue;
         int tx, ty;
         step2_shape(sh, &tx, &ty);
         Plan T;
@@ -631,6 +655,7 @@ int tune(const std::vector<Scenario *> &act) {
           d.nl = 0;
           d.sph = 1 - part;
           d.shape = sh;
+          d.dry = true;
           for (auto &tr : roots)
             if (tr.second->sph == d.sph)
               add_layer_items(d, dev_view(*tr.first, *tr.second, false, false), tx, ty);
@@ -1017,7 +1042,7 @@ long long gcomcot_layer_footprint_(int *nx, int *ny, int *nonlinear) {
 void gcomcot_batch_set_arrival_threshold_(float *thr) { g_eng.arr_thr = *thr; }
 
 int gcomcot_batch_set_tuning_(int *autotune, int *shape) {
-  if (*shape >= batch_num_shapes()) return fail(34, "batch: tile shape %d out of range", *shape);
+  if (*shape >= kBatchForcedShapes) return fail(34, "batch: tile shape %d out of range", *shape);
   g_eng.autotune = *autotune != 0;
   g_eng.forced_shape = *shape;
   invalidate();

@@ -4,8 +4,6 @@
 #include <hip/hip_runtime.h>
 #include <stddef.h>
 
-#include <algorithm>
-
 namespace gc {
 
 // What one step kernel needs of a layer.  Planes are column-major NX*NY
@@ -47,6 +45,9 @@ struct DevLayer {
   // end the write-back of the whole new level.  The batch kernels always
   // store through the caches.
   int stream_out;
+  // bytes of the layer's block, which starts with h and holds every plane
+  // above; 0 when they do not fit in one buffer descriptor (4 GB)
+  unsigned block_bytes;
 };
 
 // kMomentMass: the momentum half of root step k of a linear outermost
@@ -74,20 +75,6 @@ constexpr int kStep2Shapes = 7;
 // tile of two-step shape `shape`
 void step2_shape(int shape, int *tx, int *ty);
 
-// Bytes from a layer's depth plane to the end of its last plane; the
-// descriptor of the marching kernels spans them.  ~0 if a plane lies before.
-inline unsigned long long block_span(const DevLayer &L) {
-  const char *lo = reinterpret_cast<const char *>(L.h), *hi = lo;
-  for (const void *p : {(const void *)L.z1, (const void *)L.m1, (const void *)L.n1,
-                        (const void *)L.z2, (const void *)L.m2, (const void *)L.n2,
-                        (const void *)L.zmax, (const void *)L.arrival})
-    if (p) {
-      if (reinterpret_cast<const char *>(p) < lo) return ~0ull;
-      hi = std::max(hi, reinterpret_cast<const char *>(p));
-    }
-  return (unsigned long long)(hi - lo) + 4ull * L.nx * L.ny;
-}
-
 // Root steps of a spherical linear outermost layer without children in the
 // marching kernels (march.hip): 2 or 4 per launch, level 1 in, level 2 out,
 // bookkeeping as launch_step2.  march_plan gives the steps per launch that
@@ -99,7 +86,7 @@ struct MarchPlan {
 };
 MarchPlan march_plan(int nx, int ny);
 inline bool march_applies(const DevLayer &L) {
-  return L.is_root && L.rowc && !L.r24 && !L.zraw && !L.sponge_cx && block_span(L) < 0xffffffffull;
+  return L.is_root && L.rowc && !L.r24 && !L.zraw && !L.sponge_cx && L.block_bytes != 0;
 }
 hipError_t launch_march_linear(const DevLayer &L, int steps, hipStream_t st);
 
@@ -108,7 +95,7 @@ hipError_t launch_march_linear(const DevLayer &L, int steps, hipStream_t st);
 // gives the segments that suit a layer, 0 where the LDS tiles are faster.
 inline bool march_nl_applies(const DevLayer &L, bool sph) {
   return (!sph || L.rowc) && L.modscm == 1 && L.linchk == 1 && L.fric && !L.r24 && !L.zraw &&
-         !L.sponge_cx && block_span(L) < 0xffffffffull;
+         !L.sponge_cx && L.block_bytes != 0;
 }
 int march_nl_seg(int nx, int ny);
 hipError_t launch_march_nl(const DevLayer &L, bool sph, int seg, hipStream_t st);
@@ -212,17 +199,43 @@ struct BatchLaunch {
   const int *qstart;  // 9 entries: items of XCD queue q are [qstart[q], qstart[q+1])
   int *heads;         // 8 queue heads, zero before the launch
   int nitems;
+  int dry;            // 1: the layers' views carry no maximum planes
 };
-// Fused launches take tile shape `shape` (batch_shape); continuity and
+// Fused launches take tile shape `shape` (batch_shape): 0-2 the persistent
+// form and 3-5 the grid form of 64 x 8, 32 x 16 and 64 x 16 tiles, and for
+// nonlinear layers 6 = grid form of 32 x 8 tiles (one cell per thread), 7 and
+// 8 = marching strips, four waves of 8 or 14 rows to an item.  Continuity and
 // momentum halves of nested parents use 64 x 8.  prepare: only look up
 // the kernel's resident-workgroup count (do it before a graph capture).
 int batch_num_shapes();
 void batch_shape(int k, int *tx, int *ty);
+constexpr int kBatchGridShape = 3, kBatchForcedShapes = 6, kBatchSmallShape = 6, kBatchMarchShape = 7;
+inline bool batch_shape_takes(int shape, const DevLayer &L, bool nl, bool sph) {
+  return shape < kBatchSmallShape || (nl && (shape < kBatchMarchShape || march_nl_applies(L, sph)));
+}
+// The shape of a fused launch that nobody tuned: marching strips where the
+// layers together give their SIMDs enough rows (the lines of march_nl_seg),
+// one cell per thread below, 64 x 8 tiles for linear layers.
+inline int batch_rule_shape(const DevLayer *layers, int n, bool nl, int num_shapes) {
+  if (!nl || num_shapes <= kBatchMarchShape) return kBatchGridShape;
+  long long rows = 0;
+  for (int k = 0; k < n; ++k) rows += (long long)((layers[k].nx + 59) / 60) * layers[k].ny / 1024;
+  return rows < 16 ? kBatchSmallShape : (rows < 36 ? kBatchMarchShape : kBatchMarchShape + 1);
+}
 hipError_t launch_batch(const BatchLaunch &B, int mode, bool nl, bool sph, int shape,
                         hipStream_t st, bool prepare = false);
 // Two root steps of single-layer linear layers, one workgroup per item;
 // items tile each layer with step2_shape(shape) tiles.
 hipError_t launch_batch2(const BatchLaunch &B, bool sph, int shape, hipStream_t st);
+// Two-step shape 6 of the batch is the marching form for spherical layers
+// (and a tile of the same size for Cartesian ones); kStep2TileShape suits any.
+constexpr int kStep2March = 6, kStep2TileShape = 4;
+inline bool step2_shape_takes(int shape, const DevLayer &L, bool sph) {
+  return shape != kStep2March || !sph || march_applies(L);
+}
+// The marching forms of launch_batch and launch_batch2.
+hipError_t launch_batch_march_nl(const BatchLaunch &B, bool sph, int seg, hipStream_t st);
+hipError_t launch_batch_march2(const BatchLaunch &B, hipStream_t st);
 // JNQ/NEWQ and JNZ of several nests in one launch: nest n owns blocks
 // [start[n], start[n+1]) of 128 threads; *_block_count gives each one's share.
 int jnq_block_count(const DevNest &N);

@@ -2020,6 +2020,11 @@ hipError_t launch_step2(const DevLayer &L, bool sph, int shape, hipStream_t st) 
 }
 
 void step2_shape(int shape, int *tx, int *ty) {
+  if (shape == kStep2March) {  // in the batch: marching strips of 60, four waves of 8 rows
+    *tx = 60;
+    *ty = 32;
+    return;
+  }
 #define GC_S2(K, TX, TY, NT) \
   case K: *tx = TX; *ty = TY; return;
   switch (shape) {
@@ -2039,6 +2044,8 @@ hipError_t launch_batch2_t(const BatchLaunch &B, hipStream_t st) {
 
 hipError_t launch_batch2(const BatchLaunch &B, bool sph, int shape, hipStream_t st) {
   if (B.nitems <= 0) return hipSuccess;
+  if (shape == kStep2March)
+    return sph ? launch_batch_march2(B, st) : launch_batch2_t<false, 60, 32, 512>(B, st);
 #define GC_S2(K, TX, TY, NT) \
   case K: return sph ? launch_batch2_t<true, TX, TY, NT>(B, st) : launch_batch2_t<false, TX, TY, NT>(B, st);
   switch (shape) {
@@ -2081,6 +2088,14 @@ int device_cus() {
 }
 
 template <int MODE, bool NL, bool SPH, int TX, int TY>
+hipError_t launch_batch_grid_t(const BatchLaunch &B, hipStream_t st) {
+  const int per = (B.nitems + 7) / 8;
+  hipLaunchKernelGGL((k_batch_grid<MODE, NL, SPH, TX, TY>), dim3(8 * per), dim3(kThreads), 0, st,
+                     B.descs, B.items, B.nitems, per);
+  return hipGetLastError();
+}
+
+template <int MODE, bool NL, bool SPH, int TX, int TY>
 hipError_t launch_batch_t(const BatchLaunch &B, hipStream_t st, bool prepare, bool grid_form) {
   static int resident = 0;  // workgroups that fit on the chip at once
   if (!resident) {
@@ -2091,12 +2106,7 @@ hipError_t launch_batch_t(const BatchLaunch &B, hipStream_t st, bool prepare, bo
     resident = (per_cu > 0 ? per_cu : 1) * device_cus();
   }
   if (prepare) return hipSuccess;
-  if (grid_form) {
-    const int per = (B.nitems + 7) / 8;
-    hipLaunchKernelGGL((k_batch_grid<MODE, NL, SPH, TX, TY>), dim3(8 * per), dim3(kThreads), 0,
-                       st, B.descs, B.items, B.nitems, per);
-    return hipGetLastError();
-  }
+  if (grid_form) return launch_batch_grid_t<MODE, NL, SPH, TX, TY>(B, st);
   // at least four items per workgroup: fewer, and the claims cost more
   // than they balance
   int grid = resident;
@@ -2127,8 +2137,13 @@ constexpr int kNumBatchTiles = 3;
 
 }  // namespace
 
-int batch_num_shapes() { return 2 * kNumBatchTiles; }
+int batch_num_shapes() { return kBatchMarchShape + 2; }
 void batch_shape(int k, int *tx, int *ty) {
+  if (k >= kBatchSmallShape) {
+    *tx = k == kBatchSmallShape ? 32 : 60;
+    *ty = k == kBatchSmallShape ? 8 : (k == kBatchMarchShape ? 4 * 8 : 4 * 14);
+    return;
+  }
   *tx = kBatchShapes[k % kNumBatchTiles][0];
   *ty = kBatchShapes[k % kNumBatchTiles][1];
 }
@@ -2149,6 +2164,14 @@ hipError_t launch_batch(const BatchLaunch &B, int mode, bool nl, bool sph, int s
     GC_CASE(kMomentMass, false, true) GC_CASE(kMomentMass, false, false)
 #undef GC_CASE
     return hipErrorInvalidValue;
+  }
+  if (shape >= kBatchSmallShape) {
+    if (!nl) return hipErrorInvalidValue;
+    if (prepare) return hipSuccess;
+    if (shape >= kBatchMarchShape)
+      return launch_batch_march_nl(B, sph, shape == kBatchMarchShape ? 8 : 14, st);
+    return sph ? launch_batch_grid_t<kFused, true, true, 32, 8>(B, st)
+               : launch_batch_grid_t<kFused, true, false, 32, 8>(B, st);
   }
   switch (shape % kNumBatchTiles) {
     case 0: return batch_shape_t<64, 8>(B, mode, nl, sph, st, prepare, grid_form);

@@ -37,8 +37,8 @@ __device__ __forceinline__ float east(float v) {
 // stores.)
 typedef __amdgpu_buffer_rsrc_t Block;
 constexpr int kNoStore = -1;
-__device__ __forceinline__ Block block_of(const DevLayer &L, unsigned bytes) {
-  return __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(L.h), 0, bytes, 0x00027000);
+__device__ __forceinline__ Block block_of(const DevLayer &L) {
+  return __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(L.h), 0, (int)L.block_bytes, 0x00027000);
 }
 __device__ __forceinline__ unsigned plane_off(const DevLayer &L, const void *p) {
   return (unsigned)(reinterpret_cast<unsigned long long>(p) -

@@ -38,8 +38,7 @@ namespace {
 // loaded D rows ahead of its use.  MX: the wet maximum and first
 // arrival are kept.
 template <int K, bool COL, bool ROW, bool MX, bool ST>
-__device__ __forceinline__ void march_linear(const DevLayer &L, const Strip S, int step,
-                                             unsigned block_bytes) {
+__device__ __forceinline__ void march_linear(const DevLayer &L, const Strip S, int step) {
   // Rows in flight.  The row loop is unrolled by D, so a row's registers stay
   // put until its turn: rotating them would wait for loads just issued.
   constexpr int D = COL || ROW ? 2 : 4;
@@ -51,7 +50,7 @@ __device__ __forceinline__ void march_linear(const DevLayer &L, const Strip S, i
   const bool west_end = COL && i == 1, east_end = COL && i == nx;
   const int vst = own ? vld : kNoStore;
   const int ra = S.j0 - K, rb = S.j1 + K;
-  const Block B = block_of(L, block_bytes);
+  const Block B = block_of(L);
   const unsigned pitch = (unsigned)nx * 4u;
   const unsigned oz1 = plane_off(L, L.z1), om1 = plane_off(L, L.m1), on1 = plane_off(L, L.n1),
                  oz2 = plane_off(L, L.z2), om2 = plane_off(L, L.m2), on2 = plane_off(L, L.n2),
@@ -237,7 +236,7 @@ struct MarchGrid {
 // each XCD takes one contiguous run of waves, so strips that share halo
 // columns meet in one L2).
 template <int K, bool MX, bool ST>
-__global__ void __launch_bounds__(kMarchBlock) k_march_linear(DevLayer L, MarchGrid G, unsigned block_bytes) {
+__global__ void __launch_bounds__(kMarchBlock) k_march_linear(DevLayer L, MarchGrid G) {
   constexpr int W = kWave - 2 * K, WB = kMarchBlock / kWave;
   const int wb = threadIdx.x >> 6;
   int step = 0;
@@ -254,7 +253,7 @@ __global__ void __launch_bounds__(kMarchBlock) k_march_linear(DevLayer L, MarchG
     S.c0 = (k == 0 ? 0 : G.east + k - 1) * W + 1;
     S.j0 = (w / nside) * G.seg_side + 1;
     S.j1 = min(S.j0 + G.seg_side - 1, L.ny);
-    march_linear<K, true, true, MX, ST>(L, S, step, block_bytes);
+    march_linear<K, true, true, MX, ST>(L, S, step);
     return;
   }
   const int b = blockIdx.x - G.side_blocks, mid = G.east - 1;
@@ -263,8 +262,8 @@ __global__ void __launch_bounds__(kMarchBlock) k_march_linear(DevLayer L, MarchG
   S.c0 = (1 + w % mid) * W + 1;
   S.j0 = (w / mid) * G.seg + 1;
   S.j1 = min(S.j0 + G.seg - 1, L.ny);
-  if (S.j0 - K < 2 || S.j1 + K > L.ny - 1) march_linear<K, false, true, MX, ST>(L, S, step, block_bytes);
-  else march_linear<K, false, false, MX, ST>(L, S, step, block_bytes);
+  if (S.j0 - K < 2 || S.j1 + K > L.ny - 1) march_linear<K, false, true, MX, ST>(L, S, step);
+  else march_linear<K, false, false, MX, ST>(L, S, step);
 }
 
 template <int K, bool MX, bool ST>
@@ -286,7 +285,7 @@ hipError_t launch_k(const DevLayer &L, int seg, int seg_side, hipStream_t st) {
   const long long blocks = (long long)G.side_blocks + 8LL * G.per_xcd;
   if (blocks > 0x7fffffff) return hipErrorInvalidValue;
   hipLaunchKernelGGL((k_march_linear<K, MX, ST>), dim3((unsigned)blocks), dim3(kMarchBlock), 0, st,
-                     L, G, (unsigned)block_span(L));
+                     L, G);
   return hipGetLastError();
 }
 
@@ -297,6 +296,36 @@ hipError_t launch_k(const DevLayer &L, const MarchPlan &p, hipStream_t st) {
                         : launch_k<K, true, false>(L, p.seg, p.seg_side, st);
   return L.stream_out ? launch_k<K, false, true>(L, p.seg, p.seg_side, st)
                       : launch_k<K, false, false>(L, p.seg, p.seg_side, st);
+}
+
+// The batch form of two root steps: one workgroup per (layer, tile) item of a
+// 60 x 32 tiling, a wave per 8 rows.
+template <bool MX>
+__global__ void __launch_bounds__(kMarchBlock)
+    k_batch_march2(const BatchDesc *__restrict__ descs, const BatchItem *__restrict__ items, int nitems,
+                   int per_xcd) {
+  constexpr int K = 2, W = kWave - 2 * K, SEG = 8;
+  const int it = (blockIdx.x & 7) * per_xcd + (blockIdx.x >> 3);
+  if (it >= nitems) return;
+  const BatchItem w = items[it];
+  const int slot = __builtin_amdgcn_readfirstlane(w.slot), t = __builtin_amdgcn_readfirstlane(w.tile);
+  const DevLayer L = descs[slot].L;
+  const int tiles_x = descs[slot].tiles_x;
+  int step = 0;
+  if (MX) {
+    step = L.ctl[L.ctl_in] + 1;
+    if (L.advance && t == 0 && threadIdx.x == 0) L.ctl[1 - L.ctl_in] = step + K - 1;
+  }
+  Strip S;
+  S.c0 = (t % tiles_x) * W + 1;
+  S.j0 = (t / tiles_x) * 4 * SEG + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) * SEG + 1;
+  S.j1 = min(S.j0 + SEG - 1, L.ny);
+  if (S.j0 > S.j1) return;
+  const bool rows = S.j0 - K >= 2 && S.j1 + K <= L.ny - 1;
+  const bool cols = S.c0 - K >= 2 && S.c0 - K + kWave - 1 <= L.nx - 1;
+  if (cols && rows) march_linear<K, false, false, MX, false>(L, S, step);
+  else if (cols) march_linear<K, false, true, MX, false>(L, S, step);
+  else march_linear<K, true, true, MX, false>(L, S, step);
 }
 
 }  // namespace
@@ -330,6 +359,18 @@ hipError_t launch_march_linear(const DevLayer &L, int steps, hipStream_t st) {
     case 4: return launch_k<4>(L, p, st);
     default: return hipErrorInvalidValue;
   }
+}
+
+hipError_t launch_batch_march2(const BatchLaunch &B, hipStream_t st) {
+  if (B.nitems <= 0) return hipSuccess;
+  const int per = (B.nitems + 7) / 8;
+  if (B.dry)
+    hipLaunchKernelGGL(k_batch_march2<false>, dim3(8 * per), dim3(kMarchBlock), 0, st, B.descs, B.items,
+                       B.nitems, per);
+  else
+    hipLaunchKernelGGL(k_batch_march2<true>, dim3(8 * per), dim3(kMarchBlock), 0, st, B.descs, B.items,
+                       B.nitems, per);
+  return hipGetLastError();
 }
 
 }  // namespace gc

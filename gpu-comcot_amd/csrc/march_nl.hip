@@ -102,7 +102,7 @@ __device__ __forceinline__ float limited(float x, float DD, Mask act) {
 // column and the ranges of the Fortran loops apply); ROW: the same for rows;
 // otherwise all of that compiles away.
 template <bool SPH, bool COL, bool ROW, bool MX, bool ST>
-__device__ __forceinline__ void march_nl(const DevLayer &L, const Strip S, int step, unsigned block_bytes,
+__device__ __forceinline__ void march_nl(const DevLayer &L, const Strip S, int step,
                                          const gcdet::Tables &tab) {
   // halo columns and rows; rows in flight, and unrolled (the rings of three
   // rows then rotate without moves)
@@ -121,7 +121,7 @@ __device__ __forceinline__ void march_nl(const DevLayer &L, const Strip S, int s
   const Mask conv_col = COL ? GC_BALLOT(i > kSpan && i < nx - kSpan) : ~0ull;
   const Mask ghost = COL ? GC_BALLOT(i < 2) : 0;
   const int ra = S.j0 - HW, rb = S.j1 + HW;
-  const Block B = block_of(L, block_bytes);
+  const Block B = block_of(L);
   const unsigned pitch = (unsigned)nx * 4u;
   const unsigned oz1 = plane_off(L, L.z1), om1 = plane_off(L, L.m1), on1 = plane_off(L, L.n1),
                  oz2 = plane_off(L, L.z2), om2 = plane_off(L, L.m2), on2 = plane_off(L, L.n2),
@@ -394,7 +394,7 @@ __device__ __forceinline__ bool nl_first(const NlGrid &G, int ny, int w, Strip &
 }
 
 template <bool SPH, bool MX, bool ST>
-__global__ void __launch_bounds__(kMarchBlock) k_march_nl(DevLayer L, NlGrid G, unsigned block_bytes) {
+__global__ void __launch_bounds__(kMarchBlock) k_march_nl(DevLayer L, NlGrid G) {
   constexpr int WB = kMarchBlock / kWave;
   __shared__ gcdet::Tables tab;
   stage(tab);
@@ -408,9 +408,9 @@ __global__ void __launch_bounds__(kMarchBlock) k_march_nl(DevLayer L, NlGrid G, 
     const int w = __builtin_amdgcn_readfirstlane(blockIdx.x * WB + (threadIdx.x >> 6));
     if (!nl_first(G, L.ny, w, S)) return;
     if (S.j0 > kNlEnd && S.j1 <= L.ny - kNlEnd)
-      march_nl<SPH, true, false, MX, ST>(L, S, step, block_bytes, tab);
+      march_nl<SPH, true, false, MX, ST>(L, S, step, tab);
     else
-      march_nl<SPH, true, true, MX, ST>(L, S, step, block_bytes, tab);
+      march_nl<SPH, true, true, MX, ST>(L, S, step, tab);
     return;
   }
   const int b = blockIdx.x - G.first_blocks, mid = G.east - 1;
@@ -419,7 +419,7 @@ __global__ void __launch_bounds__(kMarchBlock) k_march_nl(DevLayer L, NlGrid G, 
   S.c0 = (1 + w % mid) * kNlWidth + 1;
   S.j0 = G.end_rows + (w / mid) * G.seg + 1;
   S.j1 = min(S.j0 + G.seg - 1, L.ny - G.end_rows);
-  march_nl<SPH, false, false, MX, ST>(L, S, step, block_bytes, tab);
+  march_nl<SPH, false, false, MX, ST>(L, S, step, tab);
 }
 
 template <bool SPH, bool MX, bool ST>
@@ -442,9 +442,39 @@ hipError_t launch_nl(const DevLayer &L, int seg, hipStream_t st) {
   G.per_xcd = (int)((mid + 8 * WB - 1) / (8 * WB));
   const long long blocks = (long long)G.first_blocks + 8LL * G.per_xcd;
   if (blocks > 0x7fffffff) return hipErrorInvalidValue;
-  hipLaunchKernelGGL((k_march_nl<SPH, MX, ST>), dim3((unsigned)blocks), dim3(kMarchBlock), 0, st, L, G,
-                     (unsigned)block_span(L));
+  hipLaunchKernelGGL((k_march_nl<SPH, MX, ST>), dim3((unsigned)blocks), dim3(kMarchBlock), 0, st, L, G);
   return hipGetLastError();
+}
+
+// The batch form: one workgroup per (layer, tile) item of a 60 x 4 SEG tiling,
+// a wave per SEG rows.
+template <bool SPH, bool MX, int SEG>
+__global__ void __launch_bounds__(kMarchBlock)
+    k_batch_march_nl(const BatchDesc *__restrict__ descs, const BatchItem *__restrict__ items, int nitems,
+                     int per_xcd) {
+  __shared__ gcdet::Tables tab;
+  const int it = (blockIdx.x & 7) * per_xcd + (blockIdx.x >> 3);
+  if (it >= nitems) return;
+  const BatchItem w = items[it];
+  const int slot = __builtin_amdgcn_readfirstlane(w.slot), t = __builtin_amdgcn_readfirstlane(w.tile);
+  const DevLayer L = descs[slot].L;
+  const int tiles_x = descs[slot].tiles_x;
+  stage(tab);
+  int step = 0;
+  if (MX) {
+    step = L.ctl[L.ctl_in] + 1;
+    if (L.advance && t == 0 && threadIdx.x == 0) L.ctl[1 - L.ctl_in] = step;
+  }
+  const int k = t % tiles_x, east = min(max((L.nx - kSpan - 3) / kNlWidth, 1), tiles_x);
+  Strip S;
+  S.c0 = k * kNlWidth + 1;
+  S.j0 = (t / tiles_x) * 4 * SEG + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) * SEG + 1;
+  S.j1 = min(S.j0 + SEG - 1, L.ny);
+  if (S.j0 > S.j1) return;
+  const bool rows = S.j0 > kNlEnd && S.j1 <= L.ny - kNlEnd, cols = k > 0 && k < east;
+  if (rows && cols) march_nl<SPH, false, false, MX, false>(L, S, step, tab);
+  else if (rows) march_nl<SPH, true, false, MX, false>(L, S, step, tab);
+  else march_nl<SPH, true, true, MX, false>(L, S, step, tab);
 }
 
 }  // namespace
@@ -471,6 +501,21 @@ hipError_t launch_march_nl(const DevLayer &L, bool sph, int seg, hipStream_t st)
     return L.stream_out ? launch_nl<A, C, true>(L, seg, st) : launch_nl<A, C, false>(L, seg, st);
   GC_NL(true, true) GC_NL(true, false) GC_NL(false, true) GC_NL(false, false)
 #undef GC_NL
+  return hipErrorInvalidValue;
+}
+
+hipError_t launch_batch_march_nl(const BatchLaunch &B, bool sph, int seg, hipStream_t st) {
+  if (B.nitems <= 0) return hipSuccess;
+  const int per = (B.nitems + 7) / 8;
+#define GC_BM(A, C, SEG)                                                                              \
+  if (sph == A && (B.dry == 0) == C && seg == SEG) {                                                  \
+    hipLaunchKernelGGL((k_batch_march_nl<A, C, SEG>), dim3(8 * per), dim3(kMarchBlock), 0, st, B.descs, \
+                       B.items, B.nitems, per);                                                       \
+    return hipGetLastError();                                                                         \
+  }
+  GC_BM(true, true, 8) GC_BM(true, false, 8) GC_BM(false, true, 8) GC_BM(false, false, 8)
+  GC_BM(true, true, 14) GC_BM(true, false, 14) GC_BM(false, true, 14) GC_BM(false, false, 14)
+#undef GC_BM
   return hipErrorInvalidValue;
 }
 

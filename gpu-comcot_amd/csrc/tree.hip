@@ -326,6 +326,7 @@ DevLayer dev_view(const Tree &T, const LayerRec &L, bool with_max, bool advance)
   d.sponge_cx = (L.sponge && L.id == 1) ? L.sponge : nullptr;
   d.sponge_cy = d.sponge_cx ? L.sponge + L.nx : nullptr;
   d.stream_out = streams_planes(L) ? 1 : 0;
+  d.block_bytes = L.block_bytes < 0xffffffffull ? (unsigned)L.block_bytes : 0;
   return d;
 }
 

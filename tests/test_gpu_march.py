@@ -7,7 +7,7 @@ import pytest
 
 from gcomcot import DeviceRun
 from gcomcot import scenarios as S
-from helpers import compare_device_oracle
+from helpers import compare_device_oracle, diff_report
 from oracle.bind import Oracle
 
 pytestmark = pytest.mark.gpu
@@ -104,3 +104,29 @@ def test_marched_child_matches_oracle(clc):
             dev.close()
     finally:
         lib().gcomcot_set_tile_variant_(ip(0))
+
+
+@pytest.mark.parametrize("count,nx,ny", [(2, 150, 131), (3, 905, 641), (5, 845, 717)],
+                         ids=["one-cell-tiles", "strips-of-8", "strips-of-14"])
+def test_batched_nonlinear_layers_by_size(count, nx, ny):
+    """The shapes that an untuned batch gives nonlinear layers, by the rows
+    they have together; one layer is Cartesian, and a linear one beside them
+    takes its two steps in marching strips."""
+    from gcomcot.batch import Batch
+    from helpers import BEACH
+    scs = [S.custom(laycord=k % 2, laygov=1, nx=nx - 7 * k, ny=ny - 5 * k, **BEACH) for k in range(count)]
+    scs.append(S.custom(laycord=0, laygov=0, nx=331, ny=150))
+    print(f"[gpu] batch of {count} nonlinear layers near {nx}x{ny}", flush=True)
+    b = Batch(autotune=False, two_step_shape=6)
+    sids = [b.add(sc, 15) for sc in scs]
+    b.run(15)
+    for sc, sid in zip(scs, sids):
+        orc = Oracle(sc, 32, pow_mode=1)
+        orc.step(15)
+        st, mx, o, om = b.state(sid), b.maxima(sid), orc.state(1), orc.maxima(1)
+        for k in ("z1", "m1", "n1"):
+            nb, worst = diff_report(st[k], o[k])
+            assert nb == 0, f"{sc.name} {k}: {nb} cells differ (max {worst})"
+        assert diff_report(mx["zmax_wet"], om["zmax_wet"])[0] == 0, sc.name
+        assert (mx["arrival"] == om["arrival"]).all(), sc.name
+    b.close()
