@@ -441,125 +441,42 @@ static bool marches() {
 // n root steps in the marching kernels.  The run ends with a two-step launch
 // (n even) or a single step (n odd), so level 2 then holds the state two
 // steps (one step) before level 1.
-static int run_marched(int n, int use_graph) {
+static int run_marched(int n) {
   LayerRec *R = layer(1);
   const int K = march_plan(R->nx, R->ny).steps;
-  auto enqueue = [&](int k) -> int {
+  int body = std::max(0, (n - (n % 2 ? 1 : 2)) / K);
+  n -= body * K;
+  while (body > 0 || n >= 2) {
+    const int k = body > 0 ? K : 2;
+    if (body > 0) --body;
+    else n -= 2;
     const hipError_t e = launch_march_linear(dev_view(g_tree, *R, true, true), k, g_stream);
     if (e != hipSuccess) return fail(200 + (int)e, "marching launch failed: %s", hipGetErrorString(e));
     R->cur = 1 - R->cur;
     g_tree.ctl_in = 1 - g_tree.ctl_in;
-    return 0;
-  };
-  int body = std::max(0, (n - (n % 2 ? 1 : 2)) / K);
-  n -= body * K;
-  // Launches per captured graph (an even number: it replays from the level
-  // parity it was captured at).  Capturing pays from a few replays on.
-  constexpr int kPer = 8;
-  if (use_graph && body >= 4 * kPer) {
-    hipGraph_t graph = nullptr;
-    hipGraphExec_t exec = nullptr;
-    HIPCHK(hipStreamBeginCapture(g_stream, hipStreamCaptureModeThreadLocal));
-    int r = 0;
-    for (int k = 0; k < kPer && !r; ++k) r = enqueue(K);
-    hipError_t ce = hipStreamEndCapture(g_stream, &graph);
-    if (r) return r;
-    HIPCHK(ce);
-    HIPCHK(hipGraphInstantiate(&exec, graph, nullptr, nullptr, 0));
-    for (; body >= kPer; body -= kPer) HIPCHK(hipGraphLaunch(exec, g_stream));
-    HIPCHK(hipStreamSynchronize(g_stream));
-    (void)hipGraphExecDestroy(exec);
-    (void)hipGraphDestroy(graph);
   }
-  for (; body > 0; --body)
-    if (int r = enqueue(K)) return r;
-  for (; n >= 2; n -= 2)
-    if (int r = enqueue(2)) return r;
   if (n > 0)
     if (int r = tree_enqueue_root_step(g_tree, g_stream)) return r;
   return sync();
 }
 
-// n root steps of the device loop, no output files
-static int run_plain(int n, int use_graph) {
-  if (marches()) return run_marched(n, use_graph);
-  if (tree_step2_eligible(g_tree) && n >= 2) {
-    // a linear single layer: two root steps per launch; a graph of two
-    // launches (four steps) brings the level parity back for replay
-    if (use_graph && n >= 4) {
-      hipGraph_t graph = nullptr;
-      hipGraphExec_t exec = nullptr;
-      HIPCHK(hipStreamBeginCapture(g_stream, hipStreamCaptureModeThreadLocal));
-      int r = tree_enqueue_root_steps2(g_tree, g_stream);
-      if (!r) r = tree_enqueue_root_steps2(g_tree, g_stream);
-      hipError_t ce = hipStreamEndCapture(g_stream, &graph);
-      if (r) return r;
-      HIPCHK(ce);
-      HIPCHK(hipGraphInstantiate(&exec, graph, nullptr, nullptr, 0));
-      for (int k = 0; k + 3 < n; k += 4) HIPCHK(hipGraphLaunch(exec, g_stream));
-      HIPCHK(hipStreamSynchronize(g_stream));
-      (void)hipGraphExecDestroy(exec);
-      (void)hipGraphDestroy(graph);
-      n = n % 4;
-    }
+// n root steps of the device loop, no output files.  The launches are
+// enqueued one by one: the host stays ahead of the device (2 - 3 us a launch
+// against 3.6 us for the shortest kernel), and a replayed graph of one or two
+// root steps costs about 2 us per replay on top of its kernels (517x391
+// nonlinear 10.8 us per step as graphs, 8.6 enqueued; 96x72 9.3 and 7.1;
+// 1024x768 + 601x601 nest 68.5 and 65.6; linear layers 0.1 - 0.3 us).
+static int run_plain(int n) {
+  if (marches()) return run_marched(n);
+  if (tree_step2_eligible(g_tree))  // a linear single layer: two root steps per launch
     for (; n >= 2; n -= 2)
       if (int r = tree_enqueue_root_steps2(g_tree, g_stream)) return r;
-    for (; n > 0; --n)
-      if (int r = tree_enqueue_root_step(g_tree, g_stream)) return r;
-    return sync();
-  }
+  // a linear root with nested layers: every root step but the last computes
+  // the next one's continuity in its momentum launch
   g_tree.mass_ahead = false;
-  if (tree_fuses_halves(g_tree)) {
-    // every root step but the last computes the next one's continuity in
-    // its momentum launch; the first step (outside any graph) leaves the
-    // tree in the state each captured pair starts and ends in
-    int left = n;
-    if (left > 0) {
-      if (int r = tree_enqueue_root_step(g_tree, g_stream, left > 1)) return r;
-      --left;
-    }
-    if (use_graph && left >= 3 && tree_launches_per_step(g_tree) <= kGraphMaxLaunches) {
-      hipGraph_t graph = nullptr;
-      hipGraphExec_t exec = nullptr;
-      HIPCHK(hipStreamBeginCapture(g_stream, hipStreamCaptureModeThreadLocal));
-      int r = tree_enqueue_root_step(g_tree, g_stream, true);
-      if (!r) r = tree_enqueue_root_step(g_tree, g_stream, true);
-      hipError_t ce = hipStreamEndCapture(g_stream, &graph);
-      if (r) return r;
-      HIPCHK(ce);
-      HIPCHK(hipGraphInstantiate(&exec, graph, nullptr, nullptr, 0));
-      const int reps = (left - 1) / 2;  // at least one step stays for the end
-      for (int k = 0; k < reps; ++k) HIPCHK(hipGraphLaunch(exec, g_stream));
-      HIPCHK(hipStreamSynchronize(g_stream));
-      (void)hipGraphExecDestroy(exec);
-      (void)hipGraphDestroy(graph);
-      left -= 2 * reps;
-    }
-    for (; left > 0; --left)
-      if (int r = tree_enqueue_root_step(g_tree, g_stream, left > 1)) return r;
-    return sync();
-  }
-  if (use_graph && n >= 2 && tree_launches_per_step(g_tree) <= kGraphMaxLaunches) {
-    // Two root steps bring every layer's level parity back to where it
-    // started (children with odd REL_TIME flip once per root step), so a
-    // captured pair can be replayed.
-    hipGraph_t graph = nullptr;
-    hipGraphExec_t exec = nullptr;
-    HIPCHK(hipStreamBeginCapture(g_stream, hipStreamCaptureModeThreadLocal));
-    int r = tree_enqueue_root_step(g_tree, g_stream);
-    if (!r) r = tree_enqueue_root_step(g_tree, g_stream);
-    hipError_t ce = hipStreamEndCapture(g_stream, &graph);
-    if (r) return r;
-    HIPCHK(ce);
-    HIPCHK(hipGraphInstantiate(&exec, graph, nullptr, nullptr, 0));
-    for (int k = 0; k + 1 < n; k += 2) HIPCHK(hipGraphLaunch(exec, g_stream));
-    HIPCHK(hipStreamSynchronize(g_stream));
-    (void)hipGraphExecDestroy(exec);
-    (void)hipGraphDestroy(graph);
-    n = n % 2;
-  }
-  for (int k = 0; k < n; ++k)
-    if (int r = tree_enqueue_root_step(g_tree, g_stream)) return r;
+  const bool ahead = tree_fuses_halves(g_tree);
+  for (; n > 0; --n)
+    if (int r = tree_enqueue_root_step(g_tree, g_stream, ahead && n > 1)) return r;
   return sync();
 }
 
@@ -606,11 +523,12 @@ static int fire_faults(long long k) {
 }
 
 int gcomcot_run_steps_(int *nsteps, int *use_graph) {
+  (void)use_graph;
   int n = *nsteps;
   if (n < 0) return fail(23, "negative step count");
   if (!layer(1)) return fail(8, "no root layer");
   if (int e = ensure_init()) return e;
-  if (!out_active() && g_faults.empty()) return run_plain(n, *use_graph);
+  if (!out_active() && g_faults.empty()) return run_plain(n);
   // the run is cut at every root step that writes files or before which a
   // fault ruptures; files are packed on the step stream and written while
   // the loop goes on
@@ -633,7 +551,7 @@ int gcomcot_run_steps_(int *nsteps, int *use_graph) {
         break;
       }
     }
-    if (int r = run_plain((int)m, *use_graph)) return r;
+    if (int r = run_plain((int)m)) return r;
     done += (int)m;
     n -= (int)m;
     if (out_due(g_tree, done))

@@ -88,6 +88,8 @@ struct Group {
   int lane = 0;
 };
 
+constexpr int kDirectPasses = 16;  // passes over a plan before it is captured
+
 struct Plan {
   // root steps of the plan: 2, or 4 when single-layer linear roots take one
   // two-step launch per pair of root steps (their level parity comes back
@@ -102,6 +104,7 @@ struct Plan {
   hipGraphExec_t exec = nullptr;
   long long cells_per_step = 0;
   bool owns_arena = true;  // false: the engine's reusable arena
+  long long passes = 0;    // times it ran
 };
 
 struct Engine {
@@ -736,28 +739,29 @@ int build_plan(const std::vector<Scenario *> &act) {
       if (g.type == kStepGroup) cells += g.cells * (g.mode == kTwoStep ? 2 : 1);
   P.cells_per_step = cells / P.nsteps;
   if (int r = upload_plan(P, true)) return r;
-  size_t per_step = 0;
-  for (int k = 0; k < P.nsteps; ++k) per_step = std::max(per_step, P.step[k].size());
-  if (!g_eng.graphs || per_step + 1 > (size_t)kGraphMaxLaunches) {
-    // a very deep sub-stepping (huge REL_TIME) is enqueued step by step:
-    // graphs of that many nodes are not worth building
-    g_eng.plan_valid = true;
-    ++g_eng.plans_built;
-    return 0;
-  }
   for (int r = 0; r < P.nsteps; ++r)
     for (const auto &g : P.step[r])
-      if (g.type == kStepGroup && g.mode != kTwoStep)
+      if (g.type == kStepGroup && g.mode != kTwoStep)  // looked up before any capture
         HIPCHK(launch_batch(step_launch(P, g), g.mode, g.nl != 0, g.sph != 0, g.shape,
                             g_eng.st, true));
+  g_eng.plan_valid = true;
+  ++g_eng.plans_built;
+  return 0;
+}
+
+// Capture the plan's launches in a HIP graph (none for a very deep
+// sub-stepping, a huge REL_TIME: graphs of that many nodes are not worth
+// building).
+int capture_plan(Plan &P) {
+  size_t per_step = 0;
+  for (int k = 0; k < P.nsteps; ++k) per_step = std::max(per_step, P.step[k].size());
+  if (per_step + 1 > (size_t)kGraphMaxLaunches) return 0;
   HIPCHK(hipStreamBeginCapture(g_eng.st, hipStreamCaptureModeThreadLocal));
   int r = enqueue_plan(P, 0, P.nsteps);
   hipError_t ce = hipStreamEndCapture(g_eng.st, &P.graph);
   if (r) return r;
   HIPCHK(ce);
   HIPCHK(hipGraphInstantiate(&P.exec, P.graph, nullptr, nullptr, 0));
-  g_eng.plan_valid = true;
-  ++g_eng.plans_built;
   return 0;
 }
 
@@ -779,9 +783,15 @@ int run(long long n) {
                    g_eng.plan_valid ? "kept" : "rebuilt");
     if (!g_eng.plan_valid)
       if (int r = build_plan(act)) return r;
-    const Plan &P = g_eng.plan;
+    Plan &P = g_eng.plan;
     const int ns = P.nsteps;
     for (long long k = 0; k + ns <= m; k += ns) {
+      // The first passes over a plan are enqueued launch by launch, which
+      // keeps the device as busy as a graph does; building one costs 0.4 ms,
+      // as much as a pass, so only plans that live longer get theirs.
+      if (g_eng.graphs && !P.exec && P.passes == kDirectPasses)
+        if (int r = capture_plan(P)) return r;
+      ++P.passes;
       if (P.exec) {
         HIPCHK(hipGraphLaunch(P.exec, g_eng.st));
         ++g_eng.graph_replays;

@@ -149,8 +149,9 @@ int gcomcot_init_layer_ex_(int *layerid, int *parent, int *level, int *laycord, 
 
 /* Run *nsteps complete root steps on the device (mass+open, nested
  * layers, momentum, wet-only max and arrival, level rotation) as one
- * enqueued sequence (captured in a HIP graph when *use_graph != 0).
- * Returns 0 or an error code. */
+ * enqueued sequence.  *use_graph is accepted either way: replaying HIP
+ * graphs was slower than enqueuing on every layer size measured, so none
+ * are captured.  Returns 0 or an error code. */
 int gcomcot_run_steps_(int *nsteps, int *use_graph);
 
 /* Same work as gcomcot_run_steps_ without a graph, timed with HIP events
