@@ -8,8 +8,9 @@
 //   fused step of every single-layer root      } persistent step kernel,
 //   continuity half of every nested root       } one launch per layer kind
 //   for each child slot s, sub-step k = 1..max REL_TIME:
-//     JNQ/NEWQ of every child s with k <= its REL_TIME   (one launch; an
-//       SC_OPTION = 1 child takes its band and edge launches instead)
+//     JNQ/NEWQ of every child s with k <= its REL_TIME that the last one
+//       did not cover (jnq_ahead: sub-steps 1 and nhalf + 1)  (one launch;
+//       an SC_OPTION = 1 child takes its band and edge launches instead)
 //     fused step of those children                       (one per kind)
 //     JNZ of the children at their half step             (one launch; JNZ_SC
 //       per SC_OPTION = 1 child)
@@ -312,6 +313,7 @@ void emit_step(const std::vector<Scenario *> &act, std::vector<Group> &out, int 
       if (R.children.size() > sib)
         maxrt = std::max(maxrt, s->tree.layers[R.children[sib]].rel_time);
     }
+    std::vector<std::pair<int, int>> jnq(act.size(), {0, 0});  // each child's last JNQ: k0, ahead
     for (int k = 1; k <= maxrt; ++k) {
       Group jq;
       jq.type = kJnqGroup;
@@ -323,15 +325,22 @@ void emit_step(const std::vector<Scenario *> &act, std::vector<Group> &out, int 
       se.t = k;
       sz.type = kScJnzGroup;
       std::vector<LayerRec *> moved;
-      for (Scenario *s : act) {
-        Tree &T = s->tree;
+      for (size_t a = 0; a < act.size(); ++a) {
+        Tree &T = act[a]->tree;
         LayerRec &R = *T.layer(1);
         if (R.children.size() <= sib) continue;
         LayerRec &C = T.layers[R.children[sib]];
         if (k > C.rel_time) continue;
-        if (C.sc) se.scs.push_back(sc_view(T, R, C));
-        else jq.nests.push_back(nest_view(R, C));
-        pend_add(pend, kFused, T, C, dev_view(T, C, true, false));
+        auto &[k0, ahead] = jnq[a];
+        if (C.sc) {
+          se.scs.push_back(sc_view(T, R, C));
+        } else if (k0 == 0 || k > k0 + ahead) {
+          DevNest q = nest_view(R, C);
+          k0 = k;
+          q.ahead = ahead = jnq_ahead(C, k);
+          jq.nests.push_back(q);
+        }
+        pend_add(pend, kFused, T, C, substep_view(T, C, true, k, k0, ahead));
         moved.push_back(&C);
       }
       if (!jq.nests.empty()) out.push_back(std::move(jq));

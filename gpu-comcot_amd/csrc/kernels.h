@@ -48,7 +48,14 @@ struct DevLayer {
   // bytes of the layer's block, which starts with h and holds every plane
   // above; 0 when they do not fit in one buffer descriptor (4 GB)
   unsigned block_bytes;
+  // A nested layer's boundary fluxes of the next sub-step (one slot of
+  // DevNest::edge) or null: a fused step then writes them, under JNQ's wet
+  // test, where it otherwise writes 0, and the next sub-step needs no JNQ.
+  const float *edge;
 };
+// Slot layout: M of rows 1..NY at column 1 and at column NX, then N of
+// columns 1..NX at row 1 and at row NY.
+constexpr size_t edge_floats(int nx, int ny) { return 2 * ((size_t)nx + ny); }
 
 // kMomentMass: the momentum half of root step k of a linear outermost
 // layer with nested layers, with the continuity (+ open boundary) of step
@@ -152,6 +159,10 @@ struct DevNest {
   const float *ch, *cz1, *cz2;
   float *cm1, *cn1;      // child level-1 fluxes, boundary written
   float *pz2_out;        // parent level-2 Z, footprint written by JNZ
+  // the interface fluxes of the next `ahead` sub-steps, before the wet test,
+  // go to ahead slots of edge (see DevLayer::edge)
+  int ahead;
+  float *edge;
 };
 hipError_t launch_jnq(const DevNest &N, int t, hipStream_t st);
 hipError_t launch_jnz(const DevNest &N, hipStream_t st);

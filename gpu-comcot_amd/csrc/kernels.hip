@@ -734,8 +734,8 @@ __device__ __forceinline__ void tile_body(const DevLayer &L, int t, int ti0, int
     const int i = ti0 + idx % TX, j = tj0 + idx / TX;
     if (!IN && (i > nx || j > ny)) continue;
     const size_t g = (size_t)(j - 1) * nx + (i - 1);
+    float zo = 0.0f;
     if (MODE != kMomentOnly) {
-      float zo;
       if (IN || L.is_root || (i >= 2 && j >= 2)) zo = s.Z2(i, j);
       else if (i == 1 && j == 1) zo = s.Z2(2, 2);  // UPDATE ghosts, all_grids.f90:323-324
       else if (i == 1) zo = s.Z2(2, j);
@@ -772,6 +772,11 @@ __device__ __forceinline__ void tile_body(const DevLayer &L, int t, int ti0, int
           m2v = m2v + cx * L.dt * s.M(i, j);
           n2v = n2v + cy * L.dt * s.N(i, j);
         }
+      }
+      if (MODE == kFused && !IN && L.edge) {  // the next sub-step's boundary fluxes
+        const bool dry = s.H(i, j) + zo <= kGx;
+        if (j >= 2 && (i == 1 || i == nx)) m2v = dry ? 0.0f : L.edge[(i == 1 ? 0 : ny) + (j - 1)];
+        if (i >= 2 && (j == 1 || j == ny)) n2v = dry ? 0.0f : L.edge[2 * ny + (j == 1 ? 0 : nx) + (i - 1)];
       }
       st_plane<ST>(L.m2 + g, m2v);
       st_plane<ST>(L.n2 + g, n2v);
@@ -1178,6 +1183,8 @@ __global__ void k_max(DevLayer L, float *zmax_raw) {
 // a few waves deep, so it lasts as long as its chain of dependent loads (the
 // form that evaluated three fluxes per thread behind their wet tests took 6.1
 // us per launch on a 512x384 + 401x401 nest, 7 - 8 us over a batch's nests).
+// One launch also makes the fluxes of the N.ahead sub-steps that follow: they
+// differ in the two weights only.
 __device__ __forceinline__ int jnq_threads(const DevNest &N) {
   return 2 * (N.je - N.js + 5) + 2 * (N.ie - N.is + 5);
 }
@@ -1216,12 +1223,14 @@ __device__ void jnq_wave(const DevNest &N, int w, int t) {
   const float *own1 = vert ? N.pm1 : N.pn1, *cross1 = vert ? N.pn1 : N.pm1;
   const float f1 = own1[f];
   float hf = 0, ha = 0, zf = 0, za = 0, x0 = 0, x1 = 0, x2 = 0, x3 = 0, rp = 0, rc = 0, cached = 0;
-  if (t > 1) {
+  const int last = t + N.ahead;
+  const bool forecast = t <= 2 && last >= 2;
+  if (last > 1) {
     hf = N.ph[f];
     ha = N.ph[a];
     zf = N.pz2[f];
     za = N.pz2[a];
-    if (t > 2) {
+    if (!forecast) {
       cached = vert ? N.yflux[(side & 1) * N.pny + (k - 1)] : N.xflux[(side & 1) * pnx + (k - 1)];
     } else if (N.p_sph) {
       // TOT_N at (I, J), (I+1, J), (I, J-1), (I+1, J-1); TOT_M at (I-1, J),
@@ -1243,50 +1252,58 @@ __device__ void jnq_wave(const DevNest &N, int w, int t) {
     zc[q] = use ? N.cz1[c0 + q * cs] : 0.0f;
   }
 
+  // The forecast, one step of the parent's linear momentum (:706-720,
+  // 778-790), is made at sub-step 2 and kept for the later ones.
+  const bool wet = (hf + zf > kGx) && (ha + za > kGx);
+  if (forecast) {
+    const float hm = hf > kGx ? 0.5f * (hf + ha) : 0.0f;
+    float x;
+    if (N.p_sph) {
+      const float tot = x0 + x1 + x2 + x3;
+      const float r = N.p_r24 || N.p_nl ? rp : rp * fmaxf(hm, 0.0f);
+      x = vert ? f1 - r * (za - zf) + rc * tot : f1 - r * (za - zf) - rc * tot;
+    } else {
+      const float h = hm + 0.5f * (zf + za);
+      x = f1 - (vert ? N.pgrx : N.pgry) * h * (za - zf);
+    }
+    if (fabsf(x) < kEps) x = 0.0f;
+    cached = x;
+    if (in && wet && lane >= 1 && lane <= kJnqSpan) {
+      if (vert) N.yflux[(side & 1) * N.pny + (k - 1)] = x;
+      else N.xflux[(side & 1) * pnx + (k - 1)] = x;
+    }
+  }
   // Parent flux on the interface line at k: JNQ takes the parent's level-1
   // flux as is (:484-487); NEWQ blends it with the forecast where both parent
-  // cells are wet and is 0 elsewhere (:703-727, 774-796).  The forecast, one
-  // step of the parent's linear momentum (:706-720, 778-790), is made at
-  // sub-step 2 and kept for the later ones.
-  float flux = f1;
-  if (t > 1) {
-    const bool wet = (hf + zf > kGx) && (ha + za > kGx);
-    if (t == 2) {
-      const float hm = hf > kGx ? 0.5f * (hf + ha) : 0.0f;
-      float x;
-      if (N.p_sph) {
-        const float tot = x0 + x1 + x2 + x3;
-        const float r = N.p_r24 || N.p_nl ? rp : rp * fmaxf(hm, 0.0f);
-        x = vert ? f1 - r * (za - zf) + rc * tot : f1 - r * (za - zf) - rc * tot;
-      } else {
-        const float h = hm + 0.5f * (zf + za);
-        x = f1 - (vert ? N.pgrx : N.pgry) * h * (za - zf);
-      }
-      if (fabsf(x) < kEps) x = 0.0f;
-      cached = x;
-      if (in && wet && lane >= 1 && lane <= kJnqSpan) {
-        if (vert) N.yflux[(side & 1) * N.pny + (k - 1)] = x;
-        else N.xflux[(side & 1) * pnx + (k - 1)] = x;
-      }
-    }
-    const float w1 = ((float)t - 1.0f) / (float)N.rel_time;
-    const float w2 = 1.0f - w1;
-    flux = wet ? w1 * cached + w2 * f1 : 0.0f;
-  }
-  // EDGEINTERP_VERT/HORI (:502-604)
-  const float fm = west(flux), fp = east(flux);
-  if (!own) return;
-  const float fs = 0.5f * (fm + flux);
-  const float fe = 0.5f * (fp + flux);
-  const float c1 = (fe - fs) / (float)(2 * R);  // == REAL((fe-fs)/DBLE(nn)), :538
-  const float c2 = -c1 + fs;
+  // cells are wet and is 0 elsewhere (:703-727, 774-796).
   float *cf = vert ? N.cm1 : N.cn1;
+  float *ef = N.edge + (vert ? (side == 0 ? 0 : N.cny) : 2 * N.cny + (side == 2 ? 0 : N.cnx)) + base;
+  for (int u = t; u <= last; ++u) {
+    float flux = f1;
+    if (u > 1) {
+      const float w1 = ((float)u - 1.0f) / (float)N.rel_time;
+      const float w2 = 1.0f - w1;
+      flux = wet ? w1 * cached + w2 * f1 : 0.0f;
+    }
+    // EDGEINTERP_VERT/HORI (:502-604)
+    const float fm = west(flux), fp = east(flux);
+    const float fs = 0.5f * (fm + flux);
+    const float fe = 0.5f * (fp + flux);
+    const float c1 = (fe - fs) / (float)(2 * R);  // == REAL((fe-fs)/DBLE(nn)), :538
+    const float c2 = -c1 + fs;
+    if (u > t) {  // a later sub-step: before the wet test
+      if (own)
+        for (int q = 0; q < R; ++q) ef[q] = 2.0f * (float)(q + 1) * c1 + c2;
+      ef += edge_floats(N.cnx, N.cny);
+    } else if (own) {
 #pragma unroll
-  for (int q = 0; q < kJnqLoads; ++q)
-    if (q < R) cf[c0 + q * cs] = hc[q] + zc[q] <= kGx ? 0.0f : 2.0f * (float)(q + 1) * c1 + c2;
-  for (int q = kJnqLoads; q < R; ++q)
-    cf[c0 + q * cs] =
-        N.ch[c0 + q * cs] + N.cz1[c0 + q * cs] <= kGx ? 0.0f : 2.0f * (float)(q + 1) * c1 + c2;
+      for (int q = 0; q < kJnqLoads; ++q)
+        if (q < R) cf[c0 + q * cs] = hc[q] + zc[q] <= kGx ? 0.0f : 2.0f * (float)(q + 1) * c1 + c2;
+      for (int q = kJnqLoads; q < R; ++q)
+        cf[c0 + q * cs] =
+            N.ch[c0 + q * cs] + N.cz1[c0 + q * cs] <= kGx ? 0.0f : 2.0f * (float)(q + 1) * c1 + c2;
+    }
+  }
 }
 
 __global__ void __launch_bounds__(128) k_jnq(DevNest N, int t) {

@@ -127,8 +127,19 @@ __device__ __forceinline__ void march_nl(const DevLayer &L, const Strip S, int s
                  oz2 = plane_off(L, L.z2), om2 = plane_off(L, L.m2), on2 = plane_off(L, L.n2),
                  omax = plane_off(L, L.zmax), oarr = plane_off(L, L.arrival);
   const float zt = breaking_floor(L.dt);
+  // a nested layer's boundary fluxes of the next sub-step: M of the side
+  // columns comes row by row, N of rows 1 and NY once.  Lanes without one, and
+  // every lane where there are none, read past the table: 0.
+  const bool has_edge = (COL || ROW) && L.edge;
+  const Block E = __builtin_amdgcn_make_buffer_rsrc(
+      const_cast<float *>(L.edge), 0, has_edge ? (int)(edge_floats(nx, ny) * sizeof(float)) : 0, 0x00027000);
+  const Mask edge_col = has_edge ? col1 | coln : 0;
+  auto edge_n = [&](int row_off) {
+    return get(E, has_edge && i >= 1 && i <= nx ? (row_off + i - 1) * 4 : kNoStore, 0);
+  };
+  const float n_lo = ROW ? edge_n(2 * ny) : 0.0f, n_hi = ROW ? edge_n(2 * ny + nx) : 0.0f;
 
-  float ph[D], pz[D], pm[D], pn[D], pq[D];
+  float ph[D], pz[D], pm[D], pn[D], pq[D], pe[D];
   auto load = [&](int j, int k) {
     const unsigned b = (unsigned)((ROW ? min(max(j, 1), ny) : min(j, rb)) - 1) * pitch;
     ph[k] = get(B, vld, b);
@@ -136,11 +147,16 @@ __device__ __forceinline__ void march_nl(const DevLayer &L, const Strip S, int s
     pm[k] = get(B, vld, om1 + b);
     pn[k] = get(B, vld, on1 + b);
     if (MX) pq[k] = get(B, vld, omax + b);
+    if (COL) {
+      const int je = min(max(j, 1), ny) - 1;
+      pe[k] = get(E, lanes(edge_col) ? ((i == 1 ? 0 : ny) + je) * 4 : kNoStore, 0);
+    }
   };
 #pragma unroll
   for (int k = 0; k < D; ++k) load(ra + k, k);
   // rows r, r - 1, r - 2 at index 0, 1, 2
   float H[3] = {}, M[2] = {}, N[3] = {}, NR[2] = {}, Z[3] = {}, DZ[3] = {}, brk[3] = {1, 1, 1};
+  float me[2] = {};
   float d1[2] = {}, xqq[2] = {}, pp[2] = {}, pc[3] = {};              // X points
   float e1[3] = {}, xpp[3] = {}, qq[4] = {}, qc[3] = {};              // Y points
   Mask W[3] = {}, ZD[3] = {};   // DZ > GX, DZ < GX
@@ -162,6 +178,7 @@ __device__ __forceinline__ void march_nl(const DevLayer &L, const Strip S, int s
     M[0] = pm[k];
     N[0] = pn[k];
     const float z1 = pz[k], zl = MX ? pq[k] : 0.0f;
+    if (COL) me[0] = pe[k];
     load(r + D, k);
     vz[0] = r >= S.j0 && r <= S.j1 ? vst : kNoStore;
 
@@ -300,6 +317,10 @@ __device__ __forceinline__ void march_nl(const DevLayer &L, const Strip S, int s
         X = div_inrange(X, 1.0f + FF);
         X = limited(X, DD, act);
       }
+      if (COL) {
+        const bool dry = H[1] + (lanes(col1) ? f.zb : Z[1]) <= kGx;
+        X = lanes(!ROW || j >= 2 ? edge_col : 0) ? (dry ? 0.0f : me[1]) : X;
+      }
       put<ST>(B, vz[1], om2 + (unsigned)(j - 1) * pitch, X);
     }
     // ---- Y momentum at row j = r - 2
@@ -330,12 +351,17 @@ __device__ __forceinline__ void march_nl(const DevLayer &L, const Strip S, int s
         Y = div_inrange(Y, 1.0f + FF);
         Y = limited(Y, DD, act);
       }
+      if (ROW && has_edge && (j == 1 || j == ny)) {
+        const bool dry = H[2] + (j == 1 ? Z[1] : Z[2]) <= kGx;
+        Y = lanes(~col1) ? (dry ? 0.0f : (j == 1 ? n_lo : n_hi)) : Y;
+      }
       put<ST>(B, vz[2], on2 + (unsigned)(j - 1) * pitch, Y);
     }
     // ---- the rows move on
 #define GC_SHIFT2(a) a[1] = a[0]
 #define GC_SHIFT3(a) a[2] = a[1], a[1] = a[0]
     GC_SHIFT3(H); GC_SHIFT2(M); GC_SHIFT3(N); GC_SHIFT2(NR); GC_SHIFT3(Z); GC_SHIFT3(DZ); GC_SHIFT3(brk);
+    if (COL) GC_SHIFT2(me);
     GC_SHIFT2(d1); GC_SHIFT2(xqq); GC_SHIFT2(pp); GC_SHIFT3(pc);
     e1[2] = e1[1]; xpp[2] = xpp[1]; qc[2] = qc[1];
     qq[3] = qq[2]; qq[2] = qq[1];

@@ -7,6 +7,7 @@
 
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cstddef>
 #include <vector>
 
@@ -14,6 +15,9 @@
 
 namespace gc {
 
+// Sub-steps whose boundary fluxes a nested layer keeps room for: JNQ runs
+// again where a REL_TIME asks for more.
+constexpr int kMaxEdgeSlots = 8;
 constexpr int kMaxLayers = 20;  // layer ids 1..19 (GPUHeader.h:51)
 // Launch sequences longer than this per root step are not captured into
 // HIP graphs (deep sub-stepping, e.g. a REL_TIME in the thousands).
@@ -35,6 +39,8 @@ struct LayerRec {
   float *dzp = nullptr, *xflux = nullptr, *yflux = nullptr;
   int *arrival = nullptr;
   float *rowc = nullptr;    // row-major copy of the coefficients (DevLayer::rowc)
+  float *edge = nullptr;    // nested layers: boundary fluxes of coming sub-steps, behind the
+  int edge_slots = 0;       // planes of block (DevLayer::edge), one slot per sub-step
   float *deform = nullptr;  // last seafloor deformation applied (on first use)
   float *sponge = nullptr;  // SPONGE_COEF: COEFX[NX] then COEFY[NY] (layer 1, when on)
   // SC_OPTION = 1 (Cartesian child of a spherical layer 1): POS, CXY, the
@@ -133,6 +139,21 @@ void tree_free(Tree &T);
 
 DevLayer dev_view(const Tree &T, const LayerRec &L, bool with_max, bool advance);
 DevNest nest_view(const LayerRec &P, const LayerRec &C);
+// JNQ of sub-step k of a child whose steps are fused launches: one launch
+// serves sub-steps k .. k + ahead.  What JNQ reads of the parent stays as it is
+// until JNZ (sub-step nhalf) writes the parent's Z; only its wet test needs
+// the child's newest Z, so each step writes the next sub-step's fluxes itself
+// (DevLayer::edge).  A JNQ is a launch of a few waves, nearly all latency
+// (3.7 us for a nest, 4.9 for a batch's); two of REL_TIME remain.  Measured:
+// 512x384 + 401x401 with REL_TIME 4 59 us per root step, 53 with two; sixteen
+// scenarios, four nested, 100 ms, 87.
+inline int jnq_ahead(const LayerRec &C, int k) {
+  const int nhalf = C.rel_time / 2 + 1, last = k <= nhalf ? nhalf : C.rel_time;
+  return !C.edge || !C.children.empty() ? 0 : std::min({last - k, C.rel_time - k, C.edge_slots});
+}
+// The fused step of sub-step k: its view, given that the JNQ of sub-step k0
+// covers it and up to k0 + ahead.
+DevLayer substep_view(const Tree &T, const LayerRec &C, bool with_max, int k, int k0, int ahead);
 // The SC_OPTION = 1 coupling views of parent P and child C of tree T.
 DevSc sc_view(const Tree &T, const LayerRec &P, const LayerRec &C);
 

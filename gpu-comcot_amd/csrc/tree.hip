@@ -217,10 +217,12 @@ int tree_create_layer(Tree &T, hipStream_t st, int id, int parent, int level, in
   L.ny = ny;
   const size_t n = L.nxy();
   L.block_bytes = layer_bytes(nx, ny, L.nl != 0, false);
+  L.edge_slots = id == 1 || sc ? 0 : std::min(L.rel_time / 2, kMaxEdgeSlots);
+  const size_t edges = (size_t)L.edge_slots * edge_floats(nx, ny) * sizeof(float);
   {
-    hipError_t e = hipMalloc(&L.block, L.block_bytes);
+    hipError_t e = hipMalloc(&L.block, L.block_bytes + edges);
     if (e != hipSuccess) {
-      const size_t want = L.block_bytes;
+      const size_t want = L.block_bytes + edges;
       L = LayerRec();
       return fail(100 + (int)e, "layer %d: %zu bytes of device memory: %s", id, want,
                   hipGetErrorString(e));
@@ -240,6 +242,7 @@ int tree_create_layer(Tree &T, hipStream_t st, int id, int parent, int level, in
   L.xflux = c.take<float>(2 * (size_t)nx);
   L.yflux = c.take<float>(2 * (size_t)ny);
   L.coef = c.take<float>((size_t)kNumCoef * ny);
+  if (L.edge_slots) L.edge = reinterpret_cast<float *>(static_cast<char *>(L.block) + L.block_bytes);
   HIPCHK(hipMemsetAsync(L.block, 0, L.block_bytes, st));
   HIPCHK(hipMemsetAsync(L.arrival, 0xff, n * sizeof(int), st));  // -1 = not arrived
   HIPCHK(hipMemcpyAsync(L.h, H, n * sizeof(float), hipMemcpyHostToDevice, st));
@@ -361,16 +364,26 @@ DevNest nest_view(const LayerRec &P, const LayerRec &C) {
   q.cm1 = C.m[C.cur];
   q.cn1 = C.n[C.cur];
   q.pz2_out = P.z[1 - P.cur];
+  q.edge = C.edge;
   return q;
 }
 
-int tree_launch(const Tree &T, const LayerRec &L, int mode, bool with_max, bool advance,
-                hipStream_t st) {
-  DevLayer d = dev_view(T, L, with_max, advance);
+DevLayer substep_view(const Tree &T, const LayerRec &C, bool with_max, int k, int k0, int ahead) {
+  DevLayer d = dev_view(T, C, with_max, false);
+  if (k < k0 + ahead) d.edge = C.edge + (size_t)(k - k0) * edge_floats(C.nx, C.ny);
+  return d;
+}
+
+static int launch_view(const Tree &T, const LayerRec &L, const DevLayer &d, int mode, hipStream_t st) {
   const int v = mode == kFused && L.variant >= 0 ? L.variant : T.variant;
   hipError_t e = launch_step(d, mode, L.nl != 0, L.sph != 0, v, st);
   if (e != hipSuccess) return fail(200 + (int)e, "step kernel launch failed: %s", hipGetErrorString(e));
   return 0;
+}
+
+int tree_launch(const Tree &T, const LayerRec &L, int mode, bool with_max, bool advance,
+                hipStream_t st) {
+  return launch_view(T, L, dev_view(T, L, with_max, advance), mode, st);
 }
 
 // ALL_GRID (all_grids.f90:34-308) / subgrid_solver_rcsv (GPUall_grids.cu:655-699)
@@ -415,12 +428,20 @@ int tree_enqueue_children(Tree &T, LayerRec &P, bool with_max, hipStream_t st) {
   for (int cid : P.children) {
     LayerRec &C = T.layers[cid];
     const int nhalf = (int)std::floor(C.rel_time / 2.0f) + 1;
+    int k0 = 0, ahead = 0;  // the last JNQ covers sub-steps k0 .. k0 + ahead
     for (int k = 1; k <= C.rel_time; ++k) {
-      hipError_t e = C.sc ? launch_sc_edges(sc_view(T, P, C), k, st)
-                          : launch_jnq(nest_view(P, C), k, st);
+      hipError_t e = hipSuccess;
+      if (C.sc) {
+        e = launch_sc_edges(sc_view(T, P, C), k, st);
+      } else if (k0 == 0 || k > k0 + ahead) {
+        DevNest q = nest_view(P, C);
+        k0 = k;
+        q.ahead = ahead = jnq_ahead(C, k);
+        e = launch_jnq(q, k, st);
+      }
       if (e != hipSuccess) return fail(201, "jnq launch failed: %s", hipGetErrorString(e));
       if (C.children.empty()) {
-        if (int r = tree_launch(T, C, kFused, with_max, false, st)) return r;
+        if (int r = launch_view(T, C, substep_view(T, C, with_max, k, k0, ahead), kFused, st)) return r;
       } else {
         if (int r = tree_launch(T, C, kMassOnly, false, false, st)) return r;
         if (int r = tree_enqueue_children(T, C, with_max, st)) return r;

@@ -130,3 +130,38 @@ def test_batched_nonlinear_layers_by_size(count, nx, ny):
         assert diff_report(mx["zmax_wet"], om["zmax_wet"])[0] == 0, sc.name
         assert (mx["arrival"] == om["arrival"]).all(), sc.name
     b.close()
+
+
+@pytest.mark.parametrize("gov", [0, 1], ids=["linear", "nonlinear"])
+@pytest.mark.parametrize("rs,rt", [(3, 1), (2, 2), (4, 4), (7, 5), (3, 9), (5, 21)],
+                         ids=["rt1", "rt2", "rt4", "rt5", "rt9", "rt21"])
+def test_substeps_that_share_a_jnq_match_oracle(rs, rt, gov):
+    """A nested layer's steps write the boundary fluxes of the sub-step that
+    follows, under its wet test: REL_TIMEs on every remainder of what one JNQ
+    covers (21 asks for more sub-steps than its table holds), in tiles, in one
+    cell per thread, in marching strips and in a batch."""
+    from gcomcot._lib import ip, lib
+    from gcomcot.batch import Batch
+    from helpers import BEACH
+    sc = S.custom(nx=70, ny=64, laygov=0, child=dict(laycord=1, laygov=gov, footprint=(31, 27),
+                                                     rel_size=rs, rel_time=rt, corner=(8, 14)), **BEACH)
+    orc = Oracle(sc, 32, pow_mode=1)
+    orc.step(21)
+    try:
+        for v in (0, 1, 6):
+            print(f"[gpu] shared jnq {rs}/{rt} gov {gov} variant {v}", flush=True)
+            assert lib().gcomcot_set_tile_variant_(ip(v)) == 0
+            dev = DeviceRun(sc)
+            dev.run(21)
+            compare_device_oracle(sc, dev, orc, f"{rs}/{rt} variant {v}")
+            dev.close()
+    finally:
+        lib().gcomcot_set_tile_variant_(ip(0))
+    b = Batch(autotune=False)
+    sid = b.add(sc, 21)
+    b.run(21)
+    for lid in (1, 2):
+        st, o = b.state(sid, lid), orc.state(lid)
+        for k in ("z1", "m1", "n1"):
+            assert diff_report(st[k], o[k])[0] == 0, (lid, k)
+    b.close()
