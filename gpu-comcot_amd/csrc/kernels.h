@@ -96,6 +96,8 @@ inline bool march_applies(const DevLayer &L) {
   return L.is_root && L.rowc && !L.r24 && !L.zraw && !L.sponge_cx && L.block_bytes != 0;
 }
 hipError_t launch_march_linear(const DevLayer &L, int steps, hipStream_t st);
+// kMomentMass of a spherical root in the marching form
+hipError_t launch_march_moment_mass(const DevLayer &L, hipStream_t st);
 
 // One fused step of a nonlinear layer with friction and convection in the
 // marching kernels (march_nl.hip), in segments of seg rows; march_nl_seg

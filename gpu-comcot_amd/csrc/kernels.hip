@@ -2002,8 +2002,9 @@ hipError_t launch_step(const DevLayer &L, int mode, bool nl, bool sph, int varia
     if (sph) return few ? launch_small<true, 4>(L, st) : launch_small<true, 8>(L, st);
     return few ? launch_small<false, 4>(L, st) : launch_small<false, 8>(L, st);
   }
-  if (mode == kMomentMass) {  // outermost linear layers with nested layers: 64x8
+  if (mode == kMomentMass) {  // outermost linear layers with nested layers
     if (nl) return hipErrorInvalidValue;
+    if (sph && march_applies(L)) return launch_march_moment_mass(L, st);
     return sph ? launch_t<kMomentMass, false, true, 64, 8>(L, st)
                : launch_t<kMomentMass, false, false, 64, 8>(L, st);
   }

@@ -165,3 +165,22 @@ def test_substeps_that_share_a_jnq_match_oracle(rs, rt, gov):
         for k in ("z1", "m1", "n1"):
             assert diff_report(st[k], o[k])[0] == 0, (lid, k)
     b.close()
+
+
+@pytest.mark.parametrize("nx,ny", [(24, 22), (61, 23), (62, 40), (63, 29), (64, 31), (124, 33), (126, 25)],
+                         ids=lambda v: str(v))
+def test_marched_moment_mass_matches_oracle(nx, ny):
+    """A nested linear root's momentum with the next step's continuity, at
+    sizes around one and two strips (62 columns) and off the segments' rows."""
+    sc = S.custom(nx=nx, ny=ny, laygov=0, cx=0.4,
+                  child=dict(laycord=1, laygov=0, footprint=(7, 6), rel_size=2, rel_time=2, corner=(6, 8)))
+    orc = Oracle(sc, 32, pow_mode=1)
+    dev = DeviceRun(sc)
+    try:
+        for n in (1, 2, 60):
+            print(f"[gpu] moment + mass {nx}x{ny} run {n}", flush=True)
+            dev.run(n)
+            orc.step(n)
+            compare_device_oracle(sc, dev, orc, f"moment + mass {nx}x{ny} after {n}")
+    finally:
+        dev.close()
