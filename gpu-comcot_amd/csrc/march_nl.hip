@@ -6,7 +6,9 @@
 // (X) and r - 1 (Y), the X momentum of row r - 1 and the Y momentum of row
 // r - 2, all from rows held in registers; neighbouring columns come from the
 // neighbouring lanes.  There is no LDS traffic but the pow/exp tables, and
-// no barrier in the loop.
+// no barrier in the loop.  A strip's halo rows skip the momentum passes: they
+// are two thirds of a row's instructions (4096x3072 118.3 us per step with
+// them, 115.5 without; 1201x901 Cartesian 20.2 and 18.3).
 //
 // The nonlinear step is bound by VALU issue (the fused tile takes 560
 // instructions per cell).  Marching shares what the tile form computes
@@ -163,7 +165,8 @@ __device__ __forceinline__ void march_nl(const DevLayer &L, const Strip S, int s
   Mask slow[3] = {};            // lanes whose breaking factor is not 1
   Mask P1[2] = {}, PX[3] = {};  // X points: depth below GX; that or a dry cell
   Mask Q1[4] = {}, QY[3] = {};  // Y points
-  int vz[3] = {kNoStore, kNoStore, kNoStore};  // store offset of the row
+  // whether row j is written: halo rows need no momentum
+  auto live = [&](int j) { return (unsigned)(j - S.j0) <= (unsigned)(S.j1 - S.j0); };
   Row4 c0 = row_coef(L, ra, 0);
 
   auto row = [&](int r, int k) __attribute__((always_inline)) {
@@ -180,7 +183,7 @@ __device__ __forceinline__ void march_nl(const DevLayer &L, const Strip S, int s
     const float z1 = pz[k], zl = MX ? pq[k] : 0.0f;
     if (COL) me[0] = pe[k];
     load(r + D, k);
-    vz[0] = r >= S.j0 && r <= S.j1 ? vst : kNoStore;
+    const int vz = live(r) ? vst : kNoStore;
 
     // ---- continuity at row r
     {
@@ -240,15 +243,15 @@ __device__ __forceinline__ void march_nl(const DevLayer &L, const Strip S, int s
         const float ze = east(Z[0]);
         const float zo = lanes(col1) ? ze : Z[0];
         if (ROW) put<ST>(B, S.j0 == 1 && r == 2 ? vst : kNoStore, oz2, zo);
-        put<ST>(B, ROW && r == 1 ? kNoStore : vz[0], oz2 + g, zo);
+        put<ST>(B, ROW && r == 1 ? kNoStore : vz, oz2 + g, zo);
       } else {
-        put<ST>(B, vz[0], oz2 + g, Z[0]);
+        put<ST>(B, vz, oz2 + g, Z[0]);
       }
       if (MX) {  // wet maximum and first arrival
         const Mask more = wet & GC_BALLOT(Z[0] > zl);
-        put<false>(B, lanes(more) ? vz[0] : kNoStore, omax + g, Z[0]);
+        put<false>(B, lanes(more) ? vz : kNoStore, omax + g, Z[0]);
         const Mask first = wet & GC_BALLOT(Z[0] >= L.arr_thr) & ~GC_BALLOT(zl >= L.arr_thr);
-        put<false>(B, lanes(first) ? vz[0] : kNoStore, oarr + g, __int_as_float(step));
+        put<false>(B, lanes(first) ? vz : kNoStore, oarr + g, __int_as_float(step));
       }
       // WAVE_BREAKING's factor (moment.f90:1272-1384; the tile kernels'
       // breaking_coef states the ranges)
@@ -296,7 +299,7 @@ __device__ __forceinline__ void march_nl(const DevLayer &L, const Strip S, int s
       const Face f{M[1], xqq[1], H[1], east(H[1]), Z[1], east(Z[1]), DZ[1], SPH ? 0.0f : east(DZ[1]),
                    d1[1], W[1], W[1] >> 1};
       float DD, DF, X = 0.0f;
-      Mask act = face_depths<SPH>(f, DD, DF);
+      Mask act = live(j) ? face_depths<SPH>(f, DD, DF) : 0;
       if (COL || ROW) act &= !ROW || (root ? j <= ny - 1 : j >= 2) ? colx : 0;
       const float pe = east(pp[1]), pw = west(pp[1]);
       if (act) {
@@ -321,14 +324,14 @@ __device__ __forceinline__ void march_nl(const DevLayer &L, const Strip S, int s
         const bool dry = H[1] + (lanes(col1) ? f.zb : Z[1]) <= kGx;
         X = lanes(!ROW || j >= 2 ? edge_col : 0) ? (dry ? 0.0f : me[1]) : X;
       }
-      put<ST>(B, vz[1], om2 + (unsigned)(j - 1) * pitch, X);
+      put<ST>(B, live(j) ? vst : kNoStore, om2 + (unsigned)(j - 1) * pitch, X);
     }
     // ---- Y momentum at row j = r - 2
     {
       const int j = r - 2;
       const Face f{N[2], xpp[2], H[2], H[1], Z[2], Z[1], DZ[2], DZ[1], e1[2], W[2], W[1]};
       float DD, DF, Y = 0.0f;
-      Mask act = face_depths<SPH>(f, DD, DF);
+      Mask act = live(j) ? face_depths<SPH>(f, DD, DF) : 0;
       if (COL || ROW) act &= !ROW || (j <= ny - 1 && (root || j >= 2)) ? coly : 0;
       const float qe = east(qc[2]), qw = west(qc[2]);
       if (act) {
@@ -355,7 +358,7 @@ __device__ __forceinline__ void march_nl(const DevLayer &L, const Strip S, int s
         const bool dry = H[2] + (j == 1 ? Z[1] : Z[2]) <= kGx;
         Y = lanes(~col1) ? (dry ? 0.0f : (j == 1 ? n_lo : n_hi)) : Y;
       }
-      put<ST>(B, vz[2], on2 + (unsigned)(j - 1) * pitch, Y);
+      put<ST>(B, live(j) ? vst : kNoStore, on2 + (unsigned)(j - 1) * pitch, Y);
     }
     // ---- the rows move on
 #define GC_SHIFT2(a) a[1] = a[0]
@@ -365,7 +368,7 @@ __device__ __forceinline__ void march_nl(const DevLayer &L, const Strip S, int s
     GC_SHIFT2(d1); GC_SHIFT2(xqq); GC_SHIFT2(pp); GC_SHIFT3(pc);
     e1[2] = e1[1]; xpp[2] = xpp[1]; qc[2] = qc[1];
     qq[3] = qq[2]; qq[2] = qq[1];
-    GC_SHIFT3(W); GC_SHIFT3(ZD); GC_SHIFT3(slow); GC_SHIFT2(P1); GC_SHIFT3(PX); GC_SHIFT3(vz);
+    GC_SHIFT3(W); GC_SHIFT3(ZD); GC_SHIFT3(slow); GC_SHIFT2(P1); GC_SHIFT3(PX);
     Q1[3] = Q1[2]; Q1[2] = Q1[1]; QY[2] = QY[1];
 #undef GC_SHIFT2
 #undef GC_SHIFT3
@@ -512,9 +515,9 @@ __global__ void __launch_bounds__(kMarchBlock)
 // 32 rows):
 //   517x391 (3 rows per SIMD)         14.4, 18.6 / 29 / 30 / 42
 //   1024x768 (13)                     21.0, 21.7 / 24 / 30 / 42
-//   1201x901 Cartesian (18)           24.9, 22.8 / 28 / 32 / 40
-//   nest 2048x1536 + 1801x1801 (54)   235, 219 / 203 / 211 / 232 per root step
-//   4096x3072 (206)                   153, 140 / 128 / 124 / 125
+//   1201x901 Cartesian (18)           24.9, 18.3 / 22.0 / 28 / 37
+//   nest 2048x1536 + 1801x1801 (54)   235, 180 / 172 / 186 / 250 per root step
+//   4096x3072 (206)                   153, 123 / 118 / 116 / 116
 int march_nl_seg(int nx, int ny) {
   const long long rows = (long long)((nx + kNlWidth - 1) / kNlWidth) * ny / 1024;
   return rows < 16 ? 0 : (rows < 36 ? 8 : (rows < 120 ? 14 : 20));
