@@ -443,7 +443,7 @@ static bool marches() {
 // steps (one step) before level 1.
 static int run_marched(int n) {
   LayerRec *R = layer(1);
-  const int K = march_plan(R->nx, R->ny).steps;
+  constexpr int K = kMarchSteps;
   int body = std::max(0, (n - (n % 2 ? 1 : 2)) / K);
   n -= body * K;
   while (body > 0 || n >= 2) {
@@ -865,7 +865,7 @@ int gcomcot_autotune_(int *reps, int *variant, int *blocking, float *ms_per_step
     }
     if (!R->nl) {
       const bool march = march_applies(dev_view(g_tree, *R, true, true));
-      const int K = march_plan(R->nx, R->ny).steps;
+      constexpr int K = kMarchSteps;
       for (int sh = 0; sh < kStep2Shapes; ++sh) {
         float ms;
         // mode 1 (shape 0) is the marching kernels where they apply

@@ -84,14 +84,10 @@ void step2_shape(int shape, int *tx, int *ty);
 
 // Root steps of a spherical linear outermost layer without children in the
 // marching kernels (march.hip): 2 or 4 per launch, level 1 in, level 2 out,
-// bookkeeping as launch_step2.  march_plan gives the steps per launch that
-// suit a layer and how its waves split it; march_applies says whether a
-// layer's view can take them (row-major coefficients, no R2/R4 planes, no
-// MAX_AMP maximum or sponge, planes within 4 GB).
-struct MarchPlan {
-  int steps, seg, seg_side;
-};
-MarchPlan march_plan(int nx, int ny);
+// bookkeeping as launch_step2.  march_applies says whether a layer's view can
+// take them (row-major coefficients, no R2/R4 planes, no MAX_AMP maximum or
+// sponge, planes within 4 GB).
+constexpr int kMarchSteps = 4;
 inline bool march_applies(const DevLayer &L) {
   return L.is_root && L.rowc && !L.r24 && !L.zraw && !L.sponge_cx && L.block_bytes != 0;
 }

@@ -8,7 +8,8 @@
 // from the neighbouring lane (DPP wave shifts, free as VALU operands).
 // There is no LDS and no barrier.  A step makes one column on each side
 // invalid, so a strip writes 64 - 2K columns, and a segment of SEG rows
-// takes SEG + 2K iterations.
+// takes SEG + 2K iterations; the first 2K, unrolled, only run the steps that
+// the strip's rows need of them (an eighth of all for SEG = 24, K = 4).
 //
 // Against the LDS tiles (k_step2) a cell costs about a third of the
 // instructions (no staging, no index arithmetic per cell, no halo ring of
@@ -96,7 +97,9 @@ __device__ __forceinline__ void march_linear(const DevLayer &L, const Strip S, i
   for (int k = 0; k < D; ++k) load(ra + k, k);
   Row4 cnext = row_coef(L, ra, 0), enext = row_coef(L, ra, 3);
 
-  auto row = [&](int r, int k) __attribute__((always_inline)) {  // k: the row's load slot
+  // k: the row's load slot; active: the steps that run (the rows that the
+  // strip's first rows need of step s + 1 begin 1 + 2 s rows after row ra)
+  auto row = [&](int r, int k, int active) __attribute__((always_inline)) {
     // ---- row r enters: shift the per-row values down
 #pragma unroll
     for (int s = K; s > 0; --s) {
@@ -137,6 +140,10 @@ __device__ __forceinline__ void march_linear(const DevLayer &L, const Strip S, i
 #pragma unroll
     for (int s = 0; s < K; ++s) {  // step s + 1 at row q
       const int q = r - s;
+      if (s >= active) {
+        if (s == active) Mb[s] = mc, Nb[s] = nc, NRb[s] = nc * C[s][2];
+        continue;
+      }
       const float hq = H[s];
       // continuity
       const float nr = nc * C[s][2];
@@ -219,9 +226,12 @@ __device__ __forceinline__ void march_linear(const DevLayer &L, const Strip S, i
   // the wait at the loop's head has to serve the entry, where they are the
   // newest operations, and would stop for everything in flight on each turn.
   __builtin_amdgcn_s_waitcnt(0x0f70);
-  for (int r = ra; r <= rb; r += D)
 #pragma unroll
-    for (int u = 0; u < D; ++u) row(r + u, u);
+  for (int u = 0; u < 2 * K; ++u) row(ra + u, u % D, (u + 1) / 2);
+  static_assert(2 * K % D == 0, "the row loop starts at load slot 0");
+  for (int r = ra + 2 * K; r <= rb; r += D)
+#pragma unroll
+    for (int u = 0; u < D; ++u) row(r + u, u, K);
 }
 
 // The momentum half of root step k of a nested linear root and the continuity
@@ -412,12 +422,12 @@ hipError_t launch_k(const DevLayer &L, int seg, int seg_side, hipStream_t st) {
 }
 
 template <int K>
-hipError_t launch_k(const DevLayer &L, const MarchPlan &p, hipStream_t st) {
+hipError_t launch_k(const DevLayer &L, int seg, int seg_side, hipStream_t st) {
   if (L.zmax)
-    return L.stream_out ? launch_k<K, true, true>(L, p.seg, p.seg_side, st)
-                        : launch_k<K, true, false>(L, p.seg, p.seg_side, st);
-  return L.stream_out ? launch_k<K, false, true>(L, p.seg, p.seg_side, st)
-                      : launch_k<K, false, false>(L, p.seg, p.seg_side, st);
+    return L.stream_out ? launch_k<K, true, true>(L, seg, seg_side, st)
+                        : launch_k<K, true, false>(L, seg, seg_side, st);
+  return L.stream_out ? launch_k<K, false, true>(L, seg, seg_side, st)
+                      : launch_k<K, false, false>(L, seg, seg_side, st);
 }
 
 // The batch form of two root steps: one workgroup per (layer, tile) item of a
@@ -454,31 +464,32 @@ __global__ void __launch_bounds__(kMarchBlock)
 
 // Rows of strips per SIMD decide the split.  With few of them a wave has
 // its SIMD to itself, an instruction then takes about 8 cycles instead of 4,
-// and a launch lasts as long as one wave's rows: short segments, and two
-// steps a launch where four would only add 2K rows to each.  Measured, us
-// per root step (two-step tiles before):
-//   517x391 (4 rows per SIMD)     K = 2, 8 rows 5.05, K = 4, 8 rows 5.58 (6.9)
-//   1024x768 (14)                 K = 4, 8 rows 5.57, 12 rows 6.9, 16 rows 7.1,
-//                                 K = 2, 8 rows 5.74 (11.0; best tile 8.5)
-//   2051x1537 (55)                K = 4, 12 rows 11.1, 16 rows 11.2, 8 rows 11.5 (28.8)
-//   4096x3072 (222)               K = 4, 24 rows 29.7, 16 rows 31, K = 2 49.7,
-//                                 K = 6, 32 rows 29.6 (99.6; best tile 72)
-// Side strips run OPEN on every row (about 1.6 times the time per row).
-MarchPlan march_plan(int nx, int ny) {
-  const long long rows = (long long)((nx + 55) / 56) * ny / 1024;
-  MarchPlan p;
-  p.steps = rows < 10 ? 2 : 4;
-  p.seg = rows < 32 ? 8 : (rows < 120 ? 12 : 24);
-  p.seg_side = rows < 120 ? 4 : 12;
-  return p;
+// and a launch lasts as long as one wave's rows: short segments.  Measured,
+// us per root step with four steps a launch (two-step tiles before):
+//   96x72 (0 rows per SIMD)  side segments of 2 rows 3.04, of 4 3.86 (6.9)
+//   517x391 (3)              4 rows, sides 2 3.33; 8, 2 3.96; 8, 4 4.00 (6.9)
+//   1024x768 (14)            8, 4 4.48; 4, 2 4.49; 12, 4 5.7 (11.0; best tile 8.5)
+//   1500x1200 (31)           12, 4 6.95; 8, 2 7.34; 4, 2 7.74
+//   2051x1537 (55)           12, 4 9.84; 20, 8 9.73; 8, 4 10.1; 16, 8 10.5 (28.8)
+//   4096x3072 (222)          20, 8 27.5; 16, 8 28.6; 24, 8 28.2; 32, 8 29.7 (99.6)
+// Two steps a launch: 3.83, 4.05, 4.90, -, 11.6, 48.  Side strips run OPEN on
+// every row (about 1.6 times the time per row).
+struct MarchPlan {
+  int seg, seg_side;
+};
+static MarchPlan march_plan(const DevLayer &L) {
+  const long long rows = (long long)((L.nx + 55) / 56) * L.ny / 1024;
+  if (rows < 10) return {4, 2};
+  if (rows < 24) return {8, 4};
+  return rows < 120 ? MarchPlan{12, 4} : MarchPlan{20, 8};
 }
 
 hipError_t launch_march_linear(const DevLayer &L, int steps, hipStream_t st) {
   if (!march_applies(L)) return hipErrorInvalidValue;
-  const MarchPlan p = march_plan(L.nx, L.ny);
+  const MarchPlan p = march_plan(L);
   switch (steps) {
-    case 2: return launch_k<2>(L, p, st);
-    case 4: return launch_k<4>(L, p, st);
+    case 2: return launch_k<2>(L, p.seg, p.seg_side, st);
+    case kMarchSteps: return launch_k<kMarchSteps>(L, p.seg, p.seg_side, st);
     default: return hipErrorInvalidValue;
   }
 }
@@ -493,11 +504,7 @@ hipError_t launch_march_linear(const DevLayer &L, int steps, hipStream_t st) {
 hipError_t launch_march_moment_mass(const DevLayer &L, hipStream_t st) {
   if (!march_applies(L)) return hipErrorInvalidValue;
   const long long rows = (long long)((L.nx + 61) / 62) * L.ny / 1024;
-  MarchPlan p;
-  p.steps = 1;
-  p.seg = rows < 8 ? 2 : (rows < 32 ? 4 : 12);
-  p.seg_side = rows < 32 ? 2 : 4;
-  return launch_k<0>(L, p, st);
+  return launch_k<0>(L, rows < 8 ? 2 : (rows < 32 ? 4 : 12), rows < 32 ? 2 : 4, st);
 }
 
 hipError_t launch_batch_march2(const BatchLaunch &B, hipStream_t st) {
