@@ -16,6 +16,7 @@
 
 #include "comcot_consts.h"
 #include "gcomcot_hip_internal.h"
+#include "hostcopy.h"
 #include "hotstart.h"
 #include "kernels.h"
 #include "output.h"
@@ -240,7 +241,7 @@ void all_grid_launch_(void) {
 
 static void copy_plane(float *host, float *dev, size_t n, bool to_dev) {
   hipError_t e = to_dev ? hipMemcpy(dev, host, n * sizeof(float), hipMemcpyHostToDevice)
-                        : hipMemcpy(host, dev, n * sizeof(float), hipMemcpyDeviceToHost);
+                        : copy_to_host(host, dev, n * sizeof(float), g_stream);
   if (e != hipSuccess) fail(204, "plane copy failed: %s", hipGetErrorString(e));
 }
 
@@ -426,6 +427,7 @@ void cuda_shutdown_(void) {
   (void)hipStreamSynchronize(g_stream);
   (void)out_disable(g_tree);
   tree_free(g_tree);
+  copy_release();
   (void)hipStreamDestroy(g_stream);
   g_stream = nullptr;
   g_init = false;
@@ -746,7 +748,7 @@ void gcomcot_get_max_(int *lid, float *zmax_wet, int *arrival) {
   if (!L) { fail(24, "gcomcot_get_max_: no layer %d", *lid); return; }
   if (sync()) return;
   copy_plane(zmax_wet, L->zmax_wet, L->nxy(), false);
-  if (hipMemcpy(arrival, L->arrival, L->nxy() * sizeof(int), hipMemcpyDeviceToHost) != hipSuccess)
+  if (copy_to_host(arrival, L->arrival, L->nxy() * sizeof(int), g_stream) != hipSuccess)
     fail(25, "arrival copy failed");
 }
 

@@ -247,7 +247,7 @@ int tree_create_layer(Tree &T, hipStream_t st, int id, int parent, int level, in
   HIPCHK(hipMemsetAsync(L.arrival, 0xff, n * sizeof(int), st));  // -1 = not arrived
   HIPCHK(hipMemcpyAsync(L.h, H, n * sizeof(float), hipMemcpyHostToDevice, st));
   HIPCHK(hipMemcpyAsync(L.z[0], Z, n * sizeof(float), hipMemcpyHostToDevice, st));
-  HIPCHK(hipMemcpyAsync(L.zmax_raw, Z, n * sizeof(float), hipMemcpyHostToDevice, st));
+  HIPCHK(hipMemcpyAsync(L.zmax_raw, L.z[0], n * sizeof(float), hipMemcpyDeviceToDevice, st));
   L.cur = 0;
   if (id != 1) T.layers[parent].children.push_back(id);
   HIPCHK(hipStreamSynchronize(st));

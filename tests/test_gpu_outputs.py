@@ -137,3 +137,29 @@ def test_outputs_off_leave_the_loop_as_it_was(tmp_path):
     dev.close()
     assert os.listdir(tmp_path) == []
     assert np.array_equal(raw.view(np.int32), np.asarray(sc.layers[0].z0, np.float32).view(np.int32))
+
+
+@pytest.mark.parametrize("nx,ny", [(2048, 1024), (2049, 1024), (1021, 6163), (4093, 2051)])
+def test_planes_read_back_whole(nx, ny):
+    """Planes on and off the sizes of the staged copy: its threshold, one slot
+    more than the ring holds, a remainder; to odd addresses, twice in a row."""
+    import ctypes
+    from gcomcot import DeviceRun
+    from gcomcot import scenarios as S
+    from gcomcot._lib import ip, last_error, lib
+    sc = S.linear_layer(nx=nx, ny=ny)
+    run = DeviceRun(sc)
+    try:
+        z = np.arange(nx * ny, dtype=np.uint32).view(np.float32)
+        lib().cuda_setz1_(z.ctypes.data_as(ctypes.c_void_p), ip(1))
+        raw = np.zeros(4 * nx * ny + 64, np.uint8)
+        for shift in (0, 4):
+            print(f"[gpu] read back {nx}x{ny} + {shift}", flush=True)
+            raw[:] = 0xa5
+            lib().cuda_getz1_(ctypes.c_void_p(raw.ctypes.data + shift), ip(1))
+            assert last_error()[0] == 0
+            assert raw[shift:shift + 4 * nx * ny].tobytes() == z.tobytes()
+            assert (raw[:shift] == 0xa5).all() and (raw[shift + 4 * nx * ny:] == 0xa5).all()
+        assert np.array_equal(run.maxima()["arrival"], np.full((ny, nx), -1, np.int32))
+    finally:
+        run.close()
