@@ -412,9 +412,13 @@ __device__ float nl_x(const DevLayer &L, const A &s, int i, int j, float brk) {
   const float p = s.M(i, j);
   const float xqq = 0.25f * (s.N(i, j) + s.N(ip1, j) + s.N(i, jm1) + s.N(ip1, jm1));
   float FF = 0.0f;
-  if (L.fric)
-    FF = div_inrange(L.kfric * sqrt_inrange(p * p + xqq * xqq),
-                     gcdet::powf_manning(DF, kManExp, *s.tab));
+  bool drag = false;
+  auto friction = [&](float x) {
+    drag = L.fric && !(SPH && drag_vanishes(kDragScale * L.kfric, p, xqq, DF, x));
+    if (drag)
+      FF = div_inrange(L.kfric * sqrt_inrange(p * p + xqq * xqq),
+                       gcdet::powf_manning(DF, kManExp, *s.tab));
+  };
   float XP;
   if (SPH) {
     const float r2 = s.CF(L, kF2, j);
@@ -426,7 +430,8 @@ __device__ float nl_x(const DevLayer &L, const A &s, int i, int j, float brk) {
     } else {
       XP = p - r2 * DD * (s.Z2(ip1, j) - s.Z2(i, j));
     }
-    if (L.fric) XP = XP - FF * p;
+    friction(XP);
+    if (drag) XP = XP - FF * p;
     XP = XP + 4.0f * s.CF(L, kR3, j) * xqq;
   } else {
     XP = p - L.grx * DD * (s.Z2(ip1, j) - s.Z2(i, j));
@@ -436,7 +441,8 @@ __device__ float nl_x(const DevLayer &L, const A &s, int i, int j, float brk) {
                    (s.Z2(i, jp1) - 2.0f * s.Z2(i, j) + s.Z2(i, jm1)));
       XP = XP - scm;
     }
-    if (L.fric) XP = XP - FF * p;
+    friction(XP);
+    if (drag) XP = XP - FF * p;
   }
   if (L.linchk == 1 && dp1_at<IN>(L, s, i, j) >= kGx &&
       (IN || (i > kSpan && i < IX - kSpan && j > kSpan && j < JY - kSpan))) {
@@ -464,7 +470,7 @@ __device__ float nl_x(const DevLayer &L, const A &s, int i, int j, float brk) {
     float advy = fy * (degy ? (qn ? -ay : ay) : (qn ? by - ay : ay - by));
     XP = XP - brk * advx - brk * advy;
   }
-  if (L.fric) XP = div_inrange(XP, 1.0f + FF);
+  if (drag) XP = div_inrange(XP, 1.0f + FF);
   if (fabsf(XP) < kEps) XP = 0.0f;
   const float lim = kVLimit * DD;
   if (fabsf(XP) > lim) XP = copysignf(lim, XP);
@@ -503,9 +509,13 @@ __device__ float nl_y(const DevLayer &L, const A &s, int i, int j, float brk) {
   const float q = s.N(i, j);
   const float xpp = 0.25f * (s.M(i, j) + s.M(i, jp1) + s.M(im1, j) + s.M(im1, jp1));
   float FF = 0.0f;
-  if (L.fric)
-    FF = div_inrange(L.kfric * sqrt_inrange(q * q + xpp * xpp),
-                     gcdet::powf_manning(DF, kManExp, *s.tab));
+  bool drag = false;
+  auto friction = [&](float x) {
+    drag = L.fric && !(SPH && drag_vanishes(kDragScale * L.kfric, q, xpp, DF, x));
+    if (drag)
+      FF = div_inrange(L.kfric * sqrt_inrange(q * q + xpp * xpp),
+                       gcdet::powf_manning(DF, kManExp, *s.tab));
+  };
   float XQ;
   if (SPH) {
     const float r4 = s.CF(L, kF4, j);
@@ -517,7 +527,8 @@ __device__ float nl_y(const DevLayer &L, const A &s, int i, int j, float brk) {
     } else {
       XQ = q - r4 * DD * (s.Z2(i, jp1) - s.Z2(i, j));
     }
-    if (L.fric) XQ = XQ - FF * q;
+    friction(XQ);
+    if (drag) XQ = XQ - FF * q;
     XQ = XQ - 4.0f * s.CF(L, kR5, j) * xpp;
   } else {
     XQ = q - L.gry * DD * (s.Z2(i, jp1) - s.Z2(i, j));
@@ -527,6 +538,7 @@ __device__ float nl_y(const DevLayer &L, const A &s, int i, int j, float brk) {
                    (s.Z2(ip1, j) - 2.0f * s.Z2(i, j) + s.Z2(im1, j)));
       XQ = XQ - scm;
     }
+    friction(XQ);
   }
   if (L.linchk == 1 && dq1_at<IN>(L, s, i, j) >= kGx &&
       (IN || (i > kSpan && i < IX - kSpan && j > kSpan && j < JY - kSpan))) {
@@ -553,7 +565,7 @@ __device__ float nl_y(const DevLayer &L, const A &s, int i, int j, float brk) {
     float advx = fx * (degx ? (pn ? -ax : ax) : (pn ? bx - ax : ax - bx));
     XQ = XQ - brk * advx - brk * advy;
   }
-  if (L.fric) XQ = div_inrange(XQ, 1.0f + FF);
+  if (drag) XQ = div_inrange(XQ, 1.0f + FF);
   if (fabsf(XQ) < kEps) XQ = 0.0f;
   const float lim = kVLimit * DD;
   if (fabsf(XQ) > lim) XQ = copysignf(lim, XQ);

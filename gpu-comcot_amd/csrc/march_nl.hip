@@ -128,7 +128,7 @@ __device__ __forceinline__ void march_nl(const DevLayer &L, const Strip S, int s
   const unsigned oz1 = plane_off(L, L.z1), om1 = plane_off(L, L.m1), on1 = plane_off(L, L.n1),
                  oz2 = plane_off(L, L.z2), om2 = plane_off(L, L.m2), on2 = plane_off(L, L.n2),
                  omax = plane_off(L, L.zmax), oarr = plane_off(L, L.arrival);
-  const float zt = breaking_floor(L.dt);
+  const float zt = breaking_floor(L.dt), kf26 = kDragScale * L.kfric;
   // a nested layer's boundary fluxes of the next sub-step: M of the side
   // columns comes row by row, N of rows 1 and NY once.  Lanes without one, and
   // every lane where there are none, read past the table: 0.
@@ -303,9 +303,13 @@ __device__ __forceinline__ void march_nl(const DevLayer &L, const Strip S, int s
       if (COL || ROW) act &= !ROW || (root ? j <= ny - 1 : j >= 2) ? colx : 0;
       const float pe = east(pp[1]), pw = west(pp[1]);
       if (act) {
-        const float FF = friction(L, f, DF, tab);
         X = f.p - (SPH ? CX[0] : L.grx) * DD * (f.zb - f.za);
-        X = X - FF * f.p;
+        const Mask drag = SPH ? act & ~GC_BALLOT(drag_vanishes(kf26, f.p, f.cross, DF, X)) : ~0ull;
+        float FF = 0.0f;
+        if (drag) {
+          FF = friction(L, f, DF, tab);
+          X = X - FF * f.p;
+        }
         if (SPH) X = X + CX[1] * f.cross;
         Mask conv = ~P1[1];
         if (COL || ROW) conv &= !ROW || (j > kSpan && j < ny - kSpan) ? conv_col : 0;
@@ -317,7 +321,7 @@ __device__ __forceinline__ void march_nl(const DevLayer &L, const Strip S, int s
         if (slow[1]) ax = brk[1] * ax, ay = brk[1] * ay;
         const float adv = X - ax - ay;
         X = lanes(conv) ? adv : X;
-        X = div_inrange(X, 1.0f + FF);
+        if (drag) X = div_inrange(X, 1.0f + FF);
         X = limited(X, DD, act);
       }
       if (COL) {
@@ -335,12 +339,14 @@ __device__ __forceinline__ void march_nl(const DevLayer &L, const Strip S, int s
       if (COL || ROW) act &= !ROW || (j <= ny - 1 && (root || j >= 2)) ? coly : 0;
       const float qe = east(qc[2]), qw = west(qc[2]);
       if (act) {
-        const float FF = friction(L, f, DF, tab);
         Y = f.p - (SPH ? CY[0] : L.gry) * DD * (f.zb - f.za);
-        if (SPH) {
-          Y = Y - FF * f.p;
-          Y = Y - CY[1] * f.cross;
+        const Mask drag = SPH ? act & ~GC_BALLOT(drag_vanishes(kf26, f.p, f.cross, DF, Y)) : ~0ull;
+        float FF = 0.0f;
+        if (drag) {
+          FF = friction(L, f, DF, tab);
+          if (SPH) Y = Y - FF * f.p;
         }
+        if (SPH) Y = Y - CY[1] * f.cross;
         Mask conv = ~Q1[2];
         if (COL || ROW) conv &= !ROW || (j > kSpan && j < ny - kSpan) ? conv_col : 0;
         const Mask qn = GC_BALLOT(f.p < 0.0f), pn = GC_BALLOT(f.cross < 0.0f);
@@ -351,7 +357,7 @@ __device__ __forceinline__ void march_nl(const DevLayer &L, const Strip S, int s
         if (slow[2]) ax = brk[2] * ax, ay = brk[2] * ay;
         const float adv = Y - ax - ay;
         Y = lanes(conv) ? adv : Y;
-        Y = div_inrange(Y, 1.0f + FF);
+        if (drag) Y = div_inrange(Y, 1.0f + FF);
         Y = limited(Y, DD, act);
       }
       if (ROW && has_edge && (j == 1 || j == ny)) {
