@@ -52,6 +52,10 @@ struct DevLayer {
   // DevNest::edge) or null: a fused step then writes them, under JNQ's wet
   // test, where it otherwise writes 0, and the next sub-step needs no JNQ.
   const float *edge;
+  // Host side, a nested layer's fused step only: the view of its linear root
+  // whose momentum + next continuity (kMomentMass) launch_step runs beside the
+  // step, in the same launch where that is faster.
+  const DevLayer *beside;
 };
 // Slot layout: M of rows 1..NY at column 1 and at column NX, then N of
 // columns 1..NX at row 1 and at row NY.
@@ -161,6 +165,10 @@ struct DevNest {
   // go to ahead slots of edge (see DevLayer::edge)
   int ahead;
   float *edge;
+  // launch_jnz, next_t > 0: JNQ/NEWQ of sub-step next_t (after UPDATE, so on
+  // the child's level 2, whose fluxes are cm2, cn2) in the same launch
+  int next_t;
+  float *cm2, *cn2;
 };
 hipError_t launch_jnq(const DevNest &N, int t, hipStream_t st);
 hipError_t launch_jnz(const DevNest &N, hipStream_t st);

@@ -25,7 +25,7 @@
 #include "detmath.h"
 #include "fastdiv.h"
 #include "kernels.h"
-#include "march.h"
+#include "march_mm.h"
 
 namespace gc {
 
@@ -1183,6 +1183,90 @@ __global__ void k_max(DevLayer L, float *zmax_raw) {
 }
 
 // ---------------------------------------------------------------- nesting
+// JNZ (all_grids.f90:342-421): parent Z2 over the footprint = mean of the
+// wet child cells, summed in the Fortran order (KI outer, KJ inner).
+// For R = 2..5 every load of the R x R child block is issued first (for
+// one KI, KJ a wave reads one child row, R columns apart, and the R values
+// of KI fill it in), then the sums run in that order; other R take the
+// loop below.
+// R child cells along I, read in one access (rows start on any float): a
+// quarter of the loads for R = 4.
+template <int R>
+struct __attribute__((aligned(4))) ChildRow {
+  float v[R];
+};
+template <int R>
+__device__ __forceinline__ float jnz_block(const DevNest &N, int i, int j) {
+  // 0-based first child cell: II = (I-IS) R + 1 + KI, KI = 1..R (1-based)
+  const int i0 = (i - N.is) * R + 1, j0 = (j - N.js) * R + 1;
+  const bool even = (N.rel_time % 2) == 0;
+  ChildRow<R> z2[R], hh[R], z1[R] = {};
+#pragma unroll
+  for (int kj = 0; kj < R; ++kj) {
+    const size_t cg = (size_t)(j0 + kj) * N.cnx + i0;
+    z2[kj] = *reinterpret_cast<const ChildRow<R> *>(N.cz2 + cg);
+    hh[kj] = *reinterpret_cast<const ChildRow<R> *>(N.ch + cg);
+    if (even) z1[kj] = *reinterpret_cast<const ChildRow<R> *>(N.cz1 + cg);
+  }
+  const float half = (float)(R * R) / 2.0f;
+  float sum = 0.0f, count = 0.0f;
+#pragma unroll
+  for (int ki = 0; ki < R; ++ki)
+#pragma unroll
+    for (int kj = 0; kj < R; ++kj)
+      if (hh[kj].v[ki] + z2[kj].v[ki] > kGx) {
+        if (even) sum = sum + 0.5f * (z1[kj].v[ki] + z2[kj].v[ki]);
+        else sum = sum + z2[kj].v[ki];
+        count = count + 1.0f;
+      }
+  return count > half ? sum / count : 0.0f;
+}
+
+// R: REL_SIZE where it is 2..5, 0: any other, -1: not known to the caller
+template <int R>
+__device__ __forceinline__ float jnz_value(const DevNest &N, int i, int j) {
+  if constexpr (R > 0) return jnz_block<R>(N, i, j);
+  const int ir = N.rel_size;
+  if constexpr (R < 0) {
+    switch (ir) {
+      case 2: return jnz_block<2>(N, i, j);
+      case 3: return jnz_block<3>(N, i, j);
+      case 4: return jnz_block<4>(N, i, j);
+      case 5: return jnz_block<5>(N, i, j);
+      default: break;
+    }
+  }
+  const float half = (float)(ir * ir) / 2.0f;
+  const int i0 = (i - N.is) * ir + 1, j0 = (j - N.js) * ir + 1;
+  const bool even = (N.rel_time % 2) == 0;
+  float sum = 0.0f, count = 0.0f;
+  for (int ki = 1; ki <= ir; ++ki) {
+    for (int kj = 1; kj <= ir; ++kj) {
+      const size_t cg = (size_t)(j0 + kj - 1) * N.cnx + (i0 + ki - 1);
+      const float z2 = N.cz2[cg];
+      if (N.ch[cg] + z2 > kGx) {
+        if (even) sum = sum + 0.5f * (N.cz1[cg] + z2);
+        else sum = sum + z2;
+        count = count + 1.0f;
+      }
+    }
+  }
+  return count > half ? sum / count : 0.0f;
+}
+
+template <int R>
+__device__ __forceinline__ void jnz_thread(const DevNest &N, int g) {
+  const int w = N.ie - N.is + 1, hgt = N.je - N.js + 1;
+  if (g >= w * hgt) return;
+  const int i = N.is + g % w, j = N.js + g / w;
+  N.pz2_out[(size_t)(j - 1) * N.pnx + (i - 1)] = jnz_value<R>(N, i, j);
+}
+
+template <int R>
+__global__ void __launch_bounds__(128) k_jnz(DevNest N) {
+  jnz_thread<R>(N, blockIdx.x * 128 + threadIdx.x);
+}
+
 // JNQ / NEWQ for one child (all_grids.f90:452-801): lanes over the four
 // interface lines, flattened to positions p = 0..jnq_threads-1: side 0/1 the
 // lines I = IS-1 / IE (M) with k = J from JS-2 to JE+2, side 2/3 the lines
@@ -1203,7 +1287,10 @@ __device__ __forceinline__ int jnq_threads(const DevNest &N) {
 constexpr int kJnqSpan = 62;
 constexpr int kJnqLoads = 5;  // child cells loaded ahead; larger REL_SIZEs read the rest later
 
-__device__ void jnq_wave(const DevNest &N, int w, int t) {
+// JNZ: the parent's elevation inside the footprint is still to be written; Z
+// is the view of that JNZ, R its REL_SIZE as in jnz_value.
+template <bool JNZ, int R>
+__device__ __forceinline__ void jnq_wave(const DevNest &N, int w, int t, const DevNest &Z) {
   const int lane = threadIdx.x & 63;
   const int lv = N.je - N.js + 5, lh = N.ie - N.is + 5;  // k ranges incl. +-2
   const int p = w * kJnqSpan + lane - 1;
@@ -1222,12 +1309,12 @@ __device__ void jnq_wave(const DevNest &N, int w, int t) {
   const int lo = vert ? N.js : N.is, hi = vert ? N.je : N.ie;
   const int fi = vert ? (side == 0 ? N.is - 1 : N.ie) : k;
   const int fj = vert ? k : (side == 2 ? N.js - 1 : N.je);
-  const int pnx = N.pnx, R = N.rel_size;
+  const int pnx = N.pnx, rs = N.rel_size;
   const size_t f = (size_t)(fj - 1) * pnx + (fi - 1);
   const size_t a = vert ? f + 1 : f + pnx;  // the other cell of the face
   // the line of child boundary cells that k feeds
   const bool own = in && lane >= 1 && lane <= kJnqSpan && k >= lo && k <= hi;
-  const int base = (k - lo) * R + 1;  // cells base + 1 .. base + R (1-based along the line)
+  const int base = (k - lo) * rs + 1;  // cells base + 1 .. base + R (1-based along the line)
   const size_t c0 = vert ? (size_t)base * N.cnx + (side == 0 ? 0 : N.cnx - 1)
                          : (size_t)(side == 2 ? 0 : N.cny - 1) * N.cnx + base;
   const size_t cs = vert ? N.cnx : 1;
@@ -1242,6 +1329,11 @@ __device__ void jnq_wave(const DevNest &N, int w, int t) {
     ha = N.ph[a];
     zf = N.pz2[f];
     za = N.pz2[a];
+    if (JNZ && in && k >= lo && k <= hi) {  // of the face's two cells, the one inside
+      const float z = jnz_value<R>(Z, vert ? (side == 0 ? N.is : N.ie) : k, vert ? k : (side == 2 ? N.js : N.je));
+      if (side == 0 || side == 2) za = z;
+      else zf = z;
+    }
     if (!forecast) {
       cached = vert ? N.yflux[(side & 1) * N.pny + (k - 1)] : N.xflux[(side & 1) * pnx + (k - 1)];
     } else if (N.p_sph) {
@@ -1259,7 +1351,7 @@ __device__ void jnq_wave(const DevNest &N, int w, int t) {
   float hc[kJnqLoads], zc[kJnqLoads];
 #pragma unroll
   for (int q = 0; q < kJnqLoads; ++q) {
-    const bool use = own && q < R;
+    const bool use = own && q < rs;
     hc[q] = use ? N.ch[c0 + q * cs] : 0.0f;
     zc[q] = use ? N.cz1[c0 + q * cs] : 0.0f;
   }
@@ -1301,17 +1393,17 @@ __device__ void jnq_wave(const DevNest &N, int w, int t) {
     const float fm = west(flux), fp = east(flux);
     const float fs = 0.5f * (fm + flux);
     const float fe = 0.5f * (fp + flux);
-    const float c1 = (fe - fs) / (float)(2 * R);  // == REAL((fe-fs)/DBLE(nn)), :538
+    const float c1 = (fe - fs) / (float)(2 * rs);  // == REAL((fe-fs)/DBLE(nn)), :538
     const float c2 = -c1 + fs;
     if (u > t) {  // a later sub-step: before the wet test
       if (own)
-        for (int q = 0; q < R; ++q) ef[q] = 2.0f * (float)(q + 1) * c1 + c2;
+        for (int q = 0; q < rs; ++q) ef[q] = 2.0f * (float)(q + 1) * c1 + c2;
       ef += edge_floats(N.cnx, N.cny);
     } else if (own) {
 #pragma unroll
       for (int q = 0; q < kJnqLoads; ++q)
-        if (q < R) cf[c0 + q * cs] = hc[q] + zc[q] <= kGx ? 0.0f : 2.0f * (float)(q + 1) * c1 + c2;
-      for (int q = kJnqLoads; q < R; ++q)
+        if (q < rs) cf[c0 + q * cs] = hc[q] + zc[q] <= kGx ? 0.0f : 2.0f * (float)(q + 1) * c1 + c2;
+      for (int q = kJnqLoads; q < rs; ++q)
         cf[c0 + q * cs] =
             N.ch[c0 + q * cs] + N.cz1[c0 + q * cs] <= kGx ? 0.0f : 2.0f * (float)(q + 1) * c1 + c2;
     }
@@ -1319,75 +1411,23 @@ __device__ void jnq_wave(const DevNest &N, int w, int t) {
 }
 
 __global__ void __launch_bounds__(128) k_jnq(DevNest N, int t) {
-  jnq_wave(N, blockIdx.x * 2 + (threadIdx.x >> 6), t);
+  jnq_wave<false, 0>(N, blockIdx.x * 2 + (threadIdx.x >> 6), t, N);
 }
 
-// JNZ (all_grids.f90:342-421): parent Z2 over the footprint = mean of the
-// wet child cells, summed in the Fortran order (KI outer, KJ inner).
-// For R = 2..5 every load of the R x R child block is issued first (for
-// one KI, KJ a wave reads one child row, R columns apart, and the R values
-// of KI fill it in), then the sums run in that order; other R take the
-// loop below.
+// JNZ and the JNQ/NEWQ that follows it, sub-step t: the first nq blocks make
+// the interface fluxes, with the parent's elevation inside the footprint from
+// the child (JNZ's own sum, so the same bits) instead of from the cells that
+// the other blocks are writing.  Two launches before, us: 512x384 + 401x401
+// 3.65 + 4.4, now 5.3; 2048x1536 + 1801x1801 11.8 + 5.3, now 10.6 (the child's
+// three planes, 39 MB, take 8 at the rate of a copy).  One instance per
+// REL_SIZE: with all of them in one kernel every lane has the registers of the
+// largest, 8.3 and 18.5 us.
 template <int R>
-__device__ __forceinline__ void jnz_block(const DevNest &N, int i, int j) {
-  // 0-based first child cell: II = (I-IS) R + 1 + KI, KI = 1..R (1-based)
-  const int i0 = (i - N.is) * R + 1, j0 = (j - N.js) * R + 1;
-  const bool even = (N.rel_time % 2) == 0;
-  float z2[R][R], hh[R][R], z1[R][R];
-#pragma unroll
-  for (int kj = 0; kj < R; ++kj)
-#pragma unroll
-    for (int ki = 0; ki < R; ++ki) {
-      const size_t cg = (size_t)(j0 + kj) * N.cnx + (i0 + ki);
-      z2[ki][kj] = N.cz2[cg];
-      hh[ki][kj] = N.ch[cg];
-      z1[ki][kj] = even ? N.cz1[cg] : 0.0f;
-    }
-  const float half = (float)(R * R) / 2.0f;
-  float sum = 0.0f, count = 0.0f;
-#pragma unroll
-  for (int ki = 0; ki < R; ++ki)
-#pragma unroll
-    for (int kj = 0; kj < R; ++kj)
-      if (hh[ki][kj] + z2[ki][kj] > kGx) {
-        if (even) sum = sum + 0.5f * (z1[ki][kj] + z2[ki][kj]);
-        else sum = sum + z2[ki][kj];
-        count = count + 1.0f;
-      }
-  N.pz2_out[(size_t)(j - 1) * N.pnx + (i - 1)] = count > half ? sum / count : 0.0f;
+__global__ void __launch_bounds__(128) k_jnz_jnq(DevNest N, DevNest Q, int t, int nq) {
+  const int b = blockIdx.x;
+  if (b < nq) jnq_wave<true, R>(Q, b * 2 + (threadIdx.x >> 6), t, N);
+  else jnz_thread<R>(N, (b - nq) * 128 + threadIdx.x);
 }
-
-__device__ void jnz_thread(const DevNest &N, int g) {
-  const int w = N.ie - N.is + 1, hgt = N.je - N.js + 1;
-  if (g >= w * hgt) return;
-  const int i = N.is + g % w, j = N.js + g / w;
-  const int ir = N.rel_size;
-  switch (ir) {
-    case 2: jnz_block<2>(N, i, j); return;
-    case 3: jnz_block<3>(N, i, j); return;
-    case 4: jnz_block<4>(N, i, j); return;
-    case 5: jnz_block<5>(N, i, j); return;
-    default: break;
-  }
-  const float half = (float)(ir * ir) / 2.0f;
-  const int i0 = (i - N.is) * ir + 1, j0 = (j - N.js) * ir + 1;
-  const bool even = (N.rel_time % 2) == 0;
-  float sum = 0.0f, count = 0.0f;
-  for (int ki = 1; ki <= ir; ++ki) {
-    for (int kj = 1; kj <= ir; ++kj) {
-      const size_t cg = (size_t)(j0 + kj - 1) * N.cnx + (i0 + ki - 1);
-      const float z2 = N.cz2[cg];
-      if (N.ch[cg] + z2 > kGx) {
-        if (even) sum = sum + 0.5f * (N.cz1[cg] + z2);
-        else sum = sum + z2;
-        count = count + 1.0f;
-      }
-    }
-  }
-  N.pz2_out[(size_t)(j - 1) * N.pnx + (i - 1)] = count > half ? sum / count : 0.0f;
-}
-
-__global__ void k_jnz(DevNest N) { jnz_thread(N, blockIdx.x * blockDim.x + threadIdx.x); }
 
 // ------------------------------------------------------------ batch forms
 // Several nests in one launch: nest n owns blocks [start[n], start[n+1]).
@@ -1404,14 +1444,14 @@ __global__ void __launch_bounds__(128) k_jnq_multi(const DevNest *__restrict__ n
                                                    const int *__restrict__ start, int nnest, int t) {
   const int n = __builtin_amdgcn_readfirstlane(nest_of_block(start, nnest));
   const DevNest N = nests[n];
-  jnq_wave(N, (blockIdx.x - start[n]) * 2 + (threadIdx.x >> 6), t);
+  jnq_wave<false, 0>(N, (blockIdx.x - start[n]) * 2 + (threadIdx.x >> 6), t, N);
 }
 
 __global__ void k_jnz_multi(const DevNest *__restrict__ nests, const int *__restrict__ start,
                             int nnest) {
   const int n = __builtin_amdgcn_readfirstlane(nest_of_block(start, nnest));
   const DevNest N = nests[n];
-  jnz_thread(N, (blockIdx.x - start[n]) * blockDim.x + threadIdx.x);
+  jnz_thread<-1>(N, (blockIdx.x - start[n]) * blockDim.x + threadIdx.x);
 }
 
 // Streaming copy, the reference for HBM bandwidth and for scaling the
@@ -1927,10 +1967,42 @@ __global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(W
   tile_step<kFused, true, SPH, TX, TY, ST, true>(L, t, tiles_x, sm, &stab);
 }
 
+// The same beside the linear root's momentum + next continuity (DevLayer::
+// beside): 10.4 us where 401x401 tiles and a 512x384 root took 7.4 + 4.9.
+template <bool SPH, int WAVES, bool ST>
+__global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(WAVES)))
+    k_step_small_beside(DevLayer L, int tiles_x, int ntiles, int per_xcd, DevLayer R, MarchGrid RG, Beside B) {
+  constexpr int TX = 32, TY = 8;
+  static_assert(kThreads == kMarchBlock, "one workgroup size for both");
+  __shared__ float sm[6 * (TX + 4) * (TY + 4) + kNumCoef * (TY + 4)];
+  __shared__ gcdet::Tables stab;
+  const int b = beside_block(B, blockIdx.x);
+  if (b < 0) {
+    march_mm_block<true, ST>(R, RG, -1 - b);
+    return;
+  }
+  const int t = (b & 7) * per_xcd + (b >> 3);
+  if (t >= ntiles) return;
+  tile_step<kFused, true, SPH, TX, TY, ST, true>(L, t, tiles_x, sm, &stab);
+}
+
 template <bool SPH, int WAVES>
 hipError_t launch_small(const DevLayer &L, hipStream_t st) {
   const int tx = (L.nx + 31) / 32, ty = (L.ny + 7) / 8;
   const int nt = tx * ty, per = (nt + 7) / 8;
+  if (L.beside) {
+    MarchGrid RG;
+    const long long rblocks = mm_grid(*L.beside, RG);
+    if (8LL * per + rblocks > 0x7ffffff0) return hipErrorInvalidValue;
+    const Beside B = beside_split(8LL * per, rblocks);
+    if (L.stream_out)
+      hipLaunchKernelGGL((k_step_small_beside<SPH, WAVES, true>), dim3(B.total()), dim3(kThreads), 0, st, L,
+                         tx, nt, per, *L.beside, RG, B);
+    else
+      hipLaunchKernelGGL((k_step_small_beside<SPH, WAVES, false>), dim3(B.total()), dim3(kThreads), 0, st, L,
+                         tx, nt, per, *L.beside, RG, B);
+    return hipGetLastError();
+  }
   if (L.stream_out)
     hipLaunchKernelGGL((k_step_small<SPH, WAVES, true>), dim3(8 * per), dim3(kThreads), 0, st, L, tx, nt, per);
   else
@@ -1996,24 +2068,53 @@ void tile_variant_shape(int v, int *tx, int *ty) {
   *ty = kVariants[v][2];
 }
 
-hipError_t launch_step(const DevLayer &L, int mode, bool nl, bool sph, int variant,
-                       hipStream_t st) {
-  if (variant < 0 || variant >= num_tile_variants()) return hipErrorInvalidValue;
-  if (mode == kFused && kVariants[variant][0] == 0 && !(nl && march_nl_applies(L, sph))) variant = 0;
-  if (mode == kFused && nl && march_nl_applies(L, sph)) {
+// The form of a nonlinear layer's fused step: rows per segment of the marching
+// strips, 0 for 32x8 tiles, -1 for the variant's tiles.
+static int nl_form(const DevLayer &L, bool sph, int variant) {
+  if (march_nl_applies(L, sph)) {
     const int seg = kVariants[variant][0] == 0 ? kVariants[variant][2]
                     : variant == 0             ? march_nl_seg(L.nx, L.ny)
                                                : 0;
-    if (seg > 0) return launch_march_nl(L, sph, seg, st);
+    if (seg > 0) return seg;
+  } else if (kVariants[variant][0] == 0) {
+    variant = 0;
   }
-  // Measured, us per step (64x8 tiles; 32x8 with 4 and 8 waves per SIMD):
-  // 96x72 13.9; 9.4, 9.9.  517x391 14.4; 10.9, 11.3.  512x384 + 401x401 nest
-  // 84.9; 67.2, 67.9.  1024x768 21.0; 18.95, 18.3.  1201x901 24.5; 23.2, 22.8.
-  if (mode == kFused && nl && variant == 0 && (long long)L.nx * L.ny <= kSmallCells) {
-    const bool few = (long long)L.nx * L.ny <= kSmallCells / 3;
-    if (sph) return few ? launch_small<true, 4>(L, st) : launch_small<true, 8>(L, st);
-    return few ? launch_small<false, 4>(L, st) : launch_small<false, 8>(L, st);
+  return variant == 0 && (long long)L.nx * L.ny <= kSmallCells ? 0 : -1;
+}
+
+// Measured, us per step (64x8 tiles; 32x8 with 4 and 8 waves per SIMD):
+// 96x72 13.9; 9.4, 9.9.  517x391 14.4; 10.9, 11.3.  512x384 + 401x401 nest
+// 84.9; 67.2, 67.9.  1024x768 21.0; 18.95, 18.3.  1201x901 24.5; 23.2, 22.8.
+static hipError_t launch_small(const DevLayer &L, bool sph, hipStream_t st) {
+  const bool few = (long long)L.nx * L.ny <= kSmallCells / 3;
+  if (sph) return few ? launch_small<true, 4>(L, st) : launch_small<true, 8>(L, st);
+  return few ? launch_small<false, 4>(L, st) : launch_small<false, 8>(L, st);
+}
+
+// A nested layer's fused step with its root's momentum + next continuity: one
+// launch where the step is one of 32x8 tiles, which leaves the chip half idle,
+// else one after the other (a marching step of a large child fills it: 1801x1801
+// beside a 2048x1536 root takes 59.2 us in one launch, 33.3 + 20.6 in two).
+static hipError_t launch_beside(const DevLayer &L, bool nl, bool sph, int variant, hipStream_t st) {
+  const DevLayer &R = *L.beside;
+  const int form = nl && L.zmax && R.zmax && march_applies(R) ? nl_form(L, sph, variant) : -1;
+  if (form == 0) return launch_small(L, sph, st);
+  DevLayer C = L;
+  C.beside = nullptr;
+  const hipError_t e = launch_step(C, kFused, nl, sph, variant, st);
+  return e != hipSuccess ? e : launch_step(R, kMomentMass, false, R.rowc != nullptr, variant, st);
+}
+
+hipError_t launch_step(const DevLayer &L, int mode, bool nl, bool sph, int variant,
+                       hipStream_t st) {
+  if (variant < 0 || variant >= num_tile_variants()) return hipErrorInvalidValue;
+  if (mode == kFused && L.beside) return launch_beside(L, nl, sph, variant, st);
+  if (mode == kFused && nl) {
+    const int form = nl_form(L, sph, variant);
+    if (form > 0) return launch_march_nl(L, sph, form, st);
+    if (form == 0) return launch_small(L, sph, st);
   }
+  if (mode == kFused && kVariants[variant][0] == 0) variant = 0;
   if (mode == kMomentMass) {  // outermost linear layers with nested layers
     if (nl) return hipErrorInvalidValue;
     if (sph && march_applies(L)) return launch_march_moment_mass(L, st);
@@ -2096,10 +2197,32 @@ hipError_t launch_jnq(const DevNest &N, int t, hipStream_t st) {
   return hipGetLastError();
 }
 
-hipError_t launch_jnz(const DevNest &N, hipStream_t st) {
-  const int total = (N.ie - N.is + 1) * (N.je - N.js + 1);
-  hipLaunchKernelGGL(k_jnz, dim3((total + 127) / 128), dim3(128), 0, st, N);
+template <int R>
+static hipError_t launch_jnz_r(const DevNest &N, hipStream_t st) {
+  const int nz = ((N.ie - N.is + 1) * (N.je - N.js + 1) + 127) / 128;
+  if (N.next_t == 0) {
+    hipLaunchKernelGGL(k_jnz<R>, dim3(nz), dim3(128), 0, st, N);
+    return hipGetLastError();
+  }
+  if (N.next_t < 3) return hipErrorInvalidValue;  // the forecast of sub-step 2 would read the footprint too
+  DevNest Q = N;
+  Q.cz1 = N.cz2;
+  Q.cz2 = N.cz1;
+  Q.cm1 = N.cm2;
+  Q.cn1 = N.cn2;
+  const int nq = jnq_block_count(N);
+  hipLaunchKernelGGL(k_jnz_jnq<R>, dim3(nq + nz), dim3(128), 0, st, N, Q, N.next_t, nq);
   return hipGetLastError();
+}
+
+hipError_t launch_jnz(const DevNest &N, hipStream_t st) {
+  switch (N.rel_size) {
+    case 2: return launch_jnz_r<2>(N, st);
+    case 3: return launch_jnz_r<3>(N, st);
+    case 4: return launch_jnz_r<4>(N, st);
+    case 5: return launch_jnz_r<5>(N, st);
+    default: return launch_jnz_r<0>(N, st);
+  }
 }
 
 // ------------------------------------------------------------ batch launchers

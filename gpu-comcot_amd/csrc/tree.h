@@ -160,8 +160,11 @@ DevSc sc_view(const Tree &T, const LayerRec &P, const LayerRec &C);
 // One layer pass (kFused / kMassOnly / kMomentOnly) on stream st.
 int tree_launch(const Tree &T, const LayerRec &L, int mode, bool with_max, bool advance,
                 hipStream_t st);
-// Sub-steps of every child of P for one step of P (ALL_GRID order).
-int tree_enqueue_children(Tree &T, LayerRec &P, bool with_max, hipStream_t st);
+// Sub-steps of every child of P for one step of P (ALL_GRID order).  beside:
+// the view of P's momentum + next continuity, run beside a sub-step of the last
+// child that follows JNZ if there is one, and *beside is then null.
+int tree_enqueue_children(Tree &T, LayerRec &P, bool with_max, hipStream_t st,
+                          const DevLayer **beside = nullptr);
 // One complete root step: mass+open, nests, momentum + max, rotation.
 // next: another root step follows at once (its continuity may then ride in
 // this step's momentum launch, tree_fuses_halves).
@@ -185,8 +188,6 @@ int tree_enqueue_gauges(const Tree &T, hipStream_t st);
 // restore into a tree built with the same layers.
 int tree_checkpoint_save(const Tree &T, hipStream_t st, const char *path, long long done);
 int tree_checkpoint_load(Tree &T, hipStream_t st, const char *path, long long *done);
-
-long long tree_launches_per_step(Tree &T);
 
 // R2/R4 of the reference ABI as a row factor of max(HP,0) (PARA,
 // comcot.f90:733-744); false when no factor reproduces the row exactly.

@@ -424,9 +424,12 @@ DevSc sc_view(const Tree &T, const LayerRec &P, const LayerRec &C) {
   return S;
 }
 
-int tree_enqueue_children(Tree &T, LayerRec &P, bool with_max, hipStream_t st) {
+int tree_enqueue_children(Tree &T, LayerRec &P, bool with_max, hipStream_t st, const DevLayer **beside) {
   for (int cid : P.children) {
     LayerRec &C = T.layers[cid];
+    // what is left of the last child's sub-steps after JNZ does not write the
+    // parent's planes, nor read those that its next step writes
+    const bool may_pair = beside && cid == P.children.back() && C.children.empty() && !C.sc;
     const int nhalf = (int)std::floor(C.rel_time / 2.0f) + 1;
     int k0 = 0, ahead = 0;  // the last JNQ covers sub-steps k0 .. k0 + ahead
     for (int k = 1; k <= C.rel_time; ++k) {
@@ -441,14 +444,30 @@ int tree_enqueue_children(Tree &T, LayerRec &P, bool with_max, hipStream_t st) {
       }
       if (e != hipSuccess) return fail(201, "jnq launch failed: %s", hipGetErrorString(e));
       if (C.children.empty()) {
-        if (int r = launch_view(T, C, substep_view(T, C, with_max, k, k0, ahead), kFused, st)) return r;
+        DevLayer d = substep_view(T, C, with_max, k, k0, ahead);
+        if (may_pair && k > nhalf) {
+          d.beside = *beside;
+          *beside = nullptr;
+        }
+        if (int r = launch_view(T, C, d, kFused, st)) return r;
       } else {
         if (int r = tree_launch(T, C, kMassOnly, false, false, st)) return r;
         if (int r = tree_enqueue_children(T, C, with_max, st)) return r;
         if (int r = tree_launch(T, C, kMomentOnly, with_max, false, st)) return r;
       }
       if (k == nhalf) {
-        e = C.sc ? launch_sc_jnz(sc_view(T, P, C), st) : launch_jnz(nest_view(P, C), st);
+        if (C.sc) {
+          e = launch_sc_jnz(sc_view(T, P, C), st);
+        } else {
+          DevNest q = nest_view(P, C);
+          if (k < C.rel_time) {  // with the JNQ of the next sub-step
+            k0 = q.next_t = k + 1;
+            q.ahead = ahead = jnq_ahead(C, k + 1);
+            q.cm2 = C.m[1 - C.cur];
+            q.cn2 = C.n[1 - C.cur];
+          }
+          e = launch_jnz(q, st);
+        }
         if (e != hipSuccess) return fail(202, "jnz launch failed: %s", hipGetErrorString(e));
       }
       C.cur = 1 - C.cur;  // UPDATE
@@ -480,10 +499,11 @@ int tree_enqueue_root_step(Tree &T, hipStream_t st, bool next) {
     if (!T.mass_ahead)
       if (int r = tree_launch(T, *R, kMassOnly, false, false, st)) return r;
     T.mass_ahead = false;
-    if (int r = tree_enqueue_children(T, *R, true, st)) return r;
-    if (next && tree_fuses_halves(T)) {
-      const DevLayer d = fused_halves_view(T, *R);
-      hipError_t e = launch_step(d, kMomentMass, false, R->sph != 0, T.variant, st);
+    const bool fuse = next && tree_fuses_halves(T);
+    const DevLayer d = fuse ? fused_halves_view(T, *R) : DevLayer{}, *left = fuse ? &d : nullptr;
+    if (int r = tree_enqueue_children(T, *R, true, st, &left)) return r;
+    if (fuse) {
+      hipError_t e = left ? launch_step(d, kMomentMass, false, R->sph != 0, T.variant, st) : hipSuccess;
       if (e != hipSuccess)
         return fail(200 + (int)e, "step kernel launch failed: %s", hipGetErrorString(e));
       T.mass_ahead = true;
@@ -576,23 +596,6 @@ int tree_enqueue_root_steps2(Tree &T, hipStream_t st) {
   R->cur = 1 - R->cur;
   T.ctl_in = 1 - T.ctl_in;
   return 0;
-}
-
-static long long launches_below(Tree &T, const LayerRec &P) {
-  long long n = 0;
-  for (int cid : P.children) {
-    const LayerRec &C = T.layers[cid];
-    const long long inner = C.children.empty() ? 1 : 2 + launches_below(T, C);
-    // JNQ (SC: bands and edges) + step(s) per sub-step, one JNZ
-    n += (long long)C.rel_time * ((C.sc ? 2 : 1) + inner) + 1;
-  }
-  return n;
-}
-
-long long tree_launches_per_step(Tree &T) {
-  LayerRec *R = T.layer(1);
-  if (!R) return 0;
-  return R->children.empty() ? 1 : 2 + launches_below(T, *R);
 }
 
 bool row_factor(const float *R, const float *H, int nx, int ny, int j, bool is_x, float *F) {

@@ -184,3 +184,29 @@ def test_marched_moment_mass_matches_oracle(nx, ny):
             compare_device_oracle(sc, dev, orc, f"moment + mass {nx}x{ny} after {n}")
     finally:
         dev.close()
+
+
+@pytest.mark.parametrize("clc", [0, 1], ids=["sph-child", "cart-child"])
+@pytest.mark.parametrize("nx,ny,foot,rt", [(331, 290, (9, 8), 3), (70, 64, (45, 41), 4), (131, 97, (40, 33), 6)],
+                         ids=["wide-root", "wide-child", "even"])
+def test_root_beside_child_matches_oracle(nx, ny, foot, rt, clc):
+    """The root's momentum + next continuity in one launch with a step of its
+    child, where either side has more workgroups than the other (one-cell tiles),
+    or one after the other (marching strips); and the JNQ made with its JNZ."""
+    from gcomcot._lib import ip, lib
+    from helpers import BEACH
+    sc = S.custom(nx=nx, ny=ny, laygov=0, child=dict(laycord=clc, laygov=1, footprint=foot, rel_size=3,
+                                                     rel_time=rt, corner=(8, 14)), **BEACH)
+    orc = Oracle(sc, 32, pow_mode=1)
+    orc.step(24)
+    try:
+        for v in (0, 9):
+            print(f"[gpu] root beside child {nx}x{ny} {foot} {clc} variant {v}", flush=True)
+            assert lib().gcomcot_set_tile_variant_(ip(v)) == 0
+            dev = DeviceRun(sc)
+            dev.run(23)
+            dev.run(1)
+            compare_device_oracle(sc, dev, orc, f"root beside child {nx}x{ny} variant {v}")
+            dev.close()
+    finally:
+        lib().gcomcot_set_tile_variant_(ip(0))
