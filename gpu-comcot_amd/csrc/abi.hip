@@ -474,11 +474,11 @@ static int run_plain(int n) {
     for (; n >= 2; n -= 2)
       if (int r = tree_enqueue_root_steps2(g_tree, g_stream)) return r;
   // a linear root with nested layers: every root step but the last computes
-  // the next one's continuity in its momentum launch
-  g_tree.mass_ahead = false;
-  const bool ahead = tree_fuses_halves(g_tree);
+  // the next one's continuity in its momentum launch; gauges of a single layer
+  // are sampled by the next step
+  g_tree.mass_ahead = g_tree.gauges_due = false;
   for (; n > 0; --n)
-    if (int r = tree_enqueue_root_step(g_tree, g_stream, ahead && n > 1)) return r;
+    if (int r = tree_enqueue_root_step(g_tree, g_stream, n > 1)) return r;
   return sync();
 }
 
@@ -730,7 +730,7 @@ int gcomcot_time_steps_(int *nsteps, float *ms_total, float *ms_each) {
   std::vector<hipEvent_t> ev(n + 1);
   for (auto &e : ev) HIPCHK(hipEventCreate(&e));
   HIPCHK(hipEventRecord(ev[0], g_stream));
-  g_tree.mass_ahead = false;
+  g_tree.mass_ahead = g_tree.gauges_due = false;
   for (int k = 0; k < n; ++k) {
     if (int r = tree_enqueue_root_step(g_tree, g_stream, k + 1 < n)) return r;
     HIPCHK(hipEventRecord(ev[k + 1], g_stream));

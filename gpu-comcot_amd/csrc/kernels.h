@@ -6,6 +6,8 @@
 
 namespace gc {
 
+struct GaugeDev;
+
 // What one step kernel needs of a layer.  Planes are column-major NX*NY
 // float (index (J-1)*NX + I-1), time level 1 (in) and 2 (out) bound per
 // launch from the layer's current parity.
@@ -56,6 +58,12 @@ struct DevLayer {
   // whose momentum + next continuity (kMomentMass) launch_step runs beside the
   // step, in the same launch where that is faster.
   const DevLayer *beside;
+  // ngauge > 0, the fused step of an outermost layer without nested ones: the
+  // launch also samples these gauges of the step before, from z1, into
+  // gauge_ring (launch_gauges' layout)
+  const GaugeDev *gauges;
+  float *gauge_ring;
+  int ngauge, gauge_cap;
 };
 // Slot layout: M of rows 1..NY at column 1 and at column NX, then N of
 // columns 1..NX at row 1 and at row NY.

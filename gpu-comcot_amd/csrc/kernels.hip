@@ -979,7 +979,9 @@ __global__ void __launch_bounds__(kThreads)
     k_step(DevLayer L, int tiles_x, int ntiles, int per_xcd) {
   __shared__ float sm[6 * (TX + 4) * (TY + 4) + kNumCoef * (TY + 4)];
   __shared__ gcdet::Tables stab;
-  const int t = tile_of_block(per_xcd);
+  const int b = MODE == kFused ? step_block(L) : (int)blockIdx.x;
+  if (b < 0) return;
+  const int t = (b & 7) * per_xcd + (b >> 3);
   if (t >= ntiles) return;
   tile_step<MODE, NL, SPH, TX, TY, ST, NL || !SPH>(L, t, tiles_x, sm, &stab);
 }
@@ -1185,12 +1187,9 @@ __global__ void k_max(DevLayer L, float *zmax_raw) {
 // ---------------------------------------------------------------- nesting
 // JNZ (all_grids.f90:342-421): parent Z2 over the footprint = mean of the
 // wet child cells, summed in the Fortran order (KI outer, KJ inner).
-// For R = 2..5 every load of the R x R child block is issued first (for
-// one KI, KJ a wave reads one child row, R columns apart, and the R values
-// of KI fill it in), then the sums run in that order; other R take the
-// loop below.
-// R child cells along I, read in one access (rows start on any float): a
-// quarter of the loads for R = 4.
+// For R = 2..5 every load of the R x R child block is issued first, a row of
+// R cells along I in one access (they start on any float), then the sums run
+// in that order; other R take the loop below.
 template <int R>
 struct __attribute__((aligned(4))) ChildRow {
   float v[R];
@@ -1833,22 +1832,14 @@ __global__ void __launch_bounds__(256) k_apply_deform(float *z1, float *h,
   if (zraw) zraw[g] = z;
 }
 
-// Gauge samples (GET_TS, output.f90:1085-1094): the 2x2 stencil of the
-// current elevation weighted in the Fortran's operation order.
+// Gauge samples of every layer (a single layer's are made by its next step,
+// gauge_block).
 __global__ void k_gauges(const GaugeDev *__restrict__ gs, int n, ZNow zs,
                          const int *__restrict__ step_now, float *ring, int cap) {
   const int k = blockIdx.x * blockDim.x + threadIdx.x;
   if (k >= n) return;
   const GaugeDev G = gs[k];
-  const float *z = zs.z[G.lid];
-  const size_t o = (size_t)(G.kj - 1) * G.nx + (G.ki - 1);
-  const float l1 = z[o], l2 = z[o + 1], l3 = z[o + G.nx], l4 = z[o + G.nx + 1];
-  const float z1 = l1 * (1.0f - G.cx) * (1.0f - G.cy);
-  const float z2 = l2 * G.cx * (1.0f - G.cy);
-  const float z3 = l3 * (1.0f - G.cx) * G.cy;
-  const float z4 = l4 * G.cx * G.cy;
-  float dat = z1 + z2 + z3 + z4;
-  if (fabsf(G.tide) > kGx) dat = dat + G.tide;
+  const float dat = gauge_sample(G, zs.z[G.lid]);
   const int step = *step_now;
   ring[(size_t)k * cap + (step - 1) % cap] = dat;
 }
@@ -1962,7 +1953,9 @@ __global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(W
   constexpr int TX = 32, TY = 8;
   __shared__ float sm[6 * (TX + 4) * (TY + 4) + kNumCoef * (TY + 4)];
   __shared__ gcdet::Tables stab;
-  const int t = tile_of_block(per_xcd);
+  const int b = step_block(L);
+  if (b < 0) return;
+  const int t = (b & 7) * per_xcd + (b >> 3);
   if (t >= ntiles) return;
   tile_step<kFused, true, SPH, TX, TY, ST, true>(L, t, tiles_x, sm, &stab);
 }
@@ -2004,22 +1997,24 @@ hipError_t launch_small(const DevLayer &L, hipStream_t st) {
     return hipGetLastError();
   }
   if (L.stream_out)
-    hipLaunchKernelGGL((k_step_small<SPH, WAVES, true>), dim3(8 * per), dim3(kThreads), 0, st, L, tx, nt, per);
+    hipLaunchKernelGGL((k_step_small<SPH, WAVES, true>), dim3(8 * per + gauge_blocks(L)), dim3(kThreads), 0, st,
+                       L, tx, nt, per);
   else
-    hipLaunchKernelGGL((k_step_small<SPH, WAVES, false>), dim3(8 * per), dim3(kThreads), 0, st, L, tx, nt, per);
+    hipLaunchKernelGGL((k_step_small<SPH, WAVES, false>), dim3(8 * per + gauge_blocks(L)), dim3(kThreads), 0, st,
+                       L, tx, nt, per);
   return hipGetLastError();
 }
 
 template <int MODE, bool NL, bool SPH, int TX, int TY>
 hipError_t launch_t(const DevLayer &L, hipStream_t st) {
   const int tx = (L.nx + TX - 1) / TX, ty = (L.ny + TY - 1) / TY;
-  const int nt = tx * ty, per = (nt + 7) / 8;
+  const int nt = tx * ty, per = (nt + 7) / 8, grid = 8 * per + (MODE == kFused ? gauge_blocks(L) : 0);
   if (L.stream_out)
-    hipLaunchKernelGGL((k_step<MODE, NL, SPH, TX, TY, true>), dim3(8 * per), dim3(kThreads), 0,
-                       st, L, tx, nt, per);
+    hipLaunchKernelGGL((k_step<MODE, NL, SPH, TX, TY, true>), dim3(grid), dim3(kThreads), 0, st, L,
+                       tx, nt, per);
   else
-    hipLaunchKernelGGL((k_step<MODE, NL, SPH, TX, TY, false>), dim3(8 * per), dim3(kThreads), 0,
-                       st, L, tx, nt, per);
+    hipLaunchKernelGGL((k_step<MODE, NL, SPH, TX, TY, false>), dim3(grid), dim3(kThreads), 0, st, L,
+                       tx, nt, per);
   return hipGetLastError();
 }
 

@@ -82,4 +82,35 @@ __device__ __forceinline__ float radiate(float h, float cc, float a, float b, bo
   return h > kGx ? zz : 0.0f;
 }
 
+// Gauge sample (GET_TS, output.f90:1085-1094): the 2x2 stencil of the
+// elevation weighted in the Fortran's operation order.
+__device__ __forceinline__ float gauge_sample(const GaugeDev &G, const float *z) {
+  const size_t o = (size_t)(G.kj - 1) * G.nx + (G.ki - 1);
+  const float l1 = z[o], l2 = z[o + 1], l3 = z[o + G.nx], l4 = z[o + G.nx + 1];
+  const float z1 = l1 * (1.0f - G.cx) * (1.0f - G.cy);
+  const float z2 = l2 * G.cx * (1.0f - G.cy);
+  const float z3 = l3 * (1.0f - G.cx) * G.cy;
+  const float z4 = l4 * G.cx * G.cy;
+  float dat = z1 + z2 + z3 + z4;
+  if (fabsf(G.tide) > kGx) dat = dat + G.tide;
+  return dat;
+}
+
+// The gauges of the step before ride in a step's launch (DevLayer::gauges; a
+// launch of their own takes 4.5 us a step): workgroup 0 samples them, first,
+// so that its chain of loads ends with the tiles', and seven idle ones keep
+// the others on their XCDs.  step_block: this workgroup's number among the
+// step's own, -1 for those eight.
+inline int gauge_blocks(const DevLayer &L) { return L.ngauge > 0 ? 8 : 0; }
+__device__ __forceinline__ int step_block(const DevLayer &L) {
+  const int b = blockIdx.x;
+  if (L.ngauge == 0) return b;
+  if (b == 0) {
+    const int step = L.ctl[L.ctl_in];
+    for (int k = threadIdx.x; k < L.ngauge; k += blockDim.x)
+      L.gauge_ring[(size_t)k * L.gauge_cap + (step - 1) % L.gauge_cap] = gauge_sample(L.gauges[k], L.z1);
+  }
+  return b < 8 ? -1 : b - 8;
+}
+
 }  // namespace gc

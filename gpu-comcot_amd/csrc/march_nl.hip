@@ -432,15 +432,17 @@ template <bool SPH, bool MX, bool ST>
 __global__ void __launch_bounds__(kMarchBlock) k_march_nl(DevLayer L, NlGrid G) {
   constexpr int WB = kMarchBlock / kWave;
   __shared__ gcdet::Tables tab;
+  const int g = step_block(L);
+  if (g < 0) return;
   stage(tab);
   int step = 0;
   if (MX) {
     step = L.ctl[L.ctl_in] + 1;
-    if (L.advance && blockIdx.x == 0 && threadIdx.x == 0) L.ctl[1 - L.ctl_in] = step;
+    if (L.advance && g == 0 && threadIdx.x == 0) L.ctl[1 - L.ctl_in] = step;
   }
   Strip S;
-  if ((int)blockIdx.x < G.first_blocks) {
-    const int w = __builtin_amdgcn_readfirstlane(blockIdx.x * WB + (threadIdx.x >> 6));
+  if (g < G.first_blocks) {
+    const int w = __builtin_amdgcn_readfirstlane(g * WB + (threadIdx.x >> 6));
     if (!nl_first(G, L.ny, w, S)) return;
     if (S.j0 > kNlEnd && S.j1 <= L.ny - kNlEnd)
       march_nl<SPH, true, false, MX, ST>(L, S, step, tab);
@@ -448,7 +450,7 @@ __global__ void __launch_bounds__(kMarchBlock) k_march_nl(DevLayer L, NlGrid G) 
       march_nl<SPH, true, true, MX, ST>(L, S, step, tab);
     return;
   }
-  const int b = blockIdx.x - G.first_blocks, mid = G.east - 1;
+  const int b = g - G.first_blocks, mid = G.east - 1;
   const int w = __builtin_amdgcn_readfirstlane(((b & 7) * G.per_xcd + (b >> 3)) * WB + (threadIdx.x >> 6));
   if (w >= mid * G.nseg) return;
   S.c0 = (1 + w % mid) * kNlWidth + 1;
@@ -475,7 +477,7 @@ hipError_t launch_nl(const DevLayer &L, int seg, hipStream_t st) {
   const long long mid = (long long)(G.east - 1) * G.nseg;
   G.first_blocks = (int)((first + WB - 1) / WB);
   G.per_xcd = (int)((mid + 8 * WB - 1) / (8 * WB));
-  const long long blocks = (long long)G.first_blocks + 8LL * G.per_xcd;
+  const long long blocks = (long long)G.first_blocks + 8LL * G.per_xcd + gauge_blocks(L);
   if (blocks > 0x7fffffff) return hipErrorInvalidValue;
   hipLaunchKernelGGL((k_march_nl<SPH, MX, ST>), dim3((unsigned)blocks), dim3(kMarchBlock), 0, st, L, G);
   return hipGetLastError();

@@ -68,6 +68,7 @@ struct Tree {
   GaugeDev *gauges = nullptr;
   float *ring = nullptr;
   int ngauges = 0, gauge_cap = 0;
+  bool gauges_due = false;    // the last step's samples are made by the next step's launch
   long long gauge_step0 = 0;  // root steps completed when the gauges were set
   int variant = 0;     // tile variant of the step kernels
   int blocking = 1;    // two steps per launch for linear single layers: 0 off, 1+shape
@@ -167,7 +168,8 @@ int tree_enqueue_children(Tree &T, LayerRec &P, bool with_max, hipStream_t st,
                           const DevLayer **beside = nullptr);
 // One complete root step: mass+open, nests, momentum + max, rotation.
 // next: another root step follows at once (its continuity may then ride in
-// this step's momentum launch, tree_fuses_halves).
+// this step's momentum launch, tree_fuses_halves, and this step's gauges in
+// the next step's launch).
 int tree_enqueue_root_step(Tree &T, hipStream_t st, bool next = false);
 bool tree_fuses_halves(const Tree &T);
 // The view of the launch that ends root step k and starts step k+1 (z1 =

@@ -493,8 +493,17 @@ DevLayer fused_halves_view(const Tree &T, const LayerRec &R) {
 int tree_enqueue_root_step(Tree &T, hipStream_t st, bool next) {
   LayerRec *R = T.layer(1);
   if (!R) return fail(8, "no root layer");
-  if (R->children.empty()) {
-    if (int r = tree_launch(T, *R, kFused, true, true, st)) return r;
+  const bool single = R->children.empty();
+  if (single) {
+    DevLayer d = dev_view(T, *R, true, true);
+    if (T.gauges_due) {
+      d.gauges = T.gauges;
+      d.gauge_ring = T.ring;
+      d.ngauge = T.ngauges;
+      d.gauge_cap = T.gauge_cap;
+      T.gauges_due = false;
+    }
+    if (int r = launch_view(T, *R, d, kFused, st)) return r;
   } else {
     if (!T.mass_ahead)
       if (int r = tree_launch(T, *R, kMassOnly, false, false, st)) return r;
@@ -513,7 +522,8 @@ int tree_enqueue_root_step(Tree &T, hipStream_t st, bool next) {
   }
   R->cur = 1 - R->cur;
   T.ctl_in = 1 - T.ctl_in;
-  return tree_enqueue_gauges(T, st);
+  T.gauges_due = next && single && T.ngauges > 0;
+  return T.gauges_due ? 0 : tree_enqueue_gauges(T, st);
 }
 
 bool tree_step2_eligible(const Tree &T) {

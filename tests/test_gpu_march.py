@@ -210,3 +210,35 @@ def test_root_beside_child_matches_oracle(nx, ny, foot, rt, clc):
             dev.close()
     finally:
         lib().gcomcot_set_tile_variant_(ip(0))
+
+
+@pytest.mark.parametrize("gov,cord,n,variant", [(1, 0, 9, 0), (1, 1, 300, 0), (1, 0, 24, 9), (1, 1, 1, 2), (0, 0, 257, 0),
+                                                (0, 1, 24, 0)],
+                         ids=["one-cell-tiles", "many", "strips", "tiles", "linear", "linear-cart"])
+def test_gauges_sampled_by_the_next_step(gov, cord, n, variant):
+    """A run samples the gauges of a step in the launch of the next one, a run
+    of one step in a launch of its own: the same samples, ring wraps included."""
+    import numpy as np
+    from gcomcot._lib import ip, lib
+    from helpers import BEACH
+    sc = S.custom(laycord=cord, laygov=gov, nx=150, ny=131, **BEACH)
+    x, y = S.layer_coords(sc.layers[0])
+    rng = np.random.default_rng(n)
+    pts = [(float(rng.uniform(x[0], x[-1])), float(rng.uniform(y[0], y[-1])), 1) for _ in range(n)]
+    got = []
+    try:
+        assert lib().gcomcot_set_tile_variant_(ip(variant)) == 0
+        for runs in ([19, 1, 5], [1] * 25):
+            print(f"[gpu] gauges gov {gov} cord {cord} n {n} variant {variant} runs {len(runs)}", flush=True)
+            dev = DeviceRun(sc)
+            dev.set_coords()
+            dev.set_gauges(pts, 16)
+            for k in runs:
+                dev.run(k)
+            got.append((dev.gauges(25), dev.state(1)["z1"]))
+            dev.close()
+    finally:
+        lib().gcomcot_set_tile_variant_(ip(0))
+    assert np.array_equal(got[0][0].view(np.int32), got[1][0].view(np.int32))
+    assert np.array_equal(got[0][1].view(np.int32), got[1][1].view(np.int32))
+    assert n == 1 or np.any(got[0][0] != 0)  # a lone gauge may lie where the wave has not come
