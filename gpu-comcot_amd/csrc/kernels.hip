@@ -632,7 +632,7 @@ __device__ __forceinline__ int tile_of_block(int per_xcd) {
 // publishes them).  IN: the tile and its halo lie more than SPAN+2 cells
 // inside the grid, so no index clamp, boundary ring, ghost row or range
 // limit of the Fortran loops can apply and all of them compile away.
-template <int MODE, bool NL, bool SPH, int TX, int TY, bool IN, bool ST, bool TAB>
+template <int MODE, bool NL, bool SPH, int TX, int TY, bool IN, bool ST, bool TAB, int NT = kThreads>
 __device__ __forceinline__ void tile_body(const DevLayer &L, int t, int ti0, int tj0, float *sm,
                                           const gcdet::Tables *stab) {
   constexpr int P = TX + 4, R = TY + 4, A = P * R;
@@ -645,23 +645,23 @@ __device__ __forceinline__ void tile_body(const DevLayer &L, int t, int ti0, int
   // before its first LDS write, so the tile waits for memory once rather
   // than once per pass of the thread over the staged rectangle
   {
-    constexpr int KS = (A + kThreads - 1) / kThreads;
-    constexpr int KC = SPH ? (kNumCoef * R + kThreads - 1) / kThreads : 0;
+    constexpr int KS = (A + NT - 1) / NT;
+    constexpr int KC = SPH ? (kNumCoef * R + NT - 1) / NT : 0;
     constexpr bool Z1 = MODE != kMomentOnly || NL, Z2 = MODE == kMomentOnly;
     float vh[KS], vm[KS], vn[KS], vz1[KS], vz2[KS], vdz[KS], vc[KC > 0 ? KC : 1];
-    TabStage<kThreads> tb;
+    TabStage<NT> tb;
     if constexpr (TAB) tb.load(tid);
 #pragma unroll
     for (int k = 0; k < KC; ++k) {
-      const int idx = tid + k * kThreads, c = idx / R, j = tj0 - 2 + idx % R;
+      const int idx = tid + k * NT, c = idx / R, j = tj0 - 2 + idx % R;
       vc[k] = idx < kNumCoef * R && (IN || (j >= 1 && j <= ny)) ? L.coef[c * ny + (j - 1)] : 0.0f;
     }
-    Walk<P, kThreads> w(tid);
+    Walk<P, NT> w(tid);
 #pragma unroll
     for (int k = 0; k < KS; ++k, w.next()) {
-      const int idx = tid + k * kThreads;
+      const int idx = tid + k * NT;
       const int gi = ti0 - 2 + w.i, gj = tj0 - 2 + w.j;
-      const bool in = (KS * kThreads == A || idx < A) &&
+      const bool in = (KS * NT == A || idx < A) &&
                       (IN || (gi >= 1 && gi <= nx && gj >= 1 && gj <= ny));
       const size_t g = in ? (size_t)(gj - 1) * nx + (gi - 1) : 0;
       vh[k] = in ? L.h[g] : 0.0f;
@@ -676,12 +676,12 @@ __device__ __forceinline__ void tile_body(const DevLayer &L, int t, int ti0, int
       float *crow = sm + 6 * A;
 #pragma unroll
       for (int k = 0; k < KC; ++k)
-        if (tid + k * kThreads < kNumCoef * R) crow[tid + k * kThreads] = vc[k];
+        if (tid + k * NT < kNumCoef * R) crow[tid + k * NT] = vc[k];
     }
 #pragma unroll
     for (int k = 0; k < KS; ++k) {
-      const int idx = tid + k * kThreads;
-      if (!(KS * kThreads == A || idx < A)) continue;
+      const int idx = tid + k * NT;
+      if (!(KS * NT == A || idx < A)) continue;
       const int gi = ti0 - 2 + idx % P, gj = tj0 - 2 + idx / P;
       const bool in = IN || (gi >= 1 && gi <= nx && gj >= 1 && gj <= ny);
       s.h[idx] = vh[k];
@@ -718,7 +718,7 @@ __device__ __forceinline__ void tile_body(const DevLayer &L, int t, int ti0, int
     constexpr int CY = MODE == kFused ? TY + 3 : TY;
     const int ci0 = MODE == kFused ? ti0 - 1 : ti0;
     const int cj0 = MODE == kFused ? tj0 - 1 : tj0;
-    for (Walk<CX, kThreads> w(tid); w.j < CY; w.next()) {
+    for (Walk<CX, NT> w(tid); w.j < CY; w.next()) {
       const int i = ci0 + w.i, j = cj0 + w.j;
       if (!IN && (i < 1 || i > nx || j < 1 || j > ny || on_ring(L, i, j))) continue;
       float z2, dz2;
@@ -727,7 +727,7 @@ __device__ __forceinline__ void tile_body(const DevLayer &L, int t, int ti0, int
       if (NL) s.dz[s.o(i, j)] = dz2;
     }
     if (!IN)
-      ring_cells<kThreads>(L, ci0, cj0, CX, CY, tid, [&](int i, int j) {
+      ring_cells<NT>(L, ci0, cj0, CX, CY, tid, [&](int i, int j) {
         s.z2[s.o(i, j)] = open_cell(L, s, i, j);
         if (NL) s.dz[s.o(i, j)] = 0.0f;
       });
@@ -741,8 +741,13 @@ __device__ __forceinline__ void tile_body(const DevLayer &L, int t, int ti0, int
     if (L.advance && t == 0 && tid == 0) L.ctl[1 - L.ctl_in] = step;
   }
   const float rdt = recip_refined(L.dt), zt = breaking_floor(L.dt);
+  // with two threads per cell the first half of the workgroup makes M, the
+  // elevation and the maximum, the second N
+  constexpr bool SPLIT = NT == 2 * TX * TY;
+  static_assert(!SPLIT || MODE == kFused, "two threads per cell: the fused step");
+  const bool first = !SPLIT || tid < NT / 2, second = !SPLIT || !first;
 #pragma unroll 1
-  for (int idx = tid; idx < TX * TY; idx += kThreads) {
+  for (int idx = SPLIT ? tid % (NT / 2) : tid; idx < TX * TY; idx += NT) {
     const int i = ti0 + idx % TX, j = tj0 + idx / TX;
     if (!IN && (i > nx || j > ny)) continue;
     const size_t g = (size_t)(j - 1) * nx + (i - 1);
@@ -752,7 +757,7 @@ __device__ __forceinline__ void tile_body(const DevLayer &L, int t, int ti0, int
       else if (i == 1 && j == 1) zo = s.Z2(2, 2);  // UPDATE ghosts, all_grids.f90:323-324
       else if (i == 1) zo = s.Z2(2, j);
       else zo = s.Z2(i, 2);
-      st_plane<ST>(L.z2 + g, zo);
+      if (first) st_plane<ST>(L.z2 + g, zo);
       if (MODE == kMassOnly && NL && L.dzp) L.dzp[g] = s.DZ(i, j);
     }
     if (MODE != kMassOnly) {
@@ -768,15 +773,15 @@ __device__ __forceinline__ void tile_body(const DevLayer &L, int t, int ti0, int
         const bool my =
             IN || (r ? (i <= nx - 1 && j <= ny - 1) : (i >= 2 && j >= 2 && j <= ny - 1));
         const float brk = L.linchk == 1 ? breaking_coef(L, s, i, j, rdt, zt) : 1.0f;
-        m2v = mx ? nl_x<SPH, IN>(L, s, i, j, brk) : 0.0f;
-        n2v = my ? nl_y<SPH, IN>(L, s, i, j, brk) : 0.0f;
+        m2v = mx && first ? nl_x<SPH, IN>(L, s, i, j, brk) : 0.0f;
+        n2v = my && second ? nl_y<SPH, IN>(L, s, i, j, brk) : 0.0f;
       } else {
         // MOMT_S / MOMT_C ranges (moment.f90:78-88, 117-119, 174-192, 233-235)
         const int lo = r ? 1 : 2;
         const bool mx = IN || (i >= lo && i <= nx - 1 && j >= lo);
         const bool my = IN || (j >= lo && j <= ny - 1 && i >= lo);
-        m2v = mx ? lin_x<SPH, IN>(L, s, i, j) : 0.0f;
-        n2v = my ? lin_y<SPH, IN>(L, s, i, j) : 0.0f;
+        m2v = mx && first ? lin_x<SPH, IN>(L, s, i, j) : 0.0f;
+        n2v = my && second ? lin_y<SPH, IN>(L, s, i, j) : 0.0f;
       }
       if (L.sponge_cx) {  // SPONGE_LAYER (boundaries.f90:228-239)
         const float cx = L.sponge_cx[i - 1], cy = L.sponge_cy[j - 1];
@@ -790,9 +795,9 @@ __device__ __forceinline__ void tile_body(const DevLayer &L, int t, int ti0, int
         if (j >= 2 && (i == 1 || i == nx)) m2v = dry ? 0.0f : L.edge[(i == 1 ? 0 : ny) + (j - 1)];
         if (i >= 2 && (j == 1 || j == ny)) n2v = dry ? 0.0f : L.edge[2 * ny + (j == 1 ? 0 : nx) + (i - 1)];
       }
-      st_plane<ST>(L.m2 + g, m2v);
-      st_plane<ST>(L.n2 + g, n2v);
-      if (L.zmax && (IN || r || (i >= 2 && j >= 2))) {
+      if (first) st_plane<ST>(L.m2 + g, m2v);
+      if (second) st_plane<ST>(L.n2 + g, n2v);
+      if (L.zmax && first && (IN || r || (i >= 2 && j >= 2))) {
         const float z2 = s.Z2(i, j);
         if (s.H(i, j) + z2 > kGx) {
           const float zm = L.zmax[g];
@@ -800,7 +805,7 @@ __device__ __forceinline__ void tile_body(const DevLayer &L, int t, int ti0, int
           if (z2 > zm) L.zmax[g] = z2;
         }
       }
-      if (L.zraw) {  // outermost layer only: every cell is its own
+      if (L.zraw && first) {  // outermost layer only: every cell is its own
         const float z2 = s.Z2(i, j);
         if (!(L.zraw[g] >= z2)) L.zraw[g] = z2;
       }
@@ -927,7 +932,7 @@ __device__ __forceinline__ void tile_body_mm(const DevLayer &L, int t, int ti0, 
 
 // TAB: the tile body also fills the workgroup's LDS copy of the pow/exp
 // tables (its loads issued with the tile's staging loads).
-template <int MODE, bool NL, bool SPH, int TX, int TY, bool ST = false, bool TAB = false>
+template <int MODE, bool NL, bool SPH, int TX, int TY, bool ST = false, bool TAB = false, int NT = kThreads>
 __device__ __forceinline__ void tile_step(const DevLayer &L, int t, int tiles_x, float *sm,
                                           const gcdet::Tables *stab) {
   const int ti0 = (t % tiles_x) * TX + 1, tj0 = (t / tiles_x) * TY + 1;
@@ -938,8 +943,8 @@ __device__ __forceinline__ void tile_step(const DevLayer &L, int t, int tiles_x,
     if (interior) tile_body_mm<SPH, TX, TY, true, ST, TAB>(L, t, ti0, tj0, sm, stab);
     else tile_body_mm<SPH, TX, TY, false, false, TAB>(L, t, ti0, tj0, sm, stab);
   } else {
-    if (interior) tile_body<MODE, NL, SPH, TX, TY, true, ST, TAB>(L, t, ti0, tj0, sm, stab);
-    else tile_body<MODE, NL, SPH, TX, TY, false, false, TAB>(L, t, ti0, tj0, sm, stab);
+    if (interior) tile_body<MODE, NL, SPH, TX, TY, true, ST, TAB, NT>(L, t, ti0, tj0, sm, stab);
+    else tile_body<MODE, NL, SPH, TX, TY, false, false, TAB, NT>(L, t, ti0, tj0, sm, stab);
   }
 }
 
@@ -1942,13 +1947,13 @@ __global__ void __launch_bounds__(NT)
 }
 
 // The fused nonlinear step of layers too small to fill the chip: 32 x 8
-// tiles, one cell per thread.  Such a launch lasts as long as one thread's
+// tiles, a thread or two (NT = 512) per cell.  Such a launch lasts as long as one thread's
 // chain of dependent operations (some 500 per cell at about 8 cycles each),
 // so the second cell of a 64 x 8 tile's thread costs more than the halo it
 // saves, and the smallest layers do not need the eight waves per SIMD that
 // the register limit of the large ones buys.
-template <bool SPH, int WAVES, bool ST>
-__global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(WAVES)))
+template <bool SPH, int NT, int WAVES, bool ST>
+__global__ void __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(WAVES)))
     k_step_small(DevLayer L, int tiles_x, int ntiles, int per_xcd) {
   constexpr int TX = 32, TY = 8;
   __shared__ float sm[6 * (TX + 4) * (TY + 4) + kNumCoef * (TY + 4)];
@@ -1957,50 +1962,49 @@ __global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(W
   if (b < 0) return;
   const int t = (b & 7) * per_xcd + (b >> 3);
   if (t >= ntiles) return;
-  tile_step<kFused, true, SPH, TX, TY, ST, true>(L, t, tiles_x, sm, &stab);
+  tile_step<kFused, true, SPH, TX, TY, ST, true, NT>(L, t, tiles_x, sm, &stab);
 }
 
 // The same beside the linear root's momentum + next continuity (DevLayer::
 // beside): 10.4 us where 401x401 tiles and a 512x384 root took 7.4 + 4.9.
-template <bool SPH, int WAVES, bool ST>
-__global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(WAVES)))
+template <bool SPH, int NT, int WAVES, bool ST>
+__global__ void __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(WAVES)))
     k_step_small_beside(DevLayer L, int tiles_x, int ntiles, int per_xcd, DevLayer R, MarchGrid RG, Beside B) {
   constexpr int TX = 32, TY = 8;
-  static_assert(kThreads == kMarchBlock, "one workgroup size for both");
   __shared__ float sm[6 * (TX + 4) * (TY + 4) + kNumCoef * (TY + 4)];
   __shared__ gcdet::Tables stab;
   const int b = beside_block(B, blockIdx.x);
   if (b < 0) {
-    march_mm_block<true, ST>(R, RG, -1 - b);
+    march_mm_block<true, ST, NT / kWave>(R, RG, -1 - b);
     return;
   }
   const int t = (b & 7) * per_xcd + (b >> 3);
   if (t >= ntiles) return;
-  tile_step<kFused, true, SPH, TX, TY, ST, true>(L, t, tiles_x, sm, &stab);
+  tile_step<kFused, true, SPH, TX, TY, ST, true, NT>(L, t, tiles_x, sm, &stab);
 }
 
-template <bool SPH, int WAVES>
+template <bool SPH, int NT, int WAVES>
 hipError_t launch_small(const DevLayer &L, hipStream_t st) {
   const int tx = (L.nx + 31) / 32, ty = (L.ny + 7) / 8;
   const int nt = tx * ty, per = (nt + 7) / 8;
   if (L.beside) {
     MarchGrid RG;
-    const long long rblocks = mm_grid(*L.beside, RG);
+    const long long rblocks = mm_grid<NT / kWave>(*L.beside, RG);
     if (8LL * per + rblocks > 0x7ffffff0) return hipErrorInvalidValue;
     const Beside B = beside_split(8LL * per, rblocks);
     if (L.stream_out)
-      hipLaunchKernelGGL((k_step_small_beside<SPH, WAVES, true>), dim3(B.total()), dim3(kThreads), 0, st, L,
+      hipLaunchKernelGGL((k_step_small_beside<SPH, NT, WAVES, true>), dim3(B.total()), dim3(NT), 0, st, L,
                          tx, nt, per, *L.beside, RG, B);
     else
-      hipLaunchKernelGGL((k_step_small_beside<SPH, WAVES, false>), dim3(B.total()), dim3(kThreads), 0, st, L,
+      hipLaunchKernelGGL((k_step_small_beside<SPH, NT, WAVES, false>), dim3(B.total()), dim3(NT), 0, st, L,
                          tx, nt, per, *L.beside, RG, B);
     return hipGetLastError();
   }
   if (L.stream_out)
-    hipLaunchKernelGGL((k_step_small<SPH, WAVES, true>), dim3(8 * per + gauge_blocks(L)), dim3(kThreads), 0, st,
+    hipLaunchKernelGGL((k_step_small<SPH, NT, WAVES, true>), dim3(8 * per + gauge_blocks(L)), dim3(NT), 0, st,
                        L, tx, nt, per);
   else
-    hipLaunchKernelGGL((k_step_small<SPH, WAVES, false>), dim3(8 * per + gauge_blocks(L)), dim3(kThreads), 0, st,
+    hipLaunchKernelGGL((k_step_small<SPH, NT, WAVES, false>), dim3(8 * per + gauge_blocks(L)), dim3(NT), 0, st,
                        L, tx, nt, per);
   return hipGetLastError();
 }
@@ -2080,10 +2084,17 @@ static int nl_form(const DevLayer &L, bool sph, int variant) {
 // Measured, us per step (64x8 tiles; 32x8 with 4 and 8 waves per SIMD):
 // 96x72 13.9; 9.4, 9.9.  517x391 14.4; 10.9, 11.3.  512x384 + 401x401 nest
 // 84.9; 67.2, 67.9.  1024x768 21.0; 18.95, 18.3.  1201x901 24.5; 23.2, 22.8.
+// Two threads per cell, M and N side by side, while the chip holds the tiles
+// three to a CU (later figures, one thread and two): 96x72 7.15, 5.7; 200x150
+// 7.15, 5.5; 300x225 7.6, 6.3; 401x401 (663 tiles) 7.8, 6.9; 517x391 (833) 7.7,
+// 8.7; 800x700 12.5, 13.5; Cartesian layers the same within 0.3.
+constexpr int kSplitTiles = 3 * 256;
 static hipError_t launch_small(const DevLayer &L, bool sph, hipStream_t st) {
+  if ((long long)((L.nx + 31) / 32) * ((L.ny + 7) / 8) <= kSplitTiles)
+    return sph ? launch_small<true, 512, 4>(L, st) : launch_small<false, 512, 4>(L, st);
   const bool few = (long long)L.nx * L.ny <= kSmallCells / 3;
-  if (sph) return few ? launch_small<true, 4>(L, st) : launch_small<true, 8>(L, st);
-  return few ? launch_small<false, 4>(L, st) : launch_small<false, 8>(L, st);
+  if (sph) return few ? launch_small<true, 256, 4>(L, st) : launch_small<true, 256, 8>(L, st);
+  return few ? launch_small<false, 256, 4>(L, st) : launch_small<false, 256, 8>(L, st);
 }
 
 // A nested layer's fused step with its root's momentum + next continuity: one

@@ -340,7 +340,7 @@ hipError_t launch_march_linear(const DevLayer &L, int steps, hipStream_t st) {
 hipError_t launch_march_moment_mass(const DevLayer &L, hipStream_t st) {
   if (!march_applies(L)) return hipErrorInvalidValue;
   MarchGrid G;
-  const long long blocks = mm_grid(L, G);
+  const long long blocks = mm_grid<>(L, G);
   return launch_grid<0>(L, G, blocks, st);
 }
 

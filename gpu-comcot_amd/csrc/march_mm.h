@@ -131,10 +131,11 @@ struct MarchGrid {
   int nstrip, east, seg, nseg, seg_side, nseg_side, side_blocks, per_xcd;
 };
 
-// The split for strips of W = 64 - 2 HW columns; its number of blocks.
-template <int HW>
+// The split for strips of W = 64 - 2 HW columns in blocks of WB waves; its
+// number of blocks.
+template <int HW, int WB = kMarchBlock / kWave>
 inline long long march_grid(const DevLayer &L, int seg, int seg_side, MarchGrid &G) {
-  constexpr int W = kWave - 2 * HW, WB = kMarchBlock / kWave;
+  constexpr int W = kWave - 2 * HW;
   G.nstrip = (L.nx + W - 1) / W;
   // first strip whose last lane lies beyond column NX - 1
   G.east = L.nx - 1 >= W + kWave - HW ? (L.nx - 1 - kWave + HW) / W + 1 : 1;
@@ -153,9 +154,9 @@ inline long long march_grid(const DevLayer &L, int seg, int seg_side, MarchGrid 
 // The strip of this wave in block b: side blocks first, then blocks in XCD
 // order (block b runs on XCD b % 8; each XCD takes one contiguous run of
 // waves, so strips that share halo columns meet in one L2).  False: none.
-template <int HW>
+template <int HW, int WB = kMarchBlock / kWave>
 __device__ __forceinline__ bool march_strip(const MarchGrid &G, int ny, int b, Strip &S) {
-  constexpr int W = kWave - 2 * HW, WB = kMarchBlock / kWave;
+  constexpr int W = kWave - 2 * HW;
   const int wb = threadIdx.x >> 6;
   if (b < G.side_blocks) {
     const int w = __builtin_amdgcn_readfirstlane(b * WB + wb);
@@ -177,7 +178,7 @@ __device__ __forceinline__ bool march_strip(const MarchGrid &G, int ny, int b, S
 }
 
 // Block b of momentum + next continuity.
-template <bool MX, bool ST>
+template <bool MX, bool ST, int WB = kMarchBlock / kWave>
 __device__ __forceinline__ void march_mm_block(const DevLayer &L, const MarchGrid &G, int b) {
   int step = 0;
   if (MX) {
@@ -185,7 +186,7 @@ __device__ __forceinline__ void march_mm_block(const DevLayer &L, const MarchGri
     if (L.advance && b == 0 && threadIdx.x == 0) L.ctl[1 - L.ctl_in] = step;
   }
   Strip S;
-  if (!march_strip<1>(G, L.ny, b, S)) return;
+  if (!march_strip<1, WB>(G, L.ny, b, S)) return;
   if (b < G.side_blocks) march_moment_mass<true, true, MX, ST>(L, S, step);
   else if (S.j0 - 1 >= 2 && S.j1 + 1 <= L.ny - 1) march_moment_mass<false, false, MX, ST>(L, S, step);
   else march_moment_mass<false, true, MX, ST>(L, S, step);
@@ -198,9 +199,10 @@ __device__ __forceinline__ void march_mm_block(const DevLayer &L, const MarchGri
 //   512x384 (3)                17.3, 18.0, 18.9, 20.1, 21.5
 //   1024x768 (12)              24.1, 23.4, 23.7, 23.7, 24.6
 //   2048x1536 (51)             36.3, 34.9, 31.8, 30.5, 30.6
+template <int WB = kMarchBlock / kWave>
 inline long long mm_grid(const DevLayer &L, MarchGrid &G) {
   const long long rows = (long long)((L.nx + 61) / 62) * L.ny / 1024;
-  return march_grid<1>(L, rows < 8 ? 2 : (rows < 32 ? 4 : 12), rows < 32 ? 2 : 4, G);
+  return march_grid<1, WB>(L, rows < 8 ? 2 : (rows < 32 ? 4 : 12), rows < 32 ? 2 : 4, G);
 }
 
 // A launch that runs a root's momentum + next continuity beside a step of its

@@ -242,3 +242,19 @@ def test_gauges_sampled_by_the_next_step(gov, cord, n, variant):
     assert np.array_equal(got[0][0].view(np.int32), got[1][0].view(np.int32))
     assert np.array_equal(got[0][1].view(np.int32), got[1][1].view(np.int32))
     assert n == 1 or np.any(got[0][0] != 0)  # a lone gauge may lie where the wave has not come
+
+
+@pytest.mark.parametrize("cord", [0, 1], ids=["sph", "cart"])
+@pytest.mark.parametrize("nx,ny", [(33, 9), (31, 25), (767, 253), (768, 256), (769, 256)], ids=lambda v: str(v))
+def test_two_threads_per_cell_matches_oracle(nx, ny, cord):
+    """Nonlinear layers either side of 768 tiles of 32x8, the most that take two
+    threads per cell, and of a tile or two."""
+    from helpers import BEACH
+    sc = S.custom(laycord=cord, laygov=1, nx=nx, ny=ny, **BEACH)
+    orc = Oracle(sc, 32, pow_mode=1)
+    print(f"[gpu] two threads per cell {nx}x{ny} cord {cord}", flush=True)
+    dev = DeviceRun(sc)
+    dev.run(21)
+    orc.step(21)
+    compare_device_oracle(sc, dev, orc, f"two threads per cell {nx}x{ny}")
+    dev.close()
