@@ -793,7 +793,7 @@ int gcomcot_autotune_(int *reps, int *variant, int *blocking, float *ms_per_step
   HIPCHK(hipEventCreate(&e0));
   HIPCHK(hipEventCreate(&e1));
   float best = 1e30f;
-  int bv = g_tree.variant, bb = 0;
+  int bv = 0, bb = 0;
   // The GPU's clocks settle over the first ~0.1 s of sustained work; the
   // candidates are timed after that, so that the first ones are not timed
   // at lower clocks than the last (dry launches of the current variant,
@@ -881,8 +881,10 @@ int gcomcot_autotune_(int *reps, int *variant, int *blocking, float *ms_per_step
   }
   (void)hipEventDestroy(e0);
   (void)hipEventDestroy(e1);
-  g_tree.variant = bv;
-  g_tree.blocking = bb;
+  // The variant is this layer's alone: a marching form that suits a large
+  // layer takes twice the default's time on the next, small one.
+  R->variant = bv;
+  if (!R->nl) g_tree.blocking = bb;
   if (variant) *variant = bv;
   if (blocking) *blocking = bb;
   if (ms_per_step) *ms_per_step = best;
@@ -1046,7 +1048,8 @@ int gcomcot_tile_variants_(int *count, int *tx, int *ty) {
   *count = num_tile_variants();
   if (tx && ty)
     for (int v = 0; v < *count; ++v) tile_variant_shape(v, &tx[v], &ty[v]);
-  return g_tree.variant;
+  const LayerRec *R = layer(1);
+  return R && R->variant >= 0 ? R->variant : g_tree.variant;
 }
 
 }  // extern "C"

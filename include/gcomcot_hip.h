@@ -341,7 +341,8 @@ int gcomcot_output_flush_(long long *nfiles);
  * shape of the two-step kernel, *reps launches each, on the live layer
  * with the maximum and the step counter switched off (such launches read
  * level 1 and write only level 2, so the state is unchanged); keep the
- * fastest for gcomcot_run_steps_ / gcomcot_time_steps_.  Reports the
+ * fastest for gcomcot_run_steps_ / gcomcot_time_steps_ on this layer (a new
+ * layer starts from gcomcot_set_tile_variant_'s again).  Reports the
  * choice and its time per root step.  In a tree with nested layers each
  * layer without nested layers of its own (the ones that run fused steps)
  * gets its own fastest tile variant the same way; *variant is then that of

@@ -258,3 +258,19 @@ def test_two_threads_per_cell_matches_oracle(nx, ny, cord):
     orc.step(21)
     compare_device_oracle(sc, dev, orc, f"two threads per cell {nx}x{ny}")
     dev.close()
+
+
+def test_a_tuned_variant_stays_with_its_layer():
+    """What the autotuner picks for one layer is not the next layer's variant."""
+    import ctypes
+    from gcomcot._lib import ip, lib
+    now = lambda: lib().gcomcot_tile_variants_(ctypes.byref(ctypes.c_int(0)), None, None)  # noqa: E731
+    assert lib().gcomcot_set_tile_variant_(ip(0)) == 0
+    print("[gpu] autotune 905x641", flush=True)
+    dev = DeviceRun(S.custom(laycord=0, laygov=1, nx=905, ny=641))
+    v, b, _ = dev.autotune(reps=3)
+    assert now() == v and b == 0
+    dev.close()
+    small = DeviceRun(S.custom(laycord=0, laygov=1, nx=64, ny=48))
+    assert now() == 0
+    small.close()
