@@ -69,17 +69,24 @@ GC_FD_HD bool div_inrange_applies(float a, float b, float q) {
 // |FF P| <= 2^-26 |X| (a quarter of an ulp at most, also just above a power of
 // two) and FF <= 2^-26.  sqrt(P^2 + Q^2) <= |P| + |Q|, and the power is at
 // least DF^2 from a depth of 1 on and 8 DF^2 (short by 1e-7) from 512 on;
-// kf26 = kDragScale * KF is 2^26 KF with 1e-3 to spare for every rounding
-// here and there.  NaN and infinite fluxes fail the comparisons, and where a
-// product underflows so does FF P.  In open water this holds for every flux
-// of a wave (4000 m deep, steps of a second or two: up to 1000 m^2/s), which
-// then needs no square root, power or quotient of it: 11 operations for 50.
+// kf26 = drag_scaled(KF) is 2^26 KF with 1e-3 to spare for every rounding
+// here and there.  Where a product underflows so does FF P.  The exact terms
+// give NaN where P^2 overflows, and no product here may overflow either: the
+// power's bound ends at 2^40 (a depth of 370 km) and kf26 starts at 2^-23, so
+// b <= w leaves fluxes of at most 2^63, and infinite and NaN ones fail.  In
+// open water this holds for every flux of a wave (4000 m deep, steps of a
+// second or two: up to 1000 m^2/s), which then needs no square root, power or
+// quotient of it: 12 operations for 50.
 // 4096x3072 spherical 115.5 -> 111.5 us per step (now bound by memory), 1024x768
 // 18.3 -> 17.2.  Cartesian layers, metre grids on shallow water, almost never
 // pass (1201x901 harbour with the test 18.3 -> 19.5): they go without it.
 constexpr float kDragScale = 0x1p26f * 1.001f;
+GC_FD_HD float drag_scaled(float kfric) {
+  const float k = kDragScale * kfric;
+  return k < 0x1p-23f ? 0x1p-23f : k;  // NaN passes
+}
 GC_FD_HD bool drag_vanishes(float kf26, float p, float q, float df, float x) {
-  const float d2 = df * df, w = df >= 512.0f ? 8.0f * d2 : d2;
+  const float d2 = df * df, w = fminf(df >= 512.0f ? 8.0f * d2 : d2, 0x1p40f);
   const float b = kf26 * (fabsf(p) + fabsf(q));
   return (df >= 1.0f) & (b <= w) & (b * fabsf(p) <= w * fabsf(x));
 }

@@ -128,7 +128,7 @@ __device__ __forceinline__ void march_nl(const DevLayer &L, const Strip S, int s
   const unsigned oz1 = plane_off(L, L.z1), om1 = plane_off(L, L.m1), on1 = plane_off(L, L.n1),
                  oz2 = plane_off(L, L.z2), om2 = plane_off(L, L.m2), on2 = plane_off(L, L.n2),
                  omax = plane_off(L, L.zmax), oarr = plane_off(L, L.arrival);
-  const float zt = breaking_floor(L.dt), kf26 = kDragScale * L.kfric;
+  const float zt = breaking_floor(L.dt), kf26 = drag_scaled(L.kfric);
   // a nested layer's boundary fluxes of the next sub-step: M of the side
   // columns comes row by row, N of rows 1 and NY once.  Lanes without one, and
   // every lane where there are none, read past the table: 0.
