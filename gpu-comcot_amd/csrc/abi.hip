@@ -436,7 +436,7 @@ void cuda_shutdown_(void) {
 // ------------------------------------------------------------- extended
 // Does the device loop advance the tree with the marching kernels?
 static bool marches() {
-  return tree_step2_eligible(g_tree) && g_tree.blocking == 1 &&
+  return tree_step2_eligible(g_tree) && blocking_mode(g_tree) == 1 &&
          march_applies(dev_view(g_tree, g_tree.layers[1], true, true));
 }
 
@@ -881,10 +881,11 @@ int gcomcot_autotune_(int *reps, int *variant, int *blocking, float *ms_per_step
   }
   (void)hipEventDestroy(e0);
   (void)hipEventDestroy(e1);
-  // The variant is this layer's alone: a marching form that suits a large
-  // layer takes twice the default's time on the next, small one.
+  // Both are this layer's alone: a marching form that suits a large layer
+  // takes twice the default's time on the next, small one, and a Cartesian
+  // layer's two-step tile keeps a spherical one from marching.
   R->variant = bv;
-  if (!R->nl) g_tree.blocking = bb;
+  if (!R->nl) R->blocking = bb;
   if (variant) *variant = bv;
   if (blocking) *blocking = bb;
   if (ms_per_step) *ms_per_step = best;
@@ -941,8 +942,11 @@ int gcomcot_set_store_policy_(int *mode) {
 int gcomcot_set_temporal_blocking_(int *mode) {
   if (*mode < 0 || *mode > kStep2Shapes) return fail(28, "temporal blocking mode %d out of range", *mode);
   g_tree.blocking = *mode;
+  for (LayerRec &L : g_tree.layers) L.blocking = -1;  // the autotuner's choice
   return 0;
 }
+
+int gcomcot_temporal_blocking_(void) { return blocking_mode(g_tree); }
 
 int gcomcot_hbm_copy_(int *mib, int *reps, float *ms_per_copy) {
   if (int e = ensure_init()) return e;

@@ -53,6 +53,7 @@ struct LayerRec {
   size_t sc_jnz_cells = 0;
   int cur = 0;  // buffer index holding time level 1
   int variant = -1;  // tile variant of this layer's fused launches (-1: the tree's)
+  int blocking = -1;  // temporal blocking mode of this layer (-1: the tree's)
   std::vector<int> children;
   size_t nxy() const { return (size_t)nx * ny; }
 };
@@ -175,6 +176,10 @@ bool tree_fuses_halves(const Tree &T);
 // The view of the launch that ends root step k and starts step k+1 (z1 =
 // Z(k), z2 = the buffer for Z(k+1)).
 DevLayer fused_halves_view(const Tree &T, const LayerRec &R);
+// The outermost layer's temporal blocking mode: the tuned one, else the tree's.
+inline int blocking_mode(const Tree &T) {
+  return T.layers[1].blocking >= 0 ? T.layers[1].blocking : T.blocking;
+}
 // True when the tree is one linear layer (two steps per launch apply).
 bool tree_step2_eligible(const Tree &T);
 // Two root steps of such a tree in one launch (temporal blocking).

@@ -530,7 +530,7 @@ bool tree_step2_eligible(const Tree &T) {
   const LayerRec &R = T.layers[1];
   // gauges sample every step and the sponge acts between steps, so both
   // keep one step per launch
-  return T.blocking > 0 && R.used && R.children.empty() && !R.nl && T.ngauges == 0 &&
+  return blocking_mode(T) > 0 && R.used && R.children.empty() && !R.nl && T.ngauges == 0 &&
          !R.sponge;
 }
 
@@ -601,7 +601,7 @@ int tree_enqueue_root_steps2(Tree &T, hipStream_t st) {
   LayerRec *R = T.layer(1);
   if (!R) return fail(8, "no root layer");
   DevLayer d = dev_view(T, *R, true, true);
-  hipError_t e = launch_step2(d, R->sph != 0, T.blocking - 1, st);
+  hipError_t e = launch_step2(d, R->sph != 0, blocking_mode(T) - 1, st);
   if (e != hipSuccess) return fail(200 + (int)e, "two-step launch failed: %s", hipGetErrorString(e));
   R->cur = 1 - R->cur;
   T.ctl_in = 1 - T.ctl_in;

@@ -193,6 +193,11 @@ module gcomcot_hip
       integer(c_int) :: mode
     end function
 
+    integer(c_int) function gcomcot_temporal_blocking() &
+        bind(C, name="gcomcot_temporal_blocking_")
+      import :: c_int
+    end function
+
     integer(c_int) function gcomcot_set_fused_halves(on) &
         bind(C, name="gcomcot_set_fused_halves_")
       import :: c_int

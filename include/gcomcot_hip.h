@@ -342,7 +342,8 @@ int gcomcot_output_flush_(long long *nfiles);
  * with the maximum and the step counter switched off (such launches read
  * level 1 and write only level 2, so the state is unchanged); keep the
  * fastest for gcomcot_run_steps_ / gcomcot_time_steps_ on this layer (a new
- * layer starts from gcomcot_set_tile_variant_'s again).  Reports the
+ * layer starts from gcomcot_set_tile_variant_'s and
+ * gcomcot_set_temporal_blocking_'s again).  Reports the
  * choice and its time per root step.  In a tree with nested layers each
  * layer without nested layers of its own (the ones that run fused steps)
  * gets its own fastest tile variant the same way; *variant is then that of
@@ -361,8 +362,10 @@ int gcomcot_autotune_(int *reps, int *variant, int *blocking, float *ms_per_step
  * autotuner picks among them).  Results are bitwise
  * those of single steps; afterwards level 2 holds the state two steps
  * before level 1 when the last launch was a two-step one.  Returns 0 if
- * valid. */
+ * valid.  Ends the mode that the autotuner chose for a layer. */
 int gcomcot_set_temporal_blocking_(int *mode);
+/* The mode that gcomcot_run_steps_ takes on the present outermost layer. */
+int gcomcot_temporal_blocking_(void);
 
 /* For an outermost linear layer with nested layers: the momentum launch of
  * each root step but the last of a gcomcot_run_steps_ / gcomcot_time_steps_

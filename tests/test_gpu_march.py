@@ -274,3 +274,26 @@ def test_a_tuned_variant_stays_with_its_layer():
     small = DeviceRun(S.custom(laycord=0, laygov=1, nx=64, ny=48))
     assert now() == 0
     small.close()
+
+
+def test_a_tuned_blocking_stays_with_its_layer():
+    """What the autotuner picks for one linear layer is not the next layer's
+    temporal blocking mode: the tree's own mode holds there."""
+    from gcomcot._lib import ip, lib
+    now = lib().gcomcot_temporal_blocking_
+    try:
+        assert lib().gcomcot_set_temporal_blocking_(ip(5)) == 0
+        print("[gpu] autotune linear 1024x768", flush=True)
+        dev = DeviceRun(S.custom(laycord=0, laygov=0, nx=1024, ny=768))
+        _, b, _ = dev.autotune(reps=3)
+        assert now() == b
+        dev.close()
+        small = DeviceRun(S.custom(laycord=0, laygov=0, nx=64, ny=48))
+        assert now() == 5
+        _, b, _ = small.autotune(reps=3)
+        assert now() == b
+        assert lib().gcomcot_set_temporal_blocking_(ip(2)) == 0
+        assert now() == 2  # the caller's mode ends the tuned one
+        small.close()
+    finally:
+        lib().gcomcot_set_temporal_blocking_(ip(1))
