@@ -793,7 +793,7 @@ int gcomcot_autotune_(int *reps, int *variant, int *blocking, float *ms_per_step
   HIPCHK(hipEventCreate(&e0));
   HIPCHK(hipEventCreate(&e1));
   float best = 1e30f;
-  int bv = 0, bb = 0;
+  int bv = 0, bb = 0, tv = -1, tb = -1;  // tv, tb: among the tiles alone
   // The GPU's clocks settle over the first ~0.1 s of sustained work; the
   // candidates are timed after that, so that the first ones are not timed
   // at lower clocks than the last (dry launches of the current variant,
@@ -865,16 +865,28 @@ int gcomcot_autotune_(int *reps, int *variant, int *blocking, float *ms_per_step
         return r;
       if (ms < best) { best = ms; bv = v; bb = 0; }
     }
+    if (R->nl && march_nl_applies(d, R->sph != 0)) {
+      DevLayer t = d;
+      t.block_bytes = 0;  // a view that does not march
+      float tile = 1e30f;
+      for (int v = 0; v < num_tile_variants() && tile_variant_is_tile(v); ++v) {
+        float ms;
+        if (int r = time_it([&] { return launch_step(t, kFused, true, R->sph != 0, v, g_stream); }, 1, &ms))
+          return r;
+        if (ms < tile) { tile = ms; tv = v; }
+      }
+    }
     if (!R->nl) {
       const bool march = march_applies(dev_view(g_tree, *R, true, true));
       constexpr int K = kMarchSteps;
+      float tile = best, ms;
+      tb = 0;
       for (int sh = 0; sh < kStep2Shapes; ++sh) {
-        float ms;
+        if (int r = time_it([&] { return launch_step2(d, R->sph != 0, sh, g_stream); }, 2, &ms)) return r;
+        if (ms < tile) { tile = ms; tb = sh + 1; }
         // mode 1 (shape 0) is the marching kernels where they apply
-        if (int r = sh == 0 && march
-                        ? time_it([&] { return launch_march_linear(d, K, g_stream); }, K, &ms)
-                        : time_it([&] { return launch_step2(d, R->sph != 0, sh, g_stream); }, 2, &ms))
-          return r;
+        if (sh == 0 && march)
+          if (int r = time_it([&] { return launch_march_linear(d, K, g_stream); }, K, &ms)) return r;
         if (ms < best) { best = ms; bb = sh + 1; }
       }
     }
@@ -885,7 +897,9 @@ int gcomcot_autotune_(int *reps, int *variant, int *blocking, float *ms_per_step
   // takes twice the default's time on the next, small one, and a Cartesian
   // layer's two-step tile keeps a spherical one from marching.
   R->variant = bv;
-  if (!R->nl) R->blocking = bb;
+  R->tile_variant = tv;
+  R->blocking = R->nl ? -1 : bb;
+  R->tile_blocking = tb;
   if (variant) *variant = bv;
   if (blocking) *blocking = bb;
   if (ms_per_step) *ms_per_step = best;
@@ -942,7 +956,7 @@ int gcomcot_set_store_policy_(int *mode) {
 int gcomcot_set_temporal_blocking_(int *mode) {
   if (*mode < 0 || *mode > kStep2Shapes) return fail(28, "temporal blocking mode %d out of range", *mode);
   g_tree.blocking = *mode;
-  for (LayerRec &L : g_tree.layers) L.blocking = -1;  // the autotuner's choice
+  for (LayerRec &L : g_tree.layers) L.blocking = L.tile_blocking = -1;  // the autotuner's choices
   return 0;
 }
 
@@ -1044,7 +1058,7 @@ int gcomcot_detmath_eval_noalloc_(long long *n, const float *x, float *pow_out,
 int gcomcot_set_tile_variant_(int *variant) {
   if (*variant < 0 || *variant >= num_tile_variants()) return 1;
   g_tree.variant = *variant;
-  for (LayerRec &L : g_tree.layers) L.variant = -1;  // the autotuner's per-layer choices
+  for (LayerRec &L : g_tree.layers) L.variant = L.tile_variant = -1;  // the autotuner's per-layer choices
   return 0;
 }
 
@@ -1053,7 +1067,7 @@ int gcomcot_tile_variants_(int *count, int *tx, int *ty) {
   if (tx && ty)
     for (int v = 0; v < *count; ++v) tile_variant_shape(v, &tx[v], &ty[v]);
   const LayerRec *R = layer(1);
-  return R && R->variant >= 0 ? R->variant : g_tree.variant;
+  return R ? fused_variant(g_tree, *R, dev_view(g_tree, *R, true, true)) : g_tree.variant;
 }
 
 }  // extern "C"

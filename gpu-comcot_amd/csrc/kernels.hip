@@ -2066,6 +2066,7 @@ void tile_variant_shape(int v, int *tx, int *ty) {
   *tx = kVariants[v][0] ? kVariants[v][1] : -kVariants[v][1];  // negative: marching strips
   *ty = kVariants[v][2];
 }
+bool tile_variant_is_tile(int v) { return kVariants[v][0] != 0; }
 
 // The form of a nonlinear layer's fused step: rows per segment of the marching
 // strips, 0 for 32x8 tiles, -1 for the variant's tiles.

@@ -54,6 +54,8 @@ struct LayerRec {
   int cur = 0;  // buffer index holding time level 1
   int variant = -1;  // tile variant of this layer's fused launches (-1: the tree's)
   int blocking = -1;  // temporal blocking mode of this layer (-1: the tree's)
+  // the tuner's choice of each among the tiles, for launches that cannot march
+  int tile_variant = -1, tile_blocking = -1;
   std::vector<int> children;
   size_t nxy() const { return (size_t)nx * ny; }
 };
@@ -177,9 +179,11 @@ bool tree_fuses_halves(const Tree &T);
 // Z(k), z2 = the buffer for Z(k+1)).
 DevLayer fused_halves_view(const Tree &T, const LayerRec &R);
 // The outermost layer's temporal blocking mode: the tuned one, else the tree's.
-inline int blocking_mode(const Tree &T) {
-  return T.layers[1].blocking >= 0 ? T.layers[1].blocking : T.blocking;
-}
+// A tuned layer whose launches cannot march (any more: files with maxima were
+// asked for, a sponge set) takes the best of the tiles.
+int blocking_mode(const Tree &T);
+// The tile variant of a fused launch of L on view d, chosen in the same way.
+int fused_variant(const Tree &T, const LayerRec &L, const DevLayer &d);
 // True when the tree is one linear layer (two steps per launch apply).
 bool tree_step2_eligible(const Tree &T);
 // Two root steps of such a tree in one launch (temporal blocking).

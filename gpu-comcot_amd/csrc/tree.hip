@@ -374,8 +374,19 @@ DevLayer substep_view(const Tree &T, const LayerRec &C, bool with_max, int k, in
   return d;
 }
 
+int fused_variant(const Tree &T, const LayerRec &L, const DevLayer &d) {
+  if (L.tile_variant >= 0 && L.nl && !march_nl_applies(d, L.sph != 0)) return L.tile_variant;
+  return L.variant >= 0 ? L.variant : T.variant;
+}
+
+int blocking_mode(const Tree &T) {
+  const LayerRec &R = T.layers[1];
+  if (R.tile_blocking >= 0 && !march_applies(dev_view(T, R, true, true))) return R.tile_blocking;
+  return R.blocking >= 0 ? R.blocking : T.blocking;
+}
+
 static int launch_view(const Tree &T, const LayerRec &L, const DevLayer &d, int mode, hipStream_t st) {
-  const int v = mode == kFused && L.variant >= 0 ? L.variant : T.variant;
+  const int v = mode == kFused ? fused_variant(T, L, d) : T.variant;
   hipError_t e = launch_step(d, mode, L.nl != 0, L.sph != 0, v, st);
   if (e != hipSuccess) return fail(200 + (int)e, "step kernel launch failed: %s", hipGetErrorString(e));
   return 0;

@@ -30,6 +30,7 @@ namespace {
 // kernels.hip kBatchShapes; shapes 3-5 are the same tiles in the other launch form
 const int kShapes[][2] = {{64, 8}, {32, 16}, {64, 16}};
 
+int g_last_variant = -1, g_last_step2 = -1;  // of launch_step and launch_step2
 long long g_fused_tiles = 0;  // tiles of momentum + next continuity launches
 
 void tile_op(const DevLayer &d, int mode, int t, int tiles_x, int TX, int TY,
@@ -228,13 +229,15 @@ void run_fill(void *a) {
 
 namespace gc {
 
-hipError_t launch_step(const DevLayer &L, int mode, bool, bool, int, hipStream_t st) {
+hipError_t launch_step(const DevLayer &L, int mode, bool, bool, int variant, hipStream_t st) {
   StepArg a{L, mode};
+  g_last_variant = variant;
   emu_submit(st, run_step, &a, sizeof(a));
   return hipSuccess;
 }
-hipError_t launch_step2(const DevLayer &L, bool, int, hipStream_t st) {
+hipError_t launch_step2(const DevLayer &L, bool, int shape, hipStream_t st) {
   StepArg a{L, kFused};
+  g_last_step2 = shape;
   emu_submit(st, run_step, &a, sizeof(a));  // the planner tests never take this path
   return hipSuccess;
 }
@@ -311,3 +314,5 @@ hipError_t launch_fill_i32(int *p, int n, int v, hipStream_t st) {
 }  // namespace gc
 
 long long emu_fused_tiles() { return g_fused_tiles; }
+int emu_last_variant() { return g_last_variant; }
+int emu_last_step2() { return g_last_step2; }

@@ -1,0 +1,81 @@
+// Checks of a single layer tree (tree.hip) against the runtime and kernel
+// stand-ins of this folder.  Usage: emu_tree CHECK; a failed check is named and
+// ends with status 2.
+#include <cstdio>
+#include <cstdlib>
+#include <cstring>
+#include <vector>
+
+#include "comcot_consts.h"
+#include "tree.h"
+
+using namespace gc;
+
+namespace {
+
+[[noreturn]] void die(const char *m) {
+  std::fprintf(stderr, "%s\n", m);
+  std::exit(2);
+}
+void ok(bool c, const char *m) {
+  if (!c) die(m);
+}
+
+void add_root(Tree &T, int laycord, int laygov, int nx, int ny) {
+  const int corners[4] = {1, nx, 1, ny};
+  const std::vector<float> h((size_t)nx * ny, 100.0f), z((size_t)nx * ny, 0.0f);
+  if (tree_create_layer(T, nullptr, 1, -1, 1, laycord, laygov, 1, 1, corners, 0, 0.013f, 1.0f, 1.0f, 1.0f,
+                        nx, ny, h.data(), z.data()) ||
+      tree_upload_coef(T.layers[1], std::vector<float>((size_t)kNumCoef * ny, 0.0f)))
+    die("layer 1");
+}
+
+// A tuned layer whose launches cannot march, because MAX_AMP's maximum is kept
+// or a sponge set, takes the tuner's best tile; as soon as they can again, its
+// tuned form.
+void tuned_fallback() {
+  Tree T;
+  add_root(T, 0, 1, 70, 60);
+  LayerRec &R = T.layers[1];
+  T.variant = 2;
+  auto step = [&] {
+    ok(tree_enqueue_root_step(T, nullptr) == 0, "root step");
+    return emu_last_variant();
+  };
+  ok(step() == 2, "an untuned layer's variant");
+  R.variant = 8;
+  R.tile_variant = 3;
+  ok(step() == 8, "a tuned layer's variant");
+  T.raw_max = 1;
+  ok(step() == 3, "the best tile where the maximum is kept");
+  T.raw_max = 0;
+  ok(step() == 8, "the tuned variant again");
+  tree_free(T);
+
+  add_root(T, 0, 0, 70, 60);
+  T.blocking = 2;
+  auto two = [&] {
+    ok(tree_step2_eligible(T), "two steps per launch");
+    ok(tree_enqueue_root_steps2(T, nullptr) == 0, "two root steps");
+    return emu_last_step2() + 1;
+  };
+  ok(two() == 2, "an untuned layer's mode");
+  T.layers[1].blocking = 1;
+  T.layers[1].tile_blocking = 5;
+  ok(blocking_mode(T) == 1, "a tuned layer's mode");
+  T.raw_max = 1;
+  ok(two() == 5, "the best two-step tile where the maximum is kept");
+  T.layers[1].tile_blocking = 0;
+  ok(!tree_step2_eligible(T), "one step per launch where that was the fastest without marching");
+  tree_free(T);
+}
+
+}  // namespace
+
+int main(int argc, char **argv) {
+  const char *check = argc > 1 ? argv[1] : "";
+  if (!std::strcmp(check, "tuned-fallback")) tuned_fallback();
+  else die("no such check");
+  if (emu_live_bytes() != 0) die("device memory leaked");
+  std::printf("%s passed\n", check);
+}

@@ -63,3 +63,6 @@ long long emu_live_bytes();
 long long emu_cross_stream_waits();
 // tiles run by momentum + next continuity launches
 long long emu_fused_tiles();
+// variant of the last single launch of a step, shape of the last two-step one
+int emu_last_variant();
+int emu_last_step2();

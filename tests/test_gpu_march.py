@@ -297,3 +297,37 @@ def test_a_tuned_blocking_stays_with_its_layer():
         small.close()
     finally:
         lib().gcomcot_set_temporal_blocking_(ip(1))
+
+
+@pytest.mark.parametrize("gov,cord", [(1, 0), (0, 0), (0, 1)], ids=["nonlinear", "linear", "linear-cart"])
+def test_a_tuned_layer_keeps_maxima_in_tiles(gov, cord, tmp_path):
+    """A tuned layer that is asked for maximum files, which the marching forms
+    cannot keep, runs the tuner's best tile, with the same bits, and its tuned
+    form again without them."""
+    import ctypes
+    import numpy as np
+    from gcomcot._lib import ip, lib
+    from helpers import BEACH
+    variant = lambda: lib().gcomcot_tile_variants_(ctypes.byref(ctypes.c_int(0)), None, None)  # noqa: E731
+    mode = lib().gcomcot_temporal_blocking_
+    assert lib().gcomcot_set_tile_variant_(ip(0)) == 0
+    sc = S.custom(laycord=cord, laygov=gov, nx=905, ny=741, **BEACH)
+    print(f"[gpu] tuned layer with maxima gov {gov} cord {cord}", flush=True)
+    got = []
+    for out_opt in (1, 2):
+        dev = DeviceRun(sc)
+        v, b, _ = dev.autotune(reps=3)
+        assert (variant(), mode()) == (v, b if gov == 0 else 1)
+        dev.set_output(tmp_path, iprt=0, out_opt=out_opt)
+        if out_opt == 2:
+            assert gov == 0 or variant() < 6
+        else:
+            assert (variant(), mode()) == (v, b if gov == 0 else 1)
+        dev.run(14)
+        got.append((dev.state(1), dev.maxima(1)))
+        dev.close()
+    (a, am), (c, cm) = got
+    for k in ("z1", "m1", "n1"):
+        assert np.array_equal(a[k].view(np.int32), c[k].view(np.int32)), k
+    for k in ("zmax_wet", "arrival"):
+        assert np.array_equal(am[k].view(np.int32), cm[k].view(np.int32)), k
