@@ -840,6 +840,7 @@ int gcomcot_autotune_(int *reps, int *variant, int *blocking, float *ms_per_step
       int lv = 0;
       for (int v = 0; v < num_tile_variants(); ++v) {
         float ms;
+        if (!tile_variant_takes(v, dl, L.nl != 0, L.sph != 0)) continue;
         if (int r = time_it([&] { return launch_step(dl, kFused, L.nl != 0, L.sph != 0, v, g_stream); },
                             1, &ms))
           return r;
@@ -860,6 +861,7 @@ int gcomcot_autotune_(int *reps, int *variant, int *blocking, float *ms_per_step
   if (fused_only) {
     for (int v = 0; v < num_tile_variants(); ++v) {
       float ms;
+      if (!tile_variant_takes(v, d, R->nl != 0, R->sph != 0)) continue;
       if (int r = time_it([&] { return launch_step(d, kFused, R->nl != 0, R->sph != 0, v, g_stream); },
                           1, &ms))
         return r;

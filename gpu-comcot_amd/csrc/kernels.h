@@ -117,6 +117,11 @@ inline bool march_nl_applies(const DevLayer &L, bool sph) {
 }
 int march_nl_seg(int nx, int ny);
 hipError_t launch_march_nl(const DevLayer &L, bool sph, int seg, hipStream_t st);
+// Whether tile variant v is a form of its own on this view: marching strips
+// that a layer cannot take are variant 0 again.
+inline bool tile_variant_takes(int v, const DevLayer &L, bool nl, bool sph) {
+  return tile_variant_is_tile(v) || (nl && march_nl_applies(L, sph));
+}
 
 // Reference-semantics maximum (no wet test) plus the wet max/arrival.
 hipError_t launch_max(const DevLayer &L, float *zmax_raw, hipStream_t st);

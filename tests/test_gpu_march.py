@@ -331,3 +331,23 @@ def test_a_tuned_layer_keeps_maxima_in_tiles(gov, cord, tmp_path):
         assert np.array_equal(a[k].view(np.int32), c[k].view(np.int32)), k
     for k in ("zmax_wet", "arrival"):
         assert np.array_equal(am[k].view(np.int32), cm[k].view(np.int32)), k
+
+
+def test_the_tuner_reports_only_forms_that_its_layer_runs():
+    """Variants 6-10 are marching strips: of a layer that cannot take them
+    (linear, without friction or convection) the tuner times and reports tiles
+    only."""
+    cases = [dict(laygov=0, laycord=0), dict(laygov=0, laycord=1), dict(laygov=1, laycord=0, fric_coef=0.0),
+             dict(laygov=9, laycord=1)]
+    for kw in cases:
+        for nx, ny in ((331, 290), (96, 72)):
+            print(f"[gpu] tuner's variants {kw} {nx}x{ny}", flush=True)
+            dev = DeviceRun(S.custom(nx=nx, ny=ny, **kw))
+            v, _, _ = dev.autotune(reps=2)
+            dev.close()
+            assert v < 6, kw
+    child = dict(laycord=1, laygov=0, footprint=(51, 41), rel_size=4, rel_time=3, corner=(8, 14))
+    dev = DeviceRun(S.custom(nx=110, ny=84, laygov=0, child=child))
+    v, _, _ = dev.autotune(reps=2)
+    dev.close()
+    assert v < 6
