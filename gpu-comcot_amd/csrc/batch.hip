@@ -1055,7 +1055,13 @@ long long gcomcot_batch_device_bytes_(int *sid) {
 }
 
 long long gcomcot_layer_footprint_(int *nx, int *ny, int *nonlinear) {
-  return (long long)layer_bytes(*nx, *ny, *nonlinear != 0, false);
+  return (long long)(layer_bytes(*nx, *ny, *nonlinear != 0, false) +
+                     layer_tail_bytes(*nx, *ny, true, 2 * kMaxEdgeSlots));
+}
+
+long long gcomcot_layer_footprint_ex_(int *nx, int *ny, int *laycord, int *nonlinear, int *rel_time) {
+  return (long long)(layer_bytes(*nx, *ny, *nonlinear != 0, false) +
+                     layer_tail_bytes(*nx, *ny, *laycord == 0, *rel_time));
 }
 
 void gcomcot_batch_set_arrival_threshold_(float *thr) { g_eng.arr_thr = *thr; }

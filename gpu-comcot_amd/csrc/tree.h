@@ -31,16 +31,19 @@ struct LayerRec {
   int fric = 0, modscm = 0, linchk = 1;
   float fric_coef = 0, dt = 0, dx = 0, dy = 0, rx = 0, ry = 0, grx = 0, gry = 0, kfric = 0;
   int nx = 0, ny = 0;
-  void *block = nullptr;  // one allocation holding every plane below
-  size_t block_bytes = 0;
+  void *block = nullptr;  // one allocation holding every plane below and, behind
+  size_t block_bytes = 0; // them, tail_bytes of tables that checkpoints leave out
+  size_t tail_bytes = 0;
   float *h = nullptr, *z[2] = {nullptr, nullptr}, *m[2] = {nullptr, nullptr},
         *n[2] = {nullptr, nullptr};
   float *zmax_raw = nullptr, *zmax_wet = nullptr, *coef = nullptr, *r24 = nullptr;
   float *dzp = nullptr, *xflux = nullptr, *yflux = nullptr;
   int *arrival = nullptr;
-  float *rowc = nullptr;    // row-major copy of the coefficients (DevLayer::rowc)
-  float *edge = nullptr;    // nested layers: boundary fluxes of coming sub-steps, behind the
-  int edge_slots = 0;       // planes of block (DevLayer::edge), one slot per sub-step
+  // behind the planes: the row-major copy of the coefficients (DevLayer::rowc),
+  // and a nested layer's boundary fluxes of coming sub-steps (DevLayer::edge),
+  // one slot per sub-step
+  float *rowc = nullptr, *edge = nullptr;
+  int edge_slots = 0;
   float *deform = nullptr;  // last seafloor deformation applied (on first use)
   float *sponge = nullptr;  // SPONGE_COEF: COEFX[NX] then COEFY[NY] (layer 1, when on)
   // SC_OPTION = 1 (Cartesian child of a spherical layer 1): POS, CXY, the
@@ -115,8 +118,12 @@ constexpr long long kStreamCells = (192ll << 20) / 36;
 constexpr long long kL2Cells = (32ll << 20) / 36;
 bool streams_planes(const LayerRec &L);
 
-// Bytes of device memory a layer of nx x ny cells takes (planes + tables).
+// Bytes of device memory a layer of nx x ny cells takes: its planes and their
+// tables, and what lies behind them for a layer of that REL_TIME (1 where no
+// boundary fluxes are made ahead).
 size_t layer_bytes(int nx, int ny, bool nl, bool r24);
+inline int edge_slots_of(int rel_time) { return std::min(rel_time / 2, kMaxEdgeSlots); }
+size_t layer_tail_bytes(int nx, int ny, bool sph, int rel_time);
 
 // Unlink nested layer id from its parent and free it (no-op for the root
 // or an unused id).

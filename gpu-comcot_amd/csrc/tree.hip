@@ -78,17 +78,22 @@ size_t layer_bytes(int nx, int ny, bool nl, bool r24) {
   return b;
 }
 
+static size_t rowc_bytes(int ny, bool sph) { return sph ? pad((size_t)kRowCoef * ny * sizeof(float)) : 0; }
+
+size_t layer_tail_bytes(int nx, int ny, bool sph, int rel_time) {
+  return rowc_bytes(ny, sph) + pad((size_t)edge_slots_of(rel_time) * edge_floats(nx, ny) * sizeof(float));
+}
+
 size_t Tree::device_bytes() const {
   size_t b = 0;
   for (const auto &L : layers)
-    if (L.used) b += L.block_bytes + (L.r24 ? 2 * L.nxy() * 4 : 0);
+    if (L.used) b += L.block_bytes + L.tail_bytes + (L.r24 ? 2 * L.nxy() * 4 : 0);
   return b;
 }
 
 static void free_layer(LayerRec &L) {
   if (L.block) (void)hipFree(L.block);
   if (L.r24) (void)hipFree(L.r24);
-  if (L.rowc) (void)hipFree(L.rowc);
   if (L.deform) (void)hipFree(L.deform);
   if (L.sponge) (void)hipFree(L.sponge);
   if (L.sc_pos) (void)hipFree(L.sc_pos);
@@ -217,12 +222,13 @@ int tree_create_layer(Tree &T, hipStream_t st, int id, int parent, int level, in
   L.ny = ny;
   const size_t n = L.nxy();
   L.block_bytes = layer_bytes(nx, ny, L.nl != 0, false);
-  L.edge_slots = id == 1 || sc ? 0 : std::min(L.rel_time / 2, kMaxEdgeSlots);
-  const size_t edges = (size_t)L.edge_slots * edge_floats(nx, ny) * sizeof(float);
+  const int ahead_of = id == 1 || sc ? 1 : L.rel_time;
+  L.edge_slots = edge_slots_of(ahead_of);
+  L.tail_bytes = layer_tail_bytes(nx, ny, L.sph != 0, ahead_of);
   {
-    hipError_t e = hipMalloc(&L.block, L.block_bytes + edges);
+    hipError_t e = hipMalloc(&L.block, L.block_bytes + L.tail_bytes);
     if (e != hipSuccess) {
-      const size_t want = L.block_bytes + edges;
+      const size_t want = L.block_bytes + L.tail_bytes;
       L = LayerRec();
       return fail(100 + (int)e, "layer %d: %zu bytes of device memory: %s", id, want,
                   hipGetErrorString(e));
@@ -242,7 +248,8 @@ int tree_create_layer(Tree &T, hipStream_t st, int id, int parent, int level, in
   L.xflux = c.take<float>(2 * (size_t)nx);
   L.yflux = c.take<float>(2 * (size_t)ny);
   L.coef = c.take<float>((size_t)kNumCoef * ny);
-  if (L.edge_slots) L.edge = reinterpret_cast<float *>(static_cast<char *>(L.block) + L.block_bytes);
+  if (L.edge_slots)
+    L.edge = reinterpret_cast<float *>(static_cast<char *>(L.block) + L.block_bytes + rowc_bytes(ny, L.sph != 0));
   HIPCHK(hipMemsetAsync(L.block, 0, L.block_bytes, st));
   HIPCHK(hipMemsetAsync(L.arrival, 0xff, n * sizeof(int), st));  // -1 = not arrived
   HIPCHK(hipMemcpyAsync(L.h, H, n * sizeof(float), hipMemcpyHostToDevice, st));
@@ -266,7 +273,7 @@ static int upload_rowc(LayerRec &L, const float *coef) {
                                  c(kF2), c(kF4),        c(kR5),  0.0f};
     std::copy(row, row + kRowCoef, rows.begin() + (size_t)j * kRowCoef);
   }
-  if (!L.rowc) HIPCHK(hipMalloc(&L.rowc, rows.size() * sizeof(float)));
+  L.rowc = reinterpret_cast<float *>(static_cast<char *>(L.block) + L.block_bytes);
   HIPCHK(hipMemcpy(L.rowc, rows.data(), rows.size() * sizeof(float), hipMemcpyHostToDevice));
   return 0;
 }

@@ -25,20 +25,27 @@ def _ll(v):
 def _setup(L):
     if getattr(L, "_batch_typed", False):
         return
-    for name in ("gcomcot_batch_device_bytes_", "gcomcot_layer_footprint_"):
+    for name in ("gcomcot_batch_device_bytes_", "gcomcot_layer_footprint_", "gcomcot_layer_footprint_ex_"):
         getattr(L, name).restype = _LL
     L._batch_typed = True
 
 
 def layer_footprint(nx, ny, nonlinear):
-    """Device bytes one layer takes (planes, tables; 256-B aligned)."""
+    """Device bytes one layer takes at most (planes, tables; 256-B aligned)."""
     L = lib()
     _setup(L)
     return int(L.gcomcot_layer_footprint_(ip(nx), ip(ny), ip(1 if nonlinear else 0)))
 
 
 def scenario_footprint(sc):
-    return sum(layer_footprint(s.nx, s.ny, _is_nl(s)) for s in sc.layers)
+    """Device bytes that a scenario's layers take."""
+    L = lib()
+    _setup(L)
+
+    def ahead(s):  # REL_TIME of the layers whose boundary fluxes are made ahead
+        return 1 if s.id == 1 or getattr(s, "sc_pos", None) is not None else s.rel_time
+    return sum(int(L.gcomcot_layer_footprint_ex_(ip(s.nx), ip(s.ny), ip(s.laycord), ip(1 if _is_nl(s) else 0),
+                                                 ip(ahead(s)))) for s in sc.layers)
 
 
 def _is_nl(s):

@@ -475,8 +475,11 @@ int gcomcot_batch_get_max_(int *sid, int *lid, float *zmax_wet, int *arrival);
 int gcomcot_batch_remove_(int *sid);
 /* device bytes held by scenario *sid (0: all scenarios) */
 long long gcomcot_batch_device_bytes_(int *sid);
-/* device bytes one layer of nx x ny cells takes (admission control) */
+/* device bytes one layer of nx x ny cells takes (admission control): at most,
+ * and exactly for its LAYCORD and REL_TIME (1 for an outermost layer and for an
+ * SC_OPTION 1 one, whose coupling tables come on top) */
 long long gcomcot_layer_footprint_(int *nx, int *ny, int *nonlinear);
+long long gcomcot_layer_footprint_ex_(int *nx, int *ny, int *laycord, int *nonlinear, int *rel_time);
 void gcomcot_batch_set_arrival_threshold_(float *thr);
 /* *autotune != 0: time the launch forms and tile shapes on the live batch;
  * *shape >= 0 forces one for the fused launches: 0/1/2 = persistent kernel

@@ -6,6 +6,7 @@
 #include <cstring>
 #include <vector>
 
+#include "../../include/gcomcot_hip.h"
 #include "comcot_consts.h"
 #include "tree.h"
 
@@ -70,11 +71,44 @@ void tuned_fallback() {
   tree_free(T);
 }
 
+// Device memory that the layers report is what they allocate: in a tree, and
+// through the batch engine's entries, whose footprint of a layer is exact with
+// its REL_TIME and a bound without.
+void footprint() {
+  const int kind[][3] = {{0, 0, 1}, {0, 1, 1}, {1, 0, 1}, {1, 1, 1}, {0, 1, 2}, {1, 1, 4}, {0, 0, 5}, {1, 0, 21}};
+  for (const auto &k : kind) {
+    int lc = k[0], lg = k[1], rt = k[2], one = 1, two = 2, root = -1, cart = 1, nx = 77, ny = 60, R = 3;
+    int corners[4] = {1, nx, 1, ny}, foot[4] = {8, 30, 9, 25}, fs = 0;
+    int cnx = 23 * R + 1, cny = 17 * R + 1, sid = 0;
+    float fc = 0.013f, dt = 1.0f, d = 1.0f;
+    long long steps = 1, live = emu_live_bytes();
+    std::vector<float> h(100 * 100, 50.0f), z(100 * 100, 0.0f), coef(10 * 100, 0.0f);
+    ok(gcomcot_batch_new_scenario_(&steps, &sid) == 0, "scenario");
+    ok(gcomcot_batch_add_layer_(&sid, &one, &root, &lc, &lg, &one, &one, corners, &fs, &fc, &dt, &d, &d,
+                                coef.data(), h.data(), z.data(), &nx, &ny) == 0, "layer 1");
+    long long want = gcomcot_layer_footprint_ex_(&nx, &ny, &lc, &lg, &one);
+    ok(want <= gcomcot_layer_footprint_(&nx, &ny, &lg), "the bound of layer 1");
+    if (rt > 1) {
+      ok(gcomcot_batch_add_layer_(&sid, &two, &one, &cart, &lg, &R, &rt, foot, &fs, &fc, &dt, &d, &d, nullptr,
+                                  h.data(), z.data(), &cnx, &cny) == 0, "layer 2");
+      const long long child = gcomcot_layer_footprint_ex_(&cnx, &cny, &cart, &lg, &rt);
+      ok(child <= gcomcot_layer_footprint_(&cnx, &cny, &lg), "the bound of layer 2");
+      want += child;
+    }
+    ok(gcomcot_batch_device_bytes_(&sid) == want, "the scenario's bytes and its layers' footprints");
+    // beside its layers a scenario holds its two step counters
+    ok(emu_live_bytes() - live == want + 2 * (long long)sizeof(int), "the bytes allocated");
+    ok(gcomcot_batch_remove_(&sid) == 0 && emu_live_bytes() == live, "removal");
+  }
+  ok(gcomcot_batch_reset_() == 0, "reset");
+}
+
 }  // namespace
 
 int main(int argc, char **argv) {
   const char *check = argc > 1 ? argv[1] : "";
   if (!std::strcmp(check, "tuned-fallback")) tuned_fallback();
+  else if (!std::strcmp(check, "footprint")) footprint();
   else die("no such check");
   if (emu_live_bytes() != 0) die("device memory leaked");
   std::printf("%s passed\n", check);

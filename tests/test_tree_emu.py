@@ -1,6 +1,6 @@
 """CPU: a single layer tree (tree.hip) against the runtime emulator of
 tests/batch_emu, compiled with g++ (AddressSanitizer and UBSan on): which forms
-its launches take."""
+its launches take, and the device memory that its layers report."""
 import os
 import shutil
 import subprocess
@@ -19,13 +19,13 @@ def emu_tree(tmp_path_factory):
     exe = str(tmp_path_factory.mktemp("tree_emu") / "emu_tree")
     subprocess.run(["g++", "-std=c++17", "-O1", "-g", "-fsanitize=address,undefined",
                     "-fno-omit-frame-pointer", "-I", EMU, "-I", CSRC, "-x", "c++",
-                    os.path.join(CSRC, "tree.hip"), "-x", "none", os.path.join(EMU, "emu_runtime.cpp"),
+                    os.path.join(CSRC, "tree.hip"), os.path.join(CSRC, "batch.hip"), "-x", "none", os.path.join(EMU, "emu_runtime.cpp"),
                     os.path.join(EMU, "emu_kernels.cpp"), os.path.join(EMU, "emu_tree.cpp"), "-o", exe],
                    check=True, capture_output=True, text=True)
     return exe
 
 
-@pytest.mark.parametrize("check", ["tuned-fallback"])
+@pytest.mark.parametrize("check", ["tuned-fallback", "footprint"])
 def test_tree(emu_tree, check):
     r = subprocess.run([emu_tree, check], capture_output=True, text=True, timeout=120,
                        env=dict(os.environ, ASAN_OPTIONS="detect_leaks=1"))
