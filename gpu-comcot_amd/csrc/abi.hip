@@ -1030,6 +1030,29 @@ int gcomcot_division_check_(long long *pairs, unsigned long long *seed, long lon
   return 0;
 }
 
+int gcomcot_reciprocal_check_(long long *tested, long long *bad, unsigned *example) {
+  if (int e = ensure_init()) return e;
+  const int blocks = 4096, lanes = blocks * 256;
+  std::vector<unsigned long long> h(3 * (size_t)lanes);
+  unsigned long long *d = nullptr;
+  HIPCHK(hipMalloc(&d, h.size() * sizeof(unsigned long long)));
+  hipError_t e = launch_reciprocal_check(d, blocks, g_stream);
+  if (e == hipSuccess)
+    e = hipMemcpyAsync(h.data(), d, h.size() * sizeof(unsigned long long), hipMemcpyDeviceToHost, g_stream);
+  if (e == hipSuccess) e = hipStreamSynchronize(g_stream);
+  (void)hipFree(d);
+  if (e != hipSuccess) return fail(205, "reciprocal check failed: %s", hipGetErrorString(e));
+  *tested = *bad = 0;
+  *example = 0;
+  for (int g = 0; g < lanes; ++g) {
+    const unsigned long long *o = h.data() + 3 * (size_t)g;
+    if (o[1] && !*bad) *example = (unsigned)o[2];
+    *tested += (long long)o[0];
+    *bad += (long long)o[1];
+  }
+  return 0;
+}
+
 int gcomcot_detmath_eval_(long long *n, const float *x, float *pow_out, float *exp_out) {
   if (*n < 0 || (*n > 0 && (!x || !pow_out || !exp_out)))
     return fail(36, "gcomcot_detmath_eval_: n must be >= 0 and the arrays given");

@@ -9,11 +9,12 @@
 //
 // div_inrange(a, b) is that sequence without the scalings, the fix-up and
 // the first residual correction.  The refined reciprocal is 1/b correctly
-// rounded for every b (all 2^23 significands, on the device), and then one
-// correction q + (a - b q)/b rounds to the IEEE quotient: before that
-// rounding it is within 2.3 * 2^-24 ulp of a/b, which leaves per divisor
-// only the numerators whose quotient comes that close to a midpoint; they
-// are all enumerated in tests/quotient_check.cpp, and none rounds wrongly.  V_DIV_SCALE leaves both operands unchanged, and V_DIV_FIXUP
+// rounded for every divisor in range (gcomcot_reciprocal_check_ tries them all
+// on the device), and then one correction q + (a - b q)/b rounds to the IEEE
+// quotient: before that rounding it is within 2.3 * 2^-24 ulp of a/b, which
+// leaves per divisor only the numerators whose quotient comes that close to a
+// midpoint; they are all enumerated in tests/quotient_check.cpp, and none
+// rounds wrongly.  V_DIV_SCALE leaves both operands unchanged, and V_DIV_FIXUP
 // passes the quotient through, unless b is 0, denormal or so large that
 // 1/b is, a is 0 or below 2^-103 in magnitude, a/b is below 2^-126 or the
 // exponents differ by 96 or more; for the other (a, b) the result is the

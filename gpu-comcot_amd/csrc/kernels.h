@@ -302,5 +302,8 @@ hipError_t launch_detmath_eval(const float *x, long long n, float *pw, float *ex
                                hipStream_t st);
 hipError_t launch_division_check(unsigned long long seed, int per_lane, unsigned long long *out,
                                  int blocks, hipStream_t st);
+// The same of its refined reciprocal: out[3g..3g+2] = lane g's divisors tested,
+// mismatches and the bits of its first one; 256*blocks lanes.
+hipError_t launch_reciprocal_check(unsigned long long *out, int blocks, hipStream_t st);
 
 }  // namespace gc

@@ -1547,6 +1547,26 @@ __global__ void __launch_bounds__(256) k_division_check(unsigned long long seed,
   out[6 * g + 5] = exsq;
 }
 
+// The refined reciprocal of every divisor of div_inrange's range, both signs,
+// against the IEEE quotient 1 / b.
+__global__ void __launch_bounds__(256) k_reciprocal_check(unsigned long long *out) {
+  const unsigned long long g = (unsigned long long)blockIdx.x * blockDim.x + threadIdx.x;
+  const unsigned long long lanes = (unsigned long long)gridDim.x * blockDim.x;
+  unsigned long long tested = 0, bad = 0, ex = 0;
+  for (unsigned long long k = g; k < (1ull << 32); k += lanes) {
+    const float b = f_of((unsigned)k);
+    if (!(fabsf(b) >= ldexpf(1.0f, -kDivRange) && fabsf(b) <= ldexpf(1.0f, kDivRange))) continue;
+    ++tested;
+    if (__float_as_uint(1.0f / b) != __float_as_uint(recip_refined(b))) {
+      if (!bad) ex = k;
+      ++bad;
+    }
+  }
+  out[3 * g] = tested;
+  out[3 * g + 1] = bad;
+  out[3 * g + 2] = ex;
+}
+
 // Dry land shows 0, else the elevation plus the tide correction when it is
 // not negligible: DATA_PRT (output.f90:781-793) and MAX_AMP (:918-931).
 __device__ __forceinline__ float shown_elevation(float z, float h, float tide) {
@@ -2385,6 +2405,11 @@ hipError_t launch_detmath_eval(const float *x, long long n, float *pw, float *ex
 hipError_t launch_division_check(unsigned long long seed, int per_lane, unsigned long long *out,
                                  int blocks, hipStream_t st) {
   hipLaunchKernelGGL(k_division_check, dim3(blocks), dim3(256), 0, st, seed, per_lane, out);
+  return hipGetLastError();
+}
+
+hipError_t launch_reciprocal_check(unsigned long long *out, int blocks, hipStream_t st) {
+  hipLaunchKernelGGL(k_reciprocal_check, dim3(blocks), dim3(256), 0, st, out);
   return hipGetLastError();
 }
 

@@ -412,6 +412,10 @@ int gcomcot_division_check_(long long *pairs, unsigned long long *seed, long lon
                             long long *bad_inrange, long long *bad_sqrt, long long *tested,
                             unsigned *example_x, unsigned *example_a, unsigned *example_b,
                             unsigned *example_s);
+/* The refined reciprocal in that quotient against the IEEE 1 / b, for every
+ * float b within 2^+-120 (*tested of them), on the device: *bad = mismatches,
+ * *example = the bits of one. */
+int gcomcot_reciprocal_check_(long long *tested, long long *bad, unsigned *example);
 
 /* The Manning depth power x^2.3333333 and the breaking exponential e^x as
  * the nonlinear momentum kernels compute them (moment.f90:459-460 and

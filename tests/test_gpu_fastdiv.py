@@ -35,3 +35,17 @@ def test_short_divisions_and_sqrt_equal_ieee(seed):
     assert bsq.value == 0, f"sqrt_inrange: {bsq.value} mismatches, e.g. x = {f(es.value)!r}"
     assert bin_.value == 0, (f"div_inrange: {bin_.value} mismatches, e.g. "
                              f"{f(ea.value)!r} / {f(eb.value)!r}")
+
+
+def test_refined_reciprocal_is_the_rounded_one_for_every_divisor():
+    """What tests/quotient_check.cpp takes as given: the reciprocal that the
+    quotient starts from is 1/b rounded to nearest, for every significand and
+    exponent of a divisor in range (2^-120 to 2^120: 240 binades and 2^120
+    itself) and both signs."""
+    print("[gpu] reciprocal check", flush=True)
+    tested, bad = ctypes.c_longlong(0), ctypes.c_longlong(-1)
+    ex = ctypes.c_uint(0)
+    check(lib().gcomcot_reciprocal_check_(ctypes.byref(tested), ctypes.byref(bad), ctypes.byref(ex)),
+          "reciprocal check")
+    assert tested.value == 2 * (240 * 2 ** 23 + 1)
+    assert bad.value == 0, f"{bad.value} mismatches, e.g. 1 / {float(np.array([ex.value], np.uint32).view(np.float32)[0])!r}"
