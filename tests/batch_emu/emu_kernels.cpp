@@ -7,16 +7,22 @@
 // the root-step counter (mirrored into arrival[0]).  Each launch checks
 // that its tiles cover every cell of every layer exactly once, that queue
 // heads were cleared, and JNQ/JNZ check the sub-step they run in against
-// the parent's and the child's step counts (all_grids.f90 order).  A
-// violated check aborts the process.
+// the parent's and the child's step counts (all_grids.f90 order).  JNQ notes
+// for which step of its child it made the boundary fluxes and stamps those that
+// it makes ahead (DevLayer::edge) with the step they are for: a child's step
+// needs its own, from JNQ or from the slot that the step before it wrote out,
+// and none made before JNZ may serve a step after it.  A violated check aborts
+// the process.
 #include <cmath>
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
+#include <map>
 #include <vector>
 
 #include "kernels.h"
 #include "source.h"
+#include "tree.h"
 
 using namespace gc;
 
@@ -32,6 +38,25 @@ const int kShapes[][2] = {{64, 8}, {32, 16}, {64, 16}};
 
 int g_last_variant = -1, g_last_step2 = -1;  // of launch_step and launch_step2
 long long g_fused_tiles = 0;  // tiles of momentum + next continuity launches
+
+// Per nested layer (its depth plane): the step (Z's count before it) whose
+// boundary fluxes are in its level-1 planes.
+std::map<const float *, float> g_boundary;
+
+// A nested layer's step finds its boundary fluxes made ...
+void check_boundary(const DevLayer &d, int mode) {
+  if (d.is_root || mode == kMomentOnly) return;
+  const auto it = g_boundary.find(d.h);
+  if (it == g_boundary.end() || it->second != d.z1[0]) die("a sub-step without its boundary fluxes");
+  if (mode != kFused && d.edge) die("boundary fluxes ahead in a split step");
+}
+// ... and writes the next step's where it is given them
+void pass_boundary(const DevLayer &d, int mode) {
+  if (d.is_root || mode != kFused || !d.edge) return;
+  for (size_t k = 0; k < edge_floats(d.nx, d.ny); ++k)
+    if (d.edge[k] != d.z1[0] + 1.0f) die("a slot of boundary fluxes of another sub-step");
+  g_boundary[d.h] = d.z1[0] + 1.0f;
+}
 
 void tile_op(const DevLayer &d, int mode, int t, int tiles_x, int TX, int TY,
              std::vector<unsigned char> &cov) {
@@ -73,9 +98,11 @@ void run_step(void *a) {
   const StepArg *s = (const StepArg *)a;
   const int tx = (s->d.nx + 63) / 64, ty = (s->d.ny + 7) / 8;
   std::vector<unsigned char> cov((size_t)s->d.nx * s->d.ny, 0);
+  check_boundary(s->d, s->mode);
   for (int t = 0; t < tx * ty; ++t) tile_op(s->d, s->mode, t, tx, 64, 8, cov);
   for (auto c : cov)
     if (c != 1) die("layer launch coverage");
+  pass_boundary(s->d, s->mode);
 }
 
 struct BatchArg {
@@ -104,6 +131,7 @@ void run_batch(void *a) {
     for (int r = 0; r < s; ++r)
       if (B.descs[r].L.z2 == bd.L.z2) die("layer twice in one launch");
     cov[s].assign((size_t)bd.L.nx * bd.L.ny, 0);
+    if (!B.dry) check_boundary(bd.L, x->mode);  // the tuner's launches have none
   }
   for (int it = 0; it < B.nitems; ++it) {
     const BatchItem w = B.items[it];
@@ -113,6 +141,8 @@ void run_batch(void *a) {
   for (auto &c : cov)
     for (auto v : c)
       if (v != 1) die("batch launch coverage");
+  for (int s = 0; s < nslot; ++s)
+    if (!B.dry) pass_boundary(B.descs[s].L, x->mode);
   for (int q = 0; q < 8; ++q) B.heads[q] = B.qstart[q + 1] - B.qstart[q] + 8;
 }
 
@@ -137,6 +167,12 @@ void check_jnq(const DevNest &N, int t) {
     std::fprintf(stderr, "t=%d cz1=%g pm1=%g RT=%d cnx=%d\n", t, N.cz1[0], ps, N.rel_time, N.cnx);
     die("JNQ in the wrong sub-step");
   }
+  const int last = t + N.ahead;
+  if (N.ahead < 0 || N.ahead > edge_slots_of(N.rel_time) || (N.ahead > 0 && !N.edge)) die("slots of boundary fluxes");
+  if (last > N.rel_time || (t <= nhalf(N.rel_time) && last > nhalf(N.rel_time))) die("boundary fluxes beyond JNZ");
+  g_boundary[N.ch] = N.cz1[0];
+  const size_t n = edge_floats(N.cnx, N.cny);
+  for (int s = 0; s < N.ahead; ++s) std::fill(N.edge + s * n, N.edge + (s + 1) * n, N.cz1[0] + 1.0f + s);
 }
 
 void check_jnz(const DevNest &N) {
@@ -145,6 +181,16 @@ void check_jnz(const DevNest &N) {
   for (size_t c = 0; c < cn; ++c)
     if (N.cz2[c] != N.cz1[c] + 1.0f) die("JNZ before the child's step");
   if (N.cz1[0] - N.pm1[0] * N.rel_time != nhalf(N.rel_time) - 1) die("JNZ in the wrong sub-step");
+  const auto it = g_boundary.find(N.ch);
+  if (it != g_boundary.end() && it->second > N.cz1[0]) die("boundary fluxes made before JNZ for a sub-step after it");
+  if (N.next_t == 0) return;
+  if (N.next_t != nhalf(N.rel_time) + 1 || N.next_t < 3) die("JNZ with the JNQ of another sub-step");
+  DevNest Q = N;  // that JNQ follows UPDATE
+  Q.cz1 = N.cz2;
+  Q.cz2 = N.cz1;
+  Q.cm1 = N.cm2;
+  Q.cn1 = N.cn2;
+  check_jnq(Q, N.next_t);
 }
 
 struct NestArg {
@@ -232,7 +278,13 @@ namespace gc {
 hipError_t launch_step(const DevLayer &L, int mode, bool, bool, int variant, hipStream_t st) {
   StepArg a{L, mode};
   g_last_variant = variant;
+  a.d.beside = nullptr;
   emu_submit(st, run_step, &a, sizeof(a));
+  if (L.beside) {  // the root's momentum + next continuity, beside a nested layer's step
+    if (mode != kFused || L.is_root) die("a root beside another step than a nested layer's");
+    StepArg r{*L.beside, kMomentMass};
+    emu_submit(st, run_step, &r, sizeof(r));
+  }
   return hipSuccess;
 }
 hipError_t launch_step2(const DevLayer &L, bool, int shape, hipStream_t st) {

@@ -71,6 +71,39 @@ void tuned_fallback() {
   tree_free(T);
 }
 
+int add_child(Tree &T, int id, int parent, int laygov, int R, int rt, const int *c) {
+  const int nx = (c[1] - c[0] + 1) * R + 1, ny = (c[3] - c[2] + 1) * R + 1;
+  const std::vector<float> h((size_t)nx * ny, 50.0f), z((size_t)nx * ny, 0.0f);
+  return tree_create_layer(T, nullptr, id, parent, T.layers[parent].level + 1, 1, laygov, R, rt, c, 0, 0.013f,
+                           1.0f, 1.0f, 1.0f, nx, ny, h.data(), z.data()) ||
+         tree_upload_coef(T.layers[id], std::vector<float>((size_t)kNumCoef * ny, 0.0f));
+}
+
+// Every sub-step of a nest finds its boundary fluxes made, whatever JNQ makes
+// ahead, JNZ takes along or the root's march runs beside: REL_TIMEs on every
+// remainder and beyond the slots, two children, and a child of a child.
+void substeps() {
+  for (int rt = 1; rt <= 21; ++rt)
+    for (int form = 0; form < 3; ++form) {  // one child; two; one with a child of its own
+      Tree T;
+      add_root(T, 0, form == 2 ? 1 : 0, 60, 50);
+      const int a[4] = {6, 13, 7, 15}, b[4] = {20, 30, 9, 18}, g[4] = {5, 12, 4, 11};
+      const int rt2 = (rt + 3) % 7 + 1;
+      ok(add_child(T, 2, 1, rt % 2, 3, rt, a) == 0, "layer 2");
+      if (form == 1) ok(add_child(T, 3, 1, 1, 2, rt2, b) == 0, "layer 3");
+      if (form == 2) ok(add_child(T, 3, 2, 1, 2, rt2, g) == 0, "layer 3");
+      const int steps = 5;
+      for (int k = 1; k <= steps; ++k) ok(tree_enqueue_root_step(T, nullptr, k < steps) == 0, "root step");
+      const int want[4] = {0, steps, steps * rt, form == 2 ? steps * rt * rt2 : steps * rt2};
+      for (int id = 1; id <= (form ? 3 : 2); ++id) {
+        const LayerRec &L = T.layers[id];
+        for (size_t c = 0; c < L.nxy(); ++c)
+          ok(L.z[L.cur][c] == want[id] && L.m[L.cur][c] == want[id] && L.n[L.cur][c] == want[id], "step count");
+      }
+      tree_free(T);
+    }
+}
+
 // Device memory that the layers report is what they allocate: in a tree, and
 // through the batch engine's entries, whose footprint of a layer is exact with
 // its REL_TIME and a bound without.
@@ -109,6 +142,7 @@ int main(int argc, char **argv) {
   const char *check = argc > 1 ? argv[1] : "";
   if (!std::strcmp(check, "tuned-fallback")) tuned_fallback();
   else if (!std::strcmp(check, "footprint")) footprint();
+  else if (!std::strcmp(check, "substeps")) substeps();
   else die("no such check");
   if (emu_live_bytes() != 0) die("device memory leaked");
   std::printf("%s passed\n", check);

@@ -1,6 +1,7 @@
 """CPU: a single layer tree (tree.hip) against the runtime emulator of
 tests/batch_emu, compiled with g++ (AddressSanitizer and UBSan on): which forms
-its launches take, and the device memory that its layers report."""
+its launches take, the device memory that its layers report, and that every
+sub-step of a nest finds its boundary fluxes made."""
 import os
 import shutil
 import subprocess
@@ -25,7 +26,7 @@ def emu_tree(tmp_path_factory):
     return exe
 
 
-@pytest.mark.parametrize("check", ["tuned-fallback", "footprint"])
+@pytest.mark.parametrize("check", ["tuned-fallback", "footprint", "substeps"])
 def test_tree(emu_tree, check):
     r = subprocess.run([emu_tree, check], capture_output=True, text=True, timeout=120,
                        env=dict(os.environ, ASAN_OPTIONS="detect_leaks=1"))
