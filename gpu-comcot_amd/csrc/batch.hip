@@ -199,8 +199,7 @@ int shape_for(int nl, int sph, long long cells, const std::vector<DevLayer> &lay
   if (g_eng.forced_shape >= 0) return g_eng.forced_shape;
   auto it = g_eng.tuned.find(kind_key(nl, sph, cells));
   const int sh = it != g_eng.tuned.end() ? it->second
-                                         : batch_rule_shape(layers.data(), (int)layers.size(), nl != 0,
-                                                            batch_num_shapes());
+                                         : batch_rule_shape(layers.data(), (int)layers.size(), nl != 0);
   for (const DevLayer &d : layers)
     if (!batch_shape_takes(sh, d, nl != 0, sph != 0)) return kBatchGridShape;
   return sh;

@@ -247,8 +247,8 @@ inline bool batch_shape_takes(int shape, const DevLayer &L, bool nl, bool sph) {
 // The shape of a fused launch that nobody tuned: marching strips where the
 // layers together give their SIMDs enough rows (the lines of march_nl_seg),
 // one cell per thread below, 64 x 8 tiles for linear layers.
-inline int batch_rule_shape(const DevLayer *layers, int n, bool nl, int num_shapes) {
-  if (!nl || num_shapes <= kBatchMarchShape) return kBatchGridShape;
+inline int batch_rule_shape(const DevLayer *layers, int n, bool nl) {
+  if (!nl) return kBatchGridShape;
   long long rows = 0;
   for (int k = 0; k < n; ++k) rows += (long long)((layers[k].nx + 59) / 60) * layers[k].ny / 1024;
   return rows < 16 ? kBatchSmallShape : (rows < 36 ? kBatchMarchShape : kBatchMarchShape + 1);

@@ -110,6 +110,10 @@ int main(int argc, char **argv) {
     shape = -1;
     if (gcomcot_batch_set_tuning_(&on, &shape)) return 3;
   }
+  if (std::getenv("EMU_RULE")) {  // the shapes of a batch that nobody tuned
+    shape = -1;
+    if (gcomcot_batch_set_tuning_(&zero, &shape)) return 3;
+  }
   if (gcomcot_batch_set_two_step_(&two, shape2 >= 0 ? &shape2 : nullptr)) return 3;
   int fuse = std::getenv("EMU_FUSE") ? std::atoi(std::getenv("EMU_FUSE")) : 1;
   if (gcomcot_batch_set_fused_halves_(&fuse)) return 3;
@@ -155,6 +159,9 @@ int main(int argc, char **argv) {
   std::printf("seed %u: %d scenarios verified, shape %d, two-step %d (shape %d), "
               "%lld cross-stream waits, fused halves %d (%lld tiles)\n", seed, checked, shape,
               two, shape2, emu_cross_stream_waits(), fuse, emu_fused_tiles());
+  std::printf("launches by shape:");
+  for (int k = 0; k < 9; ++k) std::printf(" %lld", emu_shape_launches(k));
+  std::printf("\n");
   (void)zero;
   return 0;
 }

@@ -33,8 +33,11 @@ namespace {
   std::abort();
 }
 
-// kernels.hip kBatchShapes; shapes 3-5 are the same tiles in the other launch form
-const int kShapes[][2] = {{64, 8}, {32, 16}, {64, 16}};
+// kernels.hip kBatchShapes (3-5 are the same tiles in the other launch form),
+// then the small tiles and the two marching forms of nonlinear layers
+const int kShapes[][2] = {{64, 8}, {32, 16}, {64, 16}, {64, 8}, {32, 16}, {64, 16}, {32, 8}, {60, 32}, {60, 56}};
+constexpr int kNumShapes = sizeof(kShapes) / sizeof(kShapes[0]);
+long long g_shape_launches[kNumShapes] = {};
 
 int g_last_variant = -1, g_last_step2 = -1;  // of launch_step and launch_step2
 long long g_fused_tiles = 0;  // tiles of momentum + next continuity launches
@@ -108,6 +111,7 @@ void run_step(void *a) {
 struct BatchArg {
   BatchLaunch B;
   int mode, shape;
+  bool nl, sph;
 };
 
 void run_batch(void *a) {
@@ -120,7 +124,7 @@ void run_batch(void *a) {
     if (B.heads[q] != 0) die("queue head not cleared before the launch");
   }
   int TX = 64, TY = 8;
-  if (x->mode == kFused) TX = kShapes[x->shape % 3][0], TY = kShapes[x->shape % 3][1];
+  if (x->mode == kFused) TX = kShapes[x->shape][0], TY = kShapes[x->shape][1], ++g_shape_launches[x->shape];
   int nslot = 0;
   for (int it = 0; it < B.nitems; ++it) nslot = std::max(nslot, B.items[it].slot + 1);
   std::vector<std::vector<unsigned char>> cov(nslot);
@@ -131,6 +135,7 @@ void run_batch(void *a) {
     for (int r = 0; r < s; ++r)
       if (B.descs[r].L.z2 == bd.L.z2) die("layer twice in one launch");
     cov[s].assign((size_t)bd.L.nx * bd.L.ny, 0);
+    if (x->mode == kFused && !batch_shape_takes(x->shape, bd.L, x->nl, x->sph)) die("a shape that the layer cannot take");
     if (!B.dry) check_boundary(bd.L, x->mode);  // the tuner's launches have none
   }
   for (int it = 0; it < B.nitems; ++it) {
@@ -219,10 +224,11 @@ void run_multi(void *a) {
 
 // two root steps per launch (k_batch2_grid): every plane moves by 2, the
 // maximum takes both steps and the counter advances by 2
-const int kStep2Tiles[][2] = {{64, 8}, {32, 16}, {64, 16}, {64, 16}, {64, 16}, {32, 16}, {64, 32}};
+const int kStep2Tiles[][2] = {{64, 8}, {32, 16}, {64, 16}, {64, 16}, {64, 16}, {32, 16}, {60, 32}};
 struct Batch2Arg {
   BatchLaunch B;
   int shape;
+  bool sph;
 };
 void run_batch2(void *a) {
   const Batch2Arg *x = (const Batch2Arg *)a;
@@ -236,6 +242,7 @@ void run_batch2(void *a) {
     if (bd.tiles_x != (bd.L.nx + TX - 1) / TX || bd.ntiles != bd.tiles_x * ((bd.L.ny + TY - 1) / TY))
       die("two-step descriptor tiling");
     if (!bd.L.is_root) die("two-step launch of a nested layer");
+    if (!step2_shape_takes(x->shape, bd.L, x->sph)) die("a two-step shape that the layer cannot take");
     cov[s].assign((size_t)bd.L.nx * bd.L.ny, 0);
   }
   for (int it = 0; it < B.nitems; ++it) {
@@ -317,13 +324,13 @@ hipError_t launch_jnz(const DevNest &N, hipStream_t st) {
   emu_submit(st, run_jnz, &a, sizeof(a));
   return hipSuccess;
 }
-int batch_num_shapes() { return 6; }
-void batch_shape(int k, int *tx, int *ty) { *tx = kShapes[k % 3][0]; *ty = kShapes[k % 3][1]; }
-hipError_t launch_batch(const BatchLaunch &B, int mode, bool, bool, int shape, hipStream_t st,
+int batch_num_shapes() { return kNumShapes; }
+void batch_shape(int k, int *tx, int *ty) { *tx = kShapes[k][0]; *ty = kShapes[k][1]; }
+hipError_t launch_batch(const BatchLaunch &B, int mode, bool nl, bool sph, int shape, hipStream_t st,
                         bool prepare) {
   if (prepare || B.nitems <= 0) return hipSuccess;
-  if (shape < 0 || shape >= 6) return hipErrorInvalidValue;
-  BatchArg a{B, mode, shape};
+  if (shape < 0 || shape >= kNumShapes) return hipErrorInvalidValue;
+  BatchArg a{B, mode, shape, nl, sph};
   emu_submit(st, run_batch, &a, sizeof(a));
   return hipSuccess;
 }
@@ -331,10 +338,10 @@ void step2_shape(int shape, int *tx, int *ty) {
   *tx = kStep2Tiles[shape][0];
   *ty = kStep2Tiles[shape][1];
 }
-hipError_t launch_batch2(const BatchLaunch &B, bool, int shape, hipStream_t st) {
+hipError_t launch_batch2(const BatchLaunch &B, bool sph, int shape, hipStream_t st) {
   if (B.nitems <= 0) return hipSuccess;
   if (shape < 0 || shape >= kStep2Shapes) return hipErrorInvalidValue;
-  Batch2Arg a{B, shape};
+  Batch2Arg a{B, shape, sph};
   emu_submit(st, run_batch2, &a, sizeof(a));
   return hipSuccess;
 }
@@ -368,3 +375,4 @@ hipError_t launch_fill_i32(int *p, int n, int v, hipStream_t st) {
 long long emu_fused_tiles() { return g_fused_tiles; }
 int emu_last_variant() { return g_last_variant; }
 int emu_last_step2() { return g_last_step2; }
+long long emu_shape_launches(int shape) { return g_shape_launches[shape]; }

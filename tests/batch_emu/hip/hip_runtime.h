@@ -66,3 +66,5 @@ long long emu_fused_tiles();
 // variant of the last single launch of a step, shape of the last two-step one
 int emu_last_variant();
 int emu_last_step2();
+// fused batch launches in tile shape `shape`
+long long emu_shape_launches(int shape);
