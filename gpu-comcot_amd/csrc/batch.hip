@@ -54,6 +54,14 @@
 
 using namespace gc;
 
+// Passes over a plan before it is captured (the CPU emulator of the tests, whose
+// plans live shorter, brings a number of its own).  One enqueued launch by
+// launch keeps the device as busy as a replay; building a graph costs 0.4 ms, as
+// much as a pass, so short-lived plans get none.
+#ifndef GC_DIRECT_PASSES
+#define GC_DIRECT_PASSES 16
+#endif
+
 namespace {
 
 struct Scenario {
@@ -88,8 +96,6 @@ struct Group {
   // single-layer scenarios; the lanes share no layer, so they run side by side
   int lane = 0;
 };
-
-constexpr int kDirectPasses = 16;  // passes over a plan before it is captured
 
 struct Plan {
   // root steps of the plan: 2, or 4 when single-layer linear roots take one
@@ -794,10 +800,7 @@ int run(long long n) {
     Plan &P = g_eng.plan;
     const int ns = P.nsteps;
     for (long long k = 0; k + ns <= m; k += ns) {
-      // The first passes over a plan are enqueued launch by launch, which
-      // keeps the device as busy as a graph does; building one costs 0.4 ms,
-      // as much as a pass, so only plans that live longer get theirs.
-      if (g_eng.graphs && !P.exec && P.passes == kDirectPasses)
+      if (g_eng.graphs && !P.exec && P.passes == GC_DIRECT_PASSES)
         if (int r = capture_plan(P)) return r;
       ++P.passes;
       if (P.exec) {

@@ -24,6 +24,8 @@ struct Case {
   int pnx, pny, cnx = 0, cny = 0, rt = 0;
 };
 
+int g_deep = 0;  // nests whose root step is too long for a graph
+
 [[noreturn]] void die(const char *m, int sid) {
   std::fprintf(stderr, "scenario %d: %s\n", sid, m);
   std::exit(2);
@@ -51,7 +53,10 @@ Case add_case(std::mt19937 &rng) {
     die("add root", sid);
   if (nest) {
     int R = U(2, 5), RT = U(1, 7);
-    if (!big && U(0, 29) == 0) RT = 2100 + U(0, 100);  // no-graph plans (> 4096 launches)
+    if (!big && U(0, 29) == 0) {  // no-graph plans (> 4096 launches, one JNQ to nine steps)
+      RT = 3900 + U(0, 100);
+      ++g_deep;
+    }
     int fw = U(1, (c.pnx - 6) / 2), fh = U(1, (c.pny - 6) / 2);
     if (big) fw = fh = std::min(std::min(fw, fh), 1200 / R);
     int IS = U(4, c.pnx - 2 - fw + 1), JS = U(4, c.pny - 2 - fh + 1);
@@ -98,6 +103,8 @@ int main(int argc, char **argv) {
   const int rounds = argc > 2 ? std::atoi(argv[2]) : 20;
   std::mt19937 rng(seed);
   auto U = [&](int a, int b) { return std::uniform_int_distribution<int>(a, b)(rng); };
+  // plans are captured at once, after one pass or after two
+  emu_direct_passes = (int)(seed % 3);
   int zero = 0, on = 1;
   int shape = U(-1, 5);
   if (gcomcot_batch_reset_()) return 3;
@@ -148,17 +155,20 @@ int main(int argc, char **argv) {
     verify(kv.second);
     ++checked;
   }
+  long long l = 0, g = 0, p = 0, cps = 0;
+  int tuned = 0;
+  gcomcot_batch_info_(&l, &g, &p, &cps, &tuned);  // before the reset clears it
   if (gcomcot_batch_reset_()) return 3;
   if (emu_live_bytes() != 0) {
     std::fprintf(stderr, "device memory leaked: %lld bytes\n", emu_live_bytes());
     return 6;
   }
-  long long l = 0, g = 0, p = 0, cps = 0;
-  int tuned = 0;
-  gcomcot_batch_info_(&l, &g, &p, &cps, &tuned);
   std::printf("seed %u: %d scenarios verified, shape %d, two-step %d (shape %d), "
               "%lld cross-stream waits, fused halves %d (%lld tiles)\n", seed, checked, shape,
               two, shape2, emu_cross_stream_waits(), fuse, emu_fused_tiles());
+  if (rounds >= 20 && g == 0) die("no plan was captured and replayed", 0);
+  std::printf("%lld graph replays of plans captured after %d passes, the largest of %zu launches, "
+              "%d nests too deep for one\n", g, emu_direct_passes, emu_largest_graph(), g_deep);
   std::printf("launches by shape:");
   for (int k = 0; k < 9; ++k) std::printf(" %lld", emu_shape_launches(k));
   std::printf("\n");

@@ -1,6 +1,7 @@
 // CPU stand-in for the HIP runtime calls of tree.hip / batch.hip (see
 // hip/hip_runtime.h here).  Work submitted to a stream runs at once unless
 // the stream is capturing, in which case it is recorded into the graph.
+#include <algorithm>
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
@@ -28,6 +29,8 @@ struct EmuEvent {
 };
 
 static std::map<void *, size_t> g_alloc;
+static size_t g_largest_graph = 0;
+int emu_direct_passes = 0;
 static long long g_live = 0;
 
 long long emu_live_bytes() { return g_live; }
@@ -100,10 +103,12 @@ hipError_t hipStreamEndCapture(hipStream_t s, hipGraph_t *g) {
     std::abort();
   }
   s->capturing = false;
+  if (s->graph) g_largest_graph = std::max(g_largest_graph, s->graph->work.size());
   *g = s->graph;
   s->graph = nullptr;
   return hipSuccess;
 }
+size_t emu_largest_graph() { return g_largest_graph; }
 hipError_t hipGraphInstantiate(hipGraphExec_t *e, hipGraph_t g, hipGraphNode_t *, char *, size_t) {
   *e = new EmuGraph(*g);
   return hipSuccess;

@@ -68,3 +68,8 @@ int emu_last_variant();
 int emu_last_step2();
 // fused batch launches in tile shape `shape`
 long long emu_shape_launches(int shape);
+// launches of the largest graph captured
+size_t emu_largest_graph();
+// passes over a batch plan before it is captured
+extern int emu_direct_passes;
+#define GC_DIRECT_PASSES emu_direct_passes
