@@ -1115,4 +1115,14 @@ int gcomcot_batch_info_(long long *launches, long long *graph_replays, long long
   return 0;
 }
 
+int gcomcot_batch_plan_shapes_(int *nonlinear, long long *counts, int *cap) {
+  std::fill(counts, counts + *cap, 0);
+  if (g_eng.plan_valid)
+    for (const auto &step : g_eng.plan.step)
+      for (const Group &g : step)
+        if (g.type == kStepGroup && g.mode == kFused && (g.nl != 0) == (*nonlinear != 0) && g.shape < *cap)
+          ++counts[g.shape];
+  return batch_num_shapes();
+}
+
 }  // extern "C"

@@ -208,6 +208,12 @@ class Batch:
         return {"launches": v[0].value, "graph_replays": v[1].value, "plans": v[2].value,
                 "cells_per_step": v[3].value, "tuned": t.value}
 
+    def plan_shapes(self, nonlinear=True):
+        """Fused launches of the present plan by tile shape."""
+        v = (_LL * 16)()
+        n = lib().gcomcot_batch_plan_shapes_(ip(1 if nonlinear else 0), v, ip(16))
+        return list(v)[:n]
+
     def close(self):
         lib().gcomcot_batch_reset_()
         self.specs.clear()

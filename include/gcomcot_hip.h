@@ -521,6 +521,11 @@ int gcomcot_batch_set_streams_(int *n);
 int gcomcot_batch_set_fused_halves_(int *on);
 int gcomcot_batch_info_(long long *launches, long long *graph_replays, long long *plans,
                         long long *cells_per_step, int *tuned_count);
+/* counts[0..*cap) = fused launches of the present plan by tile shape, of
+ * nonlinear or of linear layers (0 where there is no plan); returns the number
+ * of shapes: those of gcomcot_batch_set_tuning_, then 32x8 tiles and marching
+ * strips of 8 and of 14 rows, for nonlinear layers */
+int gcomcot_batch_plan_shapes_(int *nonlinear, long long *counts, int *cap);
 
 #ifdef __cplusplus
 }

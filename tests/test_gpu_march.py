@@ -351,3 +351,62 @@ def test_the_tuner_reports_only_forms_that_its_layer_runs():
     v, _, _ = dev.autotune(reps=2)
     dev.close()
     assert v < 6
+
+
+@pytest.mark.parametrize("cord", [0, 1], ids=["sph", "cart"])
+@pytest.mark.parametrize("count,nx,ny,shape", [(2, 150, 131, 6), (2, 905, 741, 7), (4, 905, 741, 8)],
+                         ids=["one-cell-tiles", "strips-of-8", "strips-of-14"])
+def test_batched_nonlinear_layers_of_one_kind_by_size(count, nx, ny, shape, cord):
+    """The rule takes the layers of one launch, which are of one coordinate kind,
+    together: every layer of the batch is of that kind, and the plan says which
+    shape it gave them."""
+    from gcomcot.batch import Batch
+    from helpers import BEACH
+    scs = [S.custom(laycord=cord, laygov=1, nx=nx - 7 * k, ny=ny - 5 * k, **BEACH) for k in range(count)]
+    print(f"[gpu] batch of {count} nonlinear layers of kind {cord} near {nx}x{ny}", flush=True)
+    b = Batch(autotune=False)
+    sids = [b.add(sc, 15) for sc in scs]
+    b.run(4)
+    shapes = b.plan_shapes()
+    assert shapes[shape] > 0 and sum(shapes) == shapes[shape], shapes
+    b.run(11)
+    for sc, sid in zip(scs, sids):
+        orc = Oracle(sc, 32, pow_mode=1)
+        orc.step(15)
+        st, mx, o, om = b.state(sid), b.maxima(sid), orc.state(1), orc.maxima(1)
+        for k in ("z1", "m1", "n1"):
+            nb, worst = diff_report(st[k], o[k])
+            assert nb == 0, f"{sc.name} {k}: {nb} cells differ (max {worst})"
+        assert diff_report(mx["zmax_wet"], om["zmax_wet"])[0] == 0, sc.name
+        assert (mx["arrival"] == om["arrival"]).all(), sc.name
+    b.close()
+
+
+@pytest.mark.parametrize("cord", [0, 1], ids=["sph", "cart"])
+@pytest.mark.parametrize("count,shape", [(2, 7), (4, 8)], ids=["strips-of-8", "strips-of-14"])
+def test_batched_children_in_marching_strips(count, shape, cord):
+    """Nested layers of a batch in marching strips, whose sides and ends write
+    the boundary fluxes of the sub-step that follows."""
+    from gcomcot.batch import Batch
+    from helpers import BEACH
+    scs = [S.custom(nx=250, ny=210, laygov=0, case=k,
+                    child=dict(laycord=cord, laygov=1, footprint=(226 - 2 * k, 185 - k), rel_size=4, rel_time=3,
+                               corner=(9, 8)), **BEACH) for k in range(count)]
+    print(f"[gpu] batch of {count} nests, children of kind {cord}", flush=True)
+    b = Batch(autotune=False, streams=2)  # the nests in one chain
+    sids = [b.add(sc, 6) for sc in scs]
+    b.run(2)
+    shapes = b.plan_shapes()
+    assert shapes[shape] > 0 and sum(shapes) == shapes[shape], shapes
+    b.run(4)
+    for sc, sid in zip(scs, sids):
+        orc = Oracle(sc, 32, pow_mode=1)
+        orc.step(6)
+        for lid in (1, 2):
+            st, mx, o, om = b.state(sid, lid), b.maxima(sid, lid), orc.state(lid), orc.maxima(lid)
+            for k in ("z1", "m1", "n1"):
+                nb, worst = diff_report(st[k], o[k])
+                assert nb == 0, f"{sc.name} layer {lid} {k}: {nb} cells differ (max {worst})"
+            assert diff_report(mx["zmax_wet"], om["zmax_wet"])[0] == 0, (sc.name, lid)
+            assert (mx["arrival"] == om["arrival"]).all(), (sc.name, lid)
+    b.close()
