@@ -32,6 +32,7 @@ struct DevLayer {
   int *ctl;            // root-step counters: read ctl[ctl_in], write ctl[1-ctl_in]
   int ctl_in, advance; // advance: this launch writes the next counter
   float arr_thr;
+  float kf26;          // drag_scaled(kfric) (fastdiv.h)
   // MAX_AMP's maximum (GPUOutput.cu:46-53: no wet test, NaN replaces),
   // fused into the step of the outermost layer when != null
   float *zraw;

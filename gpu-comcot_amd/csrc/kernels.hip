@@ -414,7 +414,7 @@ __device__ float nl_x(const DevLayer &L, const A &s, int i, int j, float brk) {
   float FF = 0.0f;
   bool drag = false;
   auto friction = [&](float x) {
-    drag = L.fric && !(SPH && drag_vanishes(drag_scaled(L.kfric), p, xqq, DF, x));
+    drag = L.fric && !(SPH && drag_vanishes(L.kf26, p, xqq, DF, x));
     if (drag)
       FF = div_inrange(L.kfric * sqrt_inrange(p * p + xqq * xqq),
                        gcdet::powf_manning(DF, kManExp, *s.tab));
@@ -511,7 +511,7 @@ __device__ float nl_y(const DevLayer &L, const A &s, int i, int j, float brk) {
   float FF = 0.0f;
   bool drag = false;
   auto friction = [&](float x) {
-    drag = L.fric && !(SPH && drag_vanishes(drag_scaled(L.kfric), q, xpp, DF, x));
+    drag = L.fric && !(SPH && drag_vanishes(L.kf26, q, xpp, DF, x));
     if (drag)
       FF = div_inrange(L.kfric * sqrt_inrange(q * q + xpp * xpp),
                        gcdet::powf_manning(DF, kManExp, *s.tab));

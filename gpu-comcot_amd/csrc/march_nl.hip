@@ -128,7 +128,7 @@ __device__ __forceinline__ void march_nl(const DevLayer &L, const Strip S, int s
   const unsigned oz1 = plane_off(L, L.z1), om1 = plane_off(L, L.m1), on1 = plane_off(L, L.n1),
                  oz2 = plane_off(L, L.z2), om2 = plane_off(L, L.m2), on2 = plane_off(L, L.n2),
                  omax = plane_off(L, L.zmax), oarr = plane_off(L, L.arrival);
-  const float zt = breaking_floor(L.dt), kf26 = drag_scaled(L.kfric);
+  const float zt = breaking_floor(L.dt);
   // a nested layer's boundary fluxes of the next sub-step: M of the side
   // columns comes row by row, N of rows 1 and NY once.  Lanes without one, and
   // every lane where there are none, read past the table: 0.
@@ -304,7 +304,7 @@ __device__ __forceinline__ void march_nl(const DevLayer &L, const Strip S, int s
       const float pe = east(pp[1]), pw = west(pp[1]);
       if (act) {
         X = f.p - (SPH ? CX[0] : L.grx) * DD * (f.zb - f.za);
-        const Mask drag = SPH ? act & ~GC_BALLOT(drag_vanishes(kf26, f.p, f.cross, DF, X)) : ~0ull;
+        const Mask drag = SPH ? act & ~GC_BALLOT(drag_vanishes(L.kf26, f.p, f.cross, DF, X)) : ~0ull;
         float FF = 0.0f;
         if (drag) {
           FF = friction(L, f, DF, tab);
@@ -340,7 +340,7 @@ __device__ __forceinline__ void march_nl(const DevLayer &L, const Strip S, int s
       const float qe = east(qc[2]), qw = west(qc[2]);
       if (act) {
         Y = f.p - (SPH ? CY[0] : L.gry) * DD * (f.zb - f.za);
-        const Mask drag = SPH ? act & ~GC_BALLOT(drag_vanishes(kf26, f.p, f.cross, DF, Y)) : ~0ull;
+        const Mask drag = SPH ? act & ~GC_BALLOT(drag_vanishes(L.kf26, f.p, f.cross, DF, Y)) : ~0ull;
         float FF = 0.0f;
         if (drag) {
           FF = friction(L, f, DF, tab);

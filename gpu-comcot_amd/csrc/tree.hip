@@ -20,6 +20,7 @@
 #include <cstring>
 
 #include "comcot_consts.h"
+#include "fastdiv.h"
 #include "tree.h"
 
 namespace gc {
@@ -315,6 +316,7 @@ DevLayer dev_view(const Tree &T, const LayerRec &L, bool with_max, bool advance)
   d.gry = L.gry;
   d.dt = L.dt;
   d.kfric = L.kfric;
+  d.kf26 = drag_scaled(L.kfric);
   d.h = L.h;
   d.coef = L.coef;
   d.rowc = L.rowc;
