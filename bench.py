@@ -50,6 +50,7 @@ sys.path.insert(0, ROOT)
 import numpy as np  # noqa: E402
 
 HBM_PEAK_GBS = 8000.0
+SIMDS, CLOCK_GHZ = 1024, 2.4
 BYTES_PER_CELL = {"linear": 28, "nonlinear_max": 36}
 METRIC = "GCUPS + %HBM roofline; batched scenarios/s with p50/p99 time-to-forecast"
 
@@ -188,13 +189,27 @@ def cpu_all_cores(sc, nsteps):
             "sample": f"{nsteps} steps (after 1 untimed), {threads} OpenMP threads, {dt:.1f} s"}
 
 
-def traffic_entry(workload_key):
+def traffic_entry(workload_key, form, tile):
+    """Counters of one launch of this form, from profiles/traffic.json, or None."""
     path = os.path.join(ROOT, "profiles", "traffic.json")
     try:
         with open(path) as f:
-            return json.load(f).get(workload_key)
+            entries = json.load(f).get(workload_key, [])
     except (OSError, ValueError):
         return None
+    return next((e for e in entries if e["form"] == form and e["tile"] == tile), None)
+
+
+def limit_text(counted, kern_ms):
+    """What bounds the headline launch, by its counters (None where that form was
+    not counted)."""
+    if not counted or "valu_instructions_per_launch" not in counted:
+        return None
+    nbytes, valu = counted["bytes_per_launch"], counted["valu_instructions_per_launch"]
+    issue_us = valu / SIMDS * 4 / CLOCK_GHZ * 1e-3
+    return (f"HBM traffic and VALU issue: {nbytes / 1e6:.0f} MB a launch "
+            f"({nbytes / kern_ms * 1e-9:.2f} TB/s) beside {valu / 1e6:.1f} M wave64 VALU instructions, "
+            f"{issue_us:.0f} us at one per SIMD every 4 cycles of {CLOCK_GHZ} GHz")
 
 
 def bench_c1(a):
@@ -223,26 +238,22 @@ def bench_c1(a):
     gcups = cells * a.steps / wall / 1e9
     mx = run.maxima(1)
     arrived = int(np.count_nonzero(mx["arrival"] >= 0))
-    run.close()
     import ctypes
-    tx = (ctypes.c_int * 64)()
-    ty = (ctypes.c_int * 64)()
-    n = ctypes.c_int(0)
-    lib().gcomcot_tile_variants_(ctypes.byref(n), tx, ty)
-    key = f"nonlinear-{a.nx}x{a.ny}"
-    tr = traffic_entry(key)
-    traffic = None
-    if tr and tr.get("tile") == [tx[variant], ty[variant]]:
-        traffic = tr.get("bytes_per_launch")
-    return sc, cells, gcups, wall, kern_ms, achieved, traffic, arrived, ms_total, \
-        (tx[variant], ty[variant])
+    tx, ty = ctypes.c_int(0), ctypes.c_int(0)
+    if lib().gcomcot_fused_form_(ip(1), ctypes.byref(tx), ctypes.byref(ty)) != 0:
+        raise RuntimeError("no form of layer 1")
+    run.close()
+    form = "marching strips" if tx.value < 0 else "tiles"
+    tile = [abs(tx.value), ty.value]
+    counted = traffic_entry(f"nonlinear-{a.nx}x{a.ny}", form, tile)
+    return sc, cells, gcups, wall, kern_ms, achieved, counted, arrived, ms_total, form, tile
 
 
 def bench_other_configs(a):
     """The single-layer linear configuration (1024x768, 2000 steps) and the
     two-level nest (2048x1536 linear parent + 1801x1801 nonlinear Cartesian
     child, REL_SIZE 4, REL_TIME 4, 3000 steps) through the whole-run device
-    loop (HIP graph): GCUPS over all layers' cell updates."""
+    loop: GCUPS over all layers' cell updates."""
     from gcomcot import DeviceRun, linear_layer, two_level_nest
     out = {}
     for name, sc, bpc in (("linear_1024x768", linear_layer(), BYTES_PER_CELL["linear"]),
@@ -266,7 +277,7 @@ def bench_other_configs(a):
 
 
 def bench_outputs(a):
-    """The headline workload through the device loop (graphs), without and
+    """The headline workload through the device loop, without and
     with the reference's output files: snapshots z/m/n every --outputs-iprt
     root steps and at step 0, MAX_AMP's maximum kept by the step kernel and
     written when due (TEND at the last step).  ms_per_step_* time the loop
@@ -517,7 +528,8 @@ def main():
         return
     from gcomcot import nonlinear_layer
 
-    sc, cells, gcups, wall, kern_ms, achieved, traffic, arrived, ms_total, tile = bench_c1(a)
+    sc, cells, gcups, wall, kern_ms, achieved, counted, arrived, ms_total, form, tile = bench_c1(a)
+    traffic = counted["bytes_per_launch"] if counted else None
     cpu = None
     if a.cpu_steps > 0:
         log("cpu baseline")
@@ -553,16 +565,14 @@ def main():
         "data": "synthetic (seeded bathymetry, dipole source)",
         "config": {"workload": f"single-layer nonlinear spherical {a.nx}x{a.ny} at 0.5 arc-min, "
                                "Manning 0.013, wet max + arrival on device",
-                   "cells": cells, "tile": list(tile), "parallelism": "single GPU"},
+                   "cells": cells, "form": form, "tile": tile, "parallelism": "single GPU"},
         "roofline": {"bound": "hbm", "achieved": round(achieved, 1), "peak": HBM_PEAK_GBS,
                      "unit": "GB/s", "frac": round(achieved / HBM_PEAK_GBS, 4),
                      "traffic": traffic,
                      "traffic_per_cell_update": round(traffic / cells, 2) if traffic else None,
                      "practical_peak": copy["read_plus_write_GBs"],
                      "frac_of_practical": round(achieved / copy["read_plus_write_GBs"], 4),
-                     "limit": "HBM traffic and VALU issue alike: the marching step counts 489 MB "
-                              "a launch (4.3 TB/s) beside 51 M wave64 VALU instructions, 84 us "
-                              "at one per SIMD every 4 cycles"},
+                     "limit": limit_text(counted, kern_ms)},
         "cpu_baseline": cpu,
         "kernel_ms_mean": round(kern_ms, 5),
         "event_ms_total": round(ms_total, 3),

@@ -1095,4 +1095,12 @@ int gcomcot_tile_variants_(int *count, int *tx, int *ty) {
   return R ? fused_variant(g_tree, *R, dev_view(g_tree, *R, true, true)) : g_tree.variant;
 }
 
+int gcomcot_fused_form_(int *lid, int *tx, int *ty) {
+  LayerRec *L = layer(*lid);
+  if (!L) return fail(48, "gcomcot_fused_form_: no layer %d", *lid);
+  const DevLayer d = dev_view(g_tree, *L, true, L->id == 1);
+  fused_form(d, L->nl != 0, L->sph != 0, fused_variant(g_tree, *L, d), tx, ty);
+  return 0;
+}
+
 }  // extern "C"

@@ -85,6 +85,9 @@ hipError_t launch_step(const DevLayer &L, int mode, bool nl, bool sph, int varia
 int num_tile_variants();
 void tile_variant_shape(int v, int *tx, int *ty);
 bool tile_variant_is_tile(int v);  // the tiles come first, marching strips after them
+// What a fused step of this view runs at variant `variant`: tiles of tx x ty, or
+// marching strips of -tx columns in segments of ty rows.
+void fused_form(const DevLayer &L, bool nl, bool sph, int variant, int *tx, int *ty);
 
 // Two root steps of a linear outermost layer without children in one
 // launch (temporal blocking); shape 0..6 = tiles of 64x8, 32x16, 64x16 with

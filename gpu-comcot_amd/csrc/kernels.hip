@@ -2102,6 +2102,17 @@ static int nl_form(const DevLayer &L, bool sph, int variant) {
   return variant == 0 && (long long)L.nx * L.ny <= kSmallCells ? 0 : -1;
 }
 
+void fused_form(const DevLayer &L, bool nl, bool sph, int variant, int *tx, int *ty) {
+  const int form = nl ? nl_form(L, sph, variant) : -1;
+  if (form >= 0) {
+    *tx = form > 0 ? -60 : 32;
+    *ty = form > 0 ? form : 8;
+    return;
+  }
+  if (kVariants[variant][0] == 0) variant = 0;
+  tile_variant_shape(variant, tx, ty);
+}
+
 // Measured, us per step (64x8 tiles; 32x8 with 4 and 8 waves per SIMD):
 // 96x72 13.9; 9.4, 9.9.  517x391 14.4; 10.9, 11.3.  512x384 + 401x401 nest
 // 84.9; 67.2, 67.9.  1024x768 21.0; 18.95, 18.3.  1201x901 24.5; 23.2, 22.8.

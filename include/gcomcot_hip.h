@@ -182,6 +182,9 @@ int gcomcot_last_error_(char *buf, int *len);
  * variant index, see gcomcot_tile_variants_.  Returns 0 if valid. */
 int gcomcot_set_tile_variant_(int *variant);
 int gcomcot_tile_variants_(int *count, int *tx, int *ty);
+/* What a fused step of layer *lid runs: tiles of *tx x *ty cells, or marching
+ * strips of -*tx columns in segments of *ty rows.  Returns 0 or an error code. */
+int gcomcot_fused_form_(int *lid, int *tx, int *ty);
 
 /* Gauges on the device (reference: GET_TS, output.f90:1035-1155, which
  * calls gcomcot_get_z_ and copies a 2x2 stencil to the host per gauge per
