@@ -23,8 +23,9 @@
 // disjoint scenarios (single-layer scenarios; two halves of the nested
 // ones) that run on three streams, forked and joined within each plan.
 // The launches of a plan (two root steps, four with two-step roots) are
-// captured in a HIP graph and replayed; the plan is rebuilt when the set
-// of active scenarios changes (a scenario finishes, is added or removed).
+// enqueued directly at first, then captured in a HIP graph and replayed; the
+// plan is rebuilt when the set of active scenarios changes (a scenario finishes,
+// is added or removed).
 //
 // Step launches run (layer, tile) items either in the persistent kernel
 // k_batch (8 per-XCD queues with atomic heads, cleared by a fill kernel at

@@ -971,7 +971,7 @@ struct StepWaves {
   static constexpr int fit = kLdsPerCu / LDS_BYTES;
   static constexpr int value = want < fit ? want : (fit > 0 ? fit : 1);
 };
-// LDS of the tile kernels (k_step, k_batch, k_batch_grid) and of k_stream
+// LDS of the tile kernels (k_step, k_batch, k_batch_grid)
 template <int TX, int TY>
 constexpr int tile_lds_bytes() {
   return (int)((6 * (TX + 4) * (TY + 4) + kNumCoef * (TY + 4)) * sizeof(float) +
@@ -1858,7 +1858,7 @@ __global__ void __launch_bounds__(256) k_apply_deform(float *z1, float *h,
 }
 
 // Gauge samples of every layer (a single layer's are made by its next step,
-// gauge_block).
+// step_block).
 __global__ void k_gauges(const GaugeDev *__restrict__ gs, int n, ZNow zs,
                          const int *__restrict__ step_now, float *ring, int cap) {
   const int k = blockIdx.x * blockDim.x + threadIdx.x;

@@ -445,9 +445,9 @@ int gcomcot_detmath_eval_noalloc_(long long *n, const float *x, float *pow_out,
  * level of nested layers and its own number of root steps, advanced
  * together: every phase of a root step is one launch over all active
  * scenarios (a persistent kernel draining per-XCD tile queues), two root
- * steps are replayed from a HIP graph, and fused tile shapes are picked
- * by an on-line autotuner.  Each scenario's planes are bit-identical to a
- * run of the same layers alone through Part 1/2.  Scenarios can be added
+ * steps are replayed from a HIP graph once a plan has run some times, and
+ * fused tile shapes are picked by an on-line autotuner.  Each scenario's
+ * planes are bit-identical to a run of the same layers alone through Part 1/2.  Scenarios can be added
  * and removed between calls (continuous batching).  All calls return 0 or
  * an error code (see gcomcot_set_error_mode_ / gcomcot_last_error_). */
 
